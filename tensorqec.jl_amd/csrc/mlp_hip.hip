@@ -42,69 +42,47 @@ typedef __attribute__((__vector_size__(8 * sizeof(short)))) short bf16x8;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 
 __device__ __forceinline__ float bf2f(bf16 h) { return __uint_as_float(((uint32_t)h) << 16); }
-__device__ __forceinline__ bf16 f2bf(float f) {
-    const uint32_t u = __float_as_uint(f);
-    return (bf16)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);   // round to nearest even
+// Round to nearest even, one v_cvt_pk_bf16_f32 for two values (rounding in
+// integer arithmetic, five instructions a value, made the fused forward kernel
+// 83 us instead of 75 at 65,536 rows).
+typedef __attribute__((__vector_size__(2 * sizeof(float)))) float f32x2;
+typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bfx2;
+__device__ __forceinline__ uint32_t f2bf2(float a, float b) {
+    const f32x2 v = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bfx2));
 }
+__device__ __forceinline__ bf16 f2bf(float f) { return (bf16)f2bf2(f, 0.f); }
 
 // ---------------------------------------------------------------------------
-// GEMM: C[M][N] = op(A)[M][K] * op(B)[K][N], BF16 in, FP32 accumulate.
-//   A: AT ? A[k*lda + m] : A[m*lda + k];   B: BT ? B[n*ldb + k] : B[k*ldb + n]
-// Block tile 128x128, K step 32, 4 waves each owning 64x64 = 2x2 MFMA tiles
-// of 32x32.  Tiles are staged in LDS as [row][k] (k contiguous) so each lane
-// reads its 8 consecutive k values with one 16-byte LDS load.  Rows/columns
-// beyond M/N are zero-filled on load and skipped on store; K must be a
-// multiple of 32.
+// Backward GEMM of the layer-by-layer path: C[M][N] = A[M][K] * B^T (B[n*ldb +
+// k]) where mask > 0, BF16 in and out, FP32 accumulate.  Block tile 128x128, K
+// step 32, 4 waves each owning 64x64 = 2x2 MFMA tiles of 32x32.  Tiles are
+// staged in LDS as [row][k] (k contiguous) so each lane reads its 8
+// consecutive k values with one 16-byte LDS load.  Rows beyond M/N are
+// zero-filled on load and skipped on store; K must be a multiple of 32.
 // ---------------------------------------------------------------------------
-
-enum Epi : int {
-    kEpiBiasReluBf16 = 0,  // out_bf16 = bf16(relu(acc + bias[col]))
-    kEpiMaskBf16 = 1,      // out_bf16 = bf16(acc) where mask_bf16 > 0, else 0
-    kEpiF32 = 2,           // out_f32 = acc
-};
 
 struct GemmArgs {
     const bf16 *A;
     const bf16 *B;
     int M, N, K, lda, ldb, ldc;
-    const float *bias;
     const bf16 *mask;
     bf16 *outb;
-    float *outf;
 };
 
 constexpr int BM = 128, BN = 128, BK = 32, LDSK = BK + 8;
 
-template <bool T>
-__device__ __forceinline__ void load_tile(bf16 *S, const bf16 *G, int rows0, int R, int k0, int K, int ld, int tid) {
-    // S[r][k] for r in [0,128), k in [0,32)
-    if (!T) {
-        // G[r*ld + k]: 128 rows x 32 k = 512 chunks of 8
-        for (int c = tid; c < 512; c += 256) {
-            const int r = c >> 2, kc = (c & 3) * 8;
-            const int gr = rows0 + r;
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (gr < R) v = *reinterpret_cast<const uint4 *>(G + (size_t)gr * ld + k0 + kc);
-            *reinterpret_cast<uint4 *>(S + r * LDSK + kc) = v;
-        }
-    } else {
-        // G[k*ld + r]: 32 k x 128 r = 512 chunks of 8 along r, transposed into S
-        for (int c = tid; c < 512; c += 256) {
-            const int k = c >> 4, rc = (c & 15) * 8;
-            const int gr = rows0 + rc;
-            bf16 v[8];
-            if (gr + 7 < R) {
-                const uint4 u = *reinterpret_cast<const uint4 *>(G + (size_t)(k0 + k) * ld + gr);
-                memcpy(v, &u, 16);
-            } else {
-                for (int j = 0; j < 8; ++j) v[j] = (gr + j < R) ? G[(size_t)(k0 + k) * ld + gr + j] : (bf16)0;
-            }
-            for (int j = 0; j < 8; ++j) S[(rc + j) * LDSK + k] = v[j];
-        }
+// S[r][k] for r in [0,128), k in [0,32) of G[r*ld + k]: 512 chunks of 8
+__device__ __forceinline__ void load_tile(bf16 *S, const bf16 *G, int rows0, int R, int k0, int ld, int tid) {
+    for (int c = tid; c < 512; c += 256) {
+        const int r = c >> 2, kc = (c & 3) * 8;
+        const int gr = rows0 + r;
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (gr < R) v = *reinterpret_cast<const uint4 *>(G + (size_t)gr * ld + k0 + kc);
+        *reinterpret_cast<uint4 *>(S + r * LDSK + kc) = v;
     }
 }
 
-template <bool AT, bool BT, int EPI>
 __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g) {
     __shared__ __align__(16) bf16 As[BM * LDSK];
     __shared__ __align__(16) bf16 Bs[BN * LDSK];
@@ -116,8 +94,8 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g) {
         for (int j = 0; j < 2; ++j)
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
     for (int k0 = 0; k0 < g.K; k0 += BK) {
-        load_tile<AT>(As, g.A, m0, g.M, k0, g.K, g.lda, tid);
-        load_tile<BT ? false : true>(Bs, g.B, n0, g.N, k0, g.K, g.ldb, tid);
+        load_tile(As, g.A, m0, g.M, k0, g.lda, tid);
+        load_tile(Bs, g.B, n0, g.N, k0, g.ldb, tid);
         __syncthreads();
         for (int kk = 0; kk < BK; kk += 16) {
             bf16x8 a[2], b[2];
@@ -140,15 +118,8 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g) {
             for (int v = 0; v < 16; ++v) {
                 const int row = m0 + wm + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
                 if (row >= g.M) continue;
-                const float x = acc[i][j][v];
                 const size_t o = (size_t)row * g.ldc + col;
-                if (EPI == kEpiBiasReluBf16) {
-                    g.outb[o] = f2bf(fmaxf(x + g.bias[col], 0.f));
-                } else if (EPI == kEpiMaskBf16) {
-                    g.outb[o] = bf2f(g.mask[o]) > 0.f ? f2bf(x) : (bf16)0;
-                } else {
-                    g.outf[o] = x;
-                }
+                g.outb[o] = bf2f(g.mask[o]) > 0.f ? f2bf(acc[i][j][v]) : (bf16)0;
             }
         }
 }
@@ -262,19 +233,41 @@ constexpr int kFusedRows = 128, kFusedHid = 512;
 
 __device__ __forceinline__ int act_off(int m, int chunk) { return m * (kFusedHid * 2) + ((chunk ^ (m & 15)) << 4); }
 
-// Fragment-ordered weights.  Hidden layer l (K x 512): for each 16-row k-step
-// s and 32-column tile t, 64 lanes x 8 BF16: lane L holds W[16 s + 8 (L >> 5)
-// + e][32 t + (L & 31)], e = 0..7.  Output layer: one 32-column tile, columns
-// >= nout zero.
-__global__ void pack_fused_kernel(const bf16 *__restrict__ W, int K, int N, int nout_pad, bf16 *__restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int tiles = nout_pad / 32;
-    if (i >= (int64_t)K * nout_pad) return;
+// Fragment-ordered weights, all of them in one launch.  Forward (wf), hidden
+// layer l (K x 512): for each 16-row k-step s and 32-column tile t, 64 lanes x
+// 8 BF16: lane L holds W[16 s + 8 (L >> 5) + e][32 t + (L & 31)], e = 0..7;
+// output layer: one 32-column tile, columns >= nout zero.  Backward (wk, the
+// two inner hidden layers), contracting over the columns: lane L holds
+// W[32 t + (L & 31)][16 s + 8 (L >> 5) + e].  Last, the output layer's rows
+// padded with zeros to 4 or 16 classes.
+constexpr int kPacks = 7;
+struct PackArgs {
+    const bf16 *W[kPacks];
+    bf16 *out[kPacks];
+    int64_t end[kPacks];   // running totals of the outputs' elements
+    int N[kPacks];         // columns of W
+    int tiles[kPacks];     // 32-wide tiles of the output index (padded rows: their length)
+    int kind[kPacks];      // 0 forward, 1 backward, 2 padded rows
+};
+
+__global__ void pack_fused_kernel(PackArgs a) {
+    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= a.end[kPacks - 1]) return;
+    int g = 0;
+    while (i >= a.end[g]) ++g;
+    if (g) i -= a.end[g - 1];
+    if (a.kind[g] == 2) {
+        const int64_t k = i / a.tiles[g];
+        const int n = (int)(i - k * a.tiles[g]);
+        a.out[g][i] = n < a.N[g] ? a.W[g][k * a.N[g] + n] : (bf16)0;
+        return;
+    }
     const int e = (int)(i & 7), L = (int)((i >> 3) & 63);
     const int64_t q = i >> 9;   // (s, t)
-    const int t = (int)(q % tiles), s = (int)(q / tiles);
+    const int t = (int)(q % a.tiles[g]), s = (int)(q / a.tiles[g]);
     const int k = 16 * s + 8 * (L >> 5) + e, n = 32 * t + (L & 31);
-    out[i] = n < N ? W[(int64_t)k * N + n] : (bf16)0;
+    if (a.kind[g] == 1) a.out[g][i] = a.W[g][(int64_t)n * a.N[g] + k];
+    else a.out[g][i] = n < a.N[g] ? a.W[g][(int64_t)k * a.N[g] + n] : (bf16)0;
 }
 
 template <int NW>
@@ -356,10 +349,9 @@ __global__ void __launch_bounds__(64 * NW) mlp_fused_fwd_kernel(const uint8_t *_
                 const int m = 32 * mt + m32;
                 for (int g = 0; g < 4; ++g) {
                     const int n0 = 32 * (wave * NT + t) + 8 * g + 4 * h;
-                    uint16_t v[4];
-                    for (int r = 0; r < 4; ++r) v[r] = f2bf(fmaxf(acc[t][mt][4 * g + r], 0.f));
                     uint2 u;
-                    memcpy(&u, v, 8);
+                    u.x = f2bf2(fmaxf(acc[t][mt][4 * g], 0.f), fmaxf(acc[t][mt][4 * g + 1], 0.f));
+                    u.y = f2bf2(fmaxf(acc[t][mt][4 * g + 2], 0.f), fmaxf(acc[t][mt][4 * g + 3], 0.f));
                     *reinterpret_cast<uint2 *>(act + act_off(m, n0 >> 3) + ((n0 & 7) << 1)) = u;
                 }
             }
@@ -384,6 +376,498 @@ __global__ void __launch_bounds__(64 * NW) mlp_fused_fwd_kernel(const uint8_t *_
                 if (n < nout) z[r * nout + n] = acc[v];
             }
     }
+}
+
+// ---------------------------------------------------------------------------
+// Training, hidden width 512: everything that is local to a row in one launch.
+// A workgroup of 8 waves takes 32 rows through the forward pass, the loss, and
+// the backward pass down to the first layer's pre-activations; all activations
+// of the tile stay in LDS (X, H1, H2, H3: 4 x 32 KB, laid out by act_off) and
+// each gradient overwrites the activations it is masked with.  What the weight
+// gradients contract over the batch goes to global memory once: X, H1, H2 and
+// dA1..dA3 (BF16); the output layer's gradient and the bias gradients leave as
+// one partial sum per tile.  32 rows, so that the trainer's 8,192 rows give
+// one workgroup to each of the 256 CUs; the bound is then the weights'
+// stream from L2 (2.1 MB per workgroup against 64 B per clock and CU), kept
+// six k-steps ahead in registers.  Products, roundings to BF16 and FP32
+// accumulation are those of the layer-by-layer kernels.  Measured at 48 inputs,
+// 4 classes, 8,192 rows: 38.5 us; the layers one by one took 75 us forward and
+// down to dA1, and sums over the batch by one thread per parameter 8.3 ms more.
+// ---------------------------------------------------------------------------
+
+constexpr int kTrainRows = 32, kTrainMaxOut = 16;
+constexpr int kTrainBuf = kTrainRows * kFusedHid * 2;   // bytes of one tile of activations
+// buffers, logit partials of the 8 waves, dz
+constexpr int kTrainLds = 4 * kTrainBuf + 8 * kTrainRows * kTrainMaxOut * 4 + kTrainRows * kTrainMaxOut * 4;
+
+struct TrainArgs {
+    const uint8_t *syn;
+    const float *q;
+    int64_t B;
+    int n_in, kin, nout;
+    const bf16 *wf[4];      // forward fragments
+    const bf16 *wk[2];      // backward fragments of layers 2 and 3
+    const bf16 *w4;         // output layer, [512][NP]
+    const float *bias[4];
+    bf16 *X, *H1, *H2, *dA1, *dA2, *dA3;
+    float *part;            // per tile: dW4 [512][nout] | db4 [nout] | db1 | db2 | db3
+    int64_t part_len;
+    float *loss_parts;
+};
+
+// acc[t] += W^T x src^T for this wave's two 32-column tiles, weights six
+// k-steps and activations two steps ahead.  start() issues the first six
+// steps' weights; it is called before the epilogue and the barrier in front of
+// the product.  Left to itself the compiler moves every load down to its use
+// (a layer then takes 20 us), so the steps are kept apart by scheduling
+// barriers.
+struct TrainGemm {
+    static constexpr int DEP = 6, XD = 2, STEPS = kFusedHid / 16;
+    bf16x8 wb[DEP][2];
+    const bf16 *base;
+    const unsigned char *src;
+    int m32, h;
+
+    __device__ __forceinline__ void wload(int slot, int s) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) wb[slot][t] = *reinterpret_cast<const bf16x8 *>(base + ((s * 16 + t) << 9));
+    }
+    __device__ __forceinline__ bf16x8 xload(int s) const {
+        return *reinterpret_cast<const bf16x8 *>(src + act_off(m32, 2 * s + h));
+    }
+    __device__ __forceinline__ void start(const bf16 *__restrict__ W, const unsigned char *from, int steps, int wave,
+                                          int lane) {
+        base = W + (wave << 10) + lane * 8;
+        src = from;
+        m32 = lane & 31;
+        h = lane >> 5;
+#pragma unroll
+        for (int s = 0; s < DEP; ++s) wload(s, min(s, steps - 1));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // K = 512
+    __device__ __forceinline__ void run(f32x16 acc[2]) {
+        bf16x8 x[XD];
+#pragma unroll
+        for (int s = 0; s < XD; ++s) x[s] = xload(s);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wb[s % DEP][t], x[s % XD], acc[t], 0, 0, 0);
+            if (s + DEP < STEPS) wload(s % DEP, s + DEP);
+            if (s + XD < STEPS) x[s % XD] = xload(s + XD);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // any number of steps (the input layer): those beyond the first six as they come
+    __device__ __forceinline__ void run(f32x16 acc[2], int steps) {
+#pragma unroll
+        for (int s = 0; s < DEP; ++s)
+            if (s < steps) {
+                const bf16x8 x = xload(s);
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wb[s][t], x, acc[t], 0, 0, 0);
+            }
+        for (int s = DEP; s < steps; ++s) {
+            const bf16x8 x = xload(s);
+            wload(0, s);
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wb[0][t], x, acc[t], 0, 0, 0);
+        }
+    }
+};
+
+// The pair of gradients (a, b) as BF16 where the activations in `h` are positive.
+__device__ __forceinline__ uint32_t masked_pair(uint32_t h, float a, float b) {
+    const uint32_t m = (bf2f((bf16)h) > 0.f ? 0xffffu : 0u) | (__uint_as_float(h & 0xffff0000u) > 0.f ? 0xffff0000u : 0u);
+    return f2bf2(a, b) & m;
+}
+
+// A tile of activations or gradients out to rows row0.. of `out`.
+__device__ __forceinline__ void train_store(const unsigned char *buf, bf16 *__restrict__ out, int64_t row0, int tid) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int m = (tid >> 6) + 8 * j, c = tid & 63;
+        *reinterpret_cast<uint4 *>(out + (row0 + m) * kFusedHid + 8 * c) =
+            *reinterpret_cast<const uint4 *>(buf + act_off(m, c));
+    }
+}
+
+// Sum over the tile's rows of column tid.
+__device__ __forceinline__ float train_colsum(const unsigned char *buf, int tid) {
+    float s = 0.f;
+#pragma unroll
+    for (int m = 0; m < kTrainRows; ++m)
+        s += bf2f(*reinterpret_cast<const bf16 *>(buf + act_off(m, tid >> 3) + ((tid & 7) << 1)));
+    return s;
+}
+
+// NP: classes, padded to 4 or 16 (dz and w4 hold zeros beyond nout).
+template <int NP>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) mlp_train_rows_kernel(TrainArgs a) {
+    extern __shared__ __align__(16) unsigned char act[];
+    unsigned char *bx = act, *b1 = act + kTrainBuf, *b2 = act + 2 * kTrainBuf, *b3 = act + 3 * kTrainBuf;
+    float *zp = reinterpret_cast<float *>(act + 4 * kTrainBuf);           // [8][32][NP]
+    float *dz = zp + 8 * kTrainRows * kTrainMaxOut;                        // [32][NP]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int m32 = lane & 31, h = lane >> 5;
+    const int64_t row0 = (int64_t)blockIdx.x * kTrainRows;
+    TrainGemm gm;
+    gm.start(a.wf[0], bx, a.kin >> 4, wave, lane);
+    // syndrome bits -> BF16 0/1 features in columns [0, kin)
+    const int cpr = a.kin >> 3;
+    for (int q = tid; q < kTrainRows * cpr; q += 512) {
+        const int m = q / cpr, c = q - m * cpr;
+        const uint8_t *row = a.syn + (row0 + m) * a.n_in;
+        uint16_t v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int f = 8 * c + e;
+            const uint8_t bit = row[min(f, a.n_in - 1)];
+            v[e] = (f < a.n_in && (bit & 1)) ? (uint16_t)0x3f80 : (uint16_t)0;
+        }
+        uint4 u;
+        memcpy(&u, v, 16);
+        *reinterpret_cast<uint4 *>(bx + act_off(m, c)) = u;
+        *reinterpret_cast<uint4 *>(a.X + (row0 + m) * a.kin + 8 * c) = u;
+    }
+    __syncthreads();
+    // forward: lane holds row m32, columns 64 wave + 32 t + 8 g + 4 h + r for v = 4 g + r
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+        unsigned char *dst = l == 0 ? b1 : (l == 1 ? b2 : b3);
+        f32x16 acc[2];
+        for (int t = 0; t < 2; ++t)
+            for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
+        float4 bias[2][4];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                bias[t][g] = *reinterpret_cast<const float4 *>(a.bias[l] + 64 * wave + 32 * t + 8 * g + 4 * h);
+        if (l == 0) gm.run(acc, a.kin >> 4);
+        else gm.run(acc);
+        if (l < 2) gm.start(a.wf[l + 1], dst, TrainGemm::STEPS, wave, lane);
+        else if (NP == 4) gm.start(a.wk[1], b3, TrainGemm::STEPS, wave, lane);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int n0 = 64 * wave + 32 * t + 8 * g + 4 * h;
+                uint2 u;
+                u.x = f2bf2(fmaxf(acc[t][4 * g] + bias[t][g].x, 0.f), fmaxf(acc[t][4 * g + 1] + bias[t][g].y, 0.f));
+                u.y = f2bf2(fmaxf(acc[t][4 * g + 2] + bias[t][g].z, 0.f), fmaxf(acc[t][4 * g + 3] + bias[t][g].w, 0.f));
+                *reinterpret_cast<uint2 *>(dst + act_off(m32, n0 >> 3) + ((n0 & 7) << 1)) = u;
+            }
+        __syncthreads();
+        if (l < 2) train_store(dst, l == 0 ? a.H1 : a.H2, row0, tid);
+    }
+    // output weights of this thread's 8 columns of dA3, on their way early
+    bf16x8 w4[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) w4[i] = *reinterpret_cast<const bf16x8 *>(a.w4 + ((tid & 63) * NP + i) * 8);
+    // and row tid's targets
+    float q[NP];
+#pragma unroll
+    for (int c = 0; c < NP; ++c)
+        if (tid < kTrainRows && c < a.nout) q[c] = a.q[(row0 + tid) * a.nout + c];
+    // logits: wave w sums hidden units [64 w, 64 w + 64)
+    {
+        f32x16 acc;
+        for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+        for (int s = 4 * wave; s < 4 * wave + 4; ++s) {
+            const bf16x8 w = *reinterpret_cast<const bf16x8 *>(a.wf[3] + (((int64_t)s << 6) + lane) * 8);
+            const bf16x8 x = *reinterpret_cast<const bf16x8 *>(b3 + act_off(m32, 2 * s + h));
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, x, acc, 0, 0, 0);
+        }
+        for (int v = 0; v < 8; ++v) {
+            const int n = 8 * (v >> 2) + 4 * h + (v & 3);
+            if (n < NP) zp[(wave * kTrainRows + m32) * NP + n] = acc[v];
+        }
+    }
+    __syncthreads();
+    if (tid < kTrainRows * NP) {
+        const int m = tid / NP, c = tid % NP;
+        float s = c < a.nout ? a.bias[3][c] : 0.f;
+        for (int w = 0; w < 8; ++w) s += zp[(w * kTrainRows + m) * NP + c];
+        dz[tid] = s;
+    }
+    __syncthreads();
+    if (tid < 64) {
+        // softmax cross-entropy of row tid, and its gradient in place of its logits
+        float l = 0.f;
+        if (tid < kTrainRows) {
+            float *z = dz + tid * NP;
+            float m = -INFINITY;
+            for (int c = 0; c < a.nout; ++c) m = fmaxf(m, z[c]);
+            float s = 0.f;
+            for (int c = 0; c < a.nout; ++c) s += expf(z[c] - m);
+            const float ls = logf(s);
+#pragma unroll
+            for (int c = 0; c < NP; ++c) {
+                if (c < a.nout) {
+                    const float lp = z[c] - m - ls;
+                    const float qc = q[c];
+                    l -= qc * lp;
+                    z[c] = (expf(lp) - qc) / (float)a.B;
+                } else {
+                    z[c] = 0.f;
+                }
+            }
+        }
+        for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
+        if (tid == 0) a.loss_parts[blockIdx.x] = l;
+    }
+    __syncthreads();
+    float *part = a.part + (int64_t)blockIdx.x * a.part_len;
+    float *db = part + (int64_t)kFusedHid * a.nout + a.nout;
+    {
+        // output layer's gradients: this thread's hidden unit against every class
+        float w[NP];
+#pragma unroll
+        for (int c = 0; c < NP; ++c) w[c] = 0.f;
+#pragma unroll 8
+        for (int m = 0; m < kTrainRows; ++m) {
+            const float x = bf2f(*reinterpret_cast<const bf16 *>(b3 + act_off(m, tid >> 3) + ((tid & 7) << 1)));
+#pragma unroll
+            for (int c = 0; c < NP; ++c) w[c] += x * dz[m * NP + c];
+        }
+#pragma unroll
+        for (int c = 0; c < NP; ++c)
+            if (c < a.nout) part[tid * a.nout + c] = w[c];
+        if (tid < a.nout) {
+            float s = 0.f;
+            for (int m = 0; m < kTrainRows; ++m) s += dz[m * NP + tid];
+            part[(int64_t)kFusedHid * a.nout + tid] = s;
+        }
+    }
+    __syncthreads();
+    // dA3 = (dz W4^T) where H3 > 0, in place: 8 columns of 4 rows per thread
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int m = wave + 8 * j;
+        float d[NP];
+#pragma unroll
+        for (int c = 0; c < NP; ++c) d[c] = dz[m * NP + c];
+        uint4 *p = reinterpret_cast<uint4 *>(b3 + act_off(m, tid & 63));
+        float s[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            s[e] = 0.f;
+#pragma unroll
+            for (int c = 0; c < NP; ++c) s[e] += d[c] * bf2f((bf16)w4[(e * NP + c) >> 3][(e * NP + c) & 7]);
+        }
+        uint4 u = *p;
+        u.x = masked_pair(u.x, s[0], s[1]);
+        u.y = masked_pair(u.y, s[2], s[3]);
+        u.z = masked_pair(u.z, s[4], s[5]);
+        u.w = masked_pair(u.w, s[6], s[7]);
+        *p = u;
+    }
+    __syncthreads();
+    train_store(b3, a.dA3, row0, tid);
+    if (NP != 4) gm.start(a.wk[1], b3, TrainGemm::STEPS, wave, lane);
+    db[2 * kFusedHid + tid] = train_colsum(b3, tid);
+    // dA2, dA1
+#pragma unroll
+    for (int l = 1; l >= 0; --l) {
+        unsigned char *dst = l == 1 ? b2 : b1;
+        f32x16 acc[2];
+        for (int t = 0; t < 2; ++t)
+            for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
+        gm.run(acc);
+        if (l == 1) gm.start(a.wk[0], b2, TrainGemm::STEPS, wave, lane);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int n0 = 64 * wave + 32 * t + 8 * g + 4 * h;
+                uint2 *p = reinterpret_cast<uint2 *>(dst + act_off(m32, n0 >> 3) + ((n0 & 7) << 1));
+                uint2 u = *p;
+                u.x = masked_pair(u.x, acc[t][4 * g], acc[t][4 * g + 1]);
+                u.y = masked_pair(u.y, acc[t][4 * g + 2], acc[t][4 * g + 3]);
+                *p = u;
+            }
+        __syncthreads();
+        train_store(dst, l == 1 ? a.dA2 : a.dA1, row0, tid);
+        db[l * kFusedHid + tid] = train_colsum(dst, tid);
+    }
+}
+
+// Weight gradients of the three hidden layers, dW_l [K_l][N] = in_l^T dA_l
+// summed over the batch, in one launch.  Both operands lie with the contracted
+// index (the batch row) outermost, so the tiles are copied to LDS as they are
+// and ds_read_b64_tr_b16 hands each lane its column's consecutive rows: for
+// each 16 lanes, lane i receives element i % 4 of the 8 bytes that lanes
+// i / 4, i / 4 + 4, .. addressed.  Rows of 320 B (256 + 64) put the four rows
+// that 32 lanes read on disjoint banks.  128 x 128 tiles, 64 rows per step,
+// two LDS buffers and two steps more in registers (a step's 16 MFMAs per wave
+// are far shorter than a load).  A batch has far more
+// rows than the gradients have tiles (36 at 64 inputs), so the rows are split
+// to fill the CUs and each split writes its own partial sum.  The split runs
+// fastest in blockIdx.x: workgroups go round the 8 XCDs, so with 8 splits each
+// XCD reads one eighth of the rows into its L2, once for all tiles.
+struct DwArgs {
+    const bf16 *in[3];
+    const bf16 *d[3];
+    int K[3];          // columns of in_l
+    int tile0[4];      // first tile of each layer, total
+    int64_t off[3];    // of dW_l in a partial sum
+    int N;
+    int nsplit;
+    int64_t B, rows;   // rows per split (a multiple of 32)
+    float *part;
+    int64_t part_len;
+};
+
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short bf16x4;
+constexpr int kDwStep = 64, kDwLd = 160;
+
+__device__ __forceinline__ bf16x8 tr_fragment(const bf16 *tile, int kk, int col, int lane) {
+    const int g = lane >> 4, i = lane & 15;
+    const bf16 *p = tile + (kk + 8 * (g >> 1) + (i >> 2)) * kDwLd + col + 16 * (g & 1) + 4 * (i & 3);
+    typedef __attribute__((address_space(3))) bf16x4 lds4;
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4 *)p);
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4 *)(p + 4 * kDwLd));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+__global__ void __launch_bounds__(256) mlp_dw_kernel(DwArgs a) {
+    __shared__ __align__(16) bf16 As[2][kDwStep * kDwLd];
+    __shared__ __align__(16) bf16 Bs[2][kDwStep * kDwLd];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int split = blockIdx.x % a.nsplit, tile = blockIdx.x / a.nsplit;
+    // selected, not indexed: an indexed argument would be copied to scratch
+    const bool l2 = tile >= a.tile0[2], l1 = tile >= a.tile0[1];
+    const int t = tile - (l2 ? a.tile0[2] : l1 ? a.tile0[1] : 0), nt = a.N / 128;
+    const int m0 = (t / nt) * 128, n0 = (t % nt) * 128;
+    const int K = l2 ? a.K[2] : l1 ? a.K[1] : a.K[0];
+    const int N = a.N;
+    const bf16 *in = l2 ? a.in[2] : l1 ? a.in[1] : a.in[0], *d = l2 ? a.d[2] : l1 ? a.d[1] : a.d[0];
+    const int64_t r0 = (int64_t)split * a.rows;
+    const int rows = (int)(min(a.B, r0 + a.rows) - r0);
+    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    // this thread's chunks: rows tr + 16 j of a step, columns tx .. tx + 7 (K is
+    // a multiple of 32, so a chunk is inside or outside as a whole); rows and
+    // columns outside are read at a valid place and stored as zeros
+    const int tr = tid >> 4, tx = (tid & 15) * 8;
+    const bool inside = m0 + tx < K;
+    const bf16 *pa = in + r0 * K + (inside ? m0 + tx : 0), *pb = d + r0 * N + n0 + tx;
+    struct Step {
+        uint4 a[4], b[4];
+    };
+    auto fetch = [&](Step &s, int k0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int r = min(k0 + tr + 16 * j, rows - 1);
+            s.a[j] = *reinterpret_cast<const uint4 *>(pa + (int64_t)r * K);
+            s.b[j] = *reinterpret_cast<const uint4 *>(pb + (int64_t)r * N);
+        }
+    };
+    auto stash = [&](const Step &s, int k0, int buf) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const bool row = k0 + tr + 16 * j < rows;
+            const uint32_t ma = row && inside ? ~0u : 0u, mb = row ? ~0u : 0u;
+            bf16 *o = &As[buf][(tr + 16 * j) * kDwLd + tx], *q = &Bs[buf][(tr + 16 * j) * kDwLd + tx];
+            *reinterpret_cast<uint4 *>(o) = make_uint4(s.a[j].x & ma, s.a[j].y & ma, s.a[j].z & ma, s.a[j].w & ma);
+            *reinterpret_cast<uint4 *>(q) = make_uint4(s.b[j].x & mb, s.b[j].y & mb, s.b[j].z & mb, s.b[j].w & mb);
+        }
+    };
+    f32x16 acc[2][2];
+    for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < 2; ++j)
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+    auto multiply = [&](int buf) {
+#pragma unroll
+        for (int kk = 0; kk < kDwStep; kk += 16) {
+            bf16x8 x[2], y[2];
+            for (int i = 0; i < 2; ++i) x[i] = tr_fragment(As[buf], kk, wm + 32 * i, lane);
+            for (int j = 0; j < 2; ++j) y[j] = tr_fragment(Bs[buf], kk, wn + 32 * j, lane);
+            for (int i = 0; i < 2; ++i)
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[i], y[j], acc[i][j], 0, 0, 0);
+        }
+    };
+    // step k in LDS buffer k / 64 % 2, the two after it in registers or on their way
+    Step s0, s1;
+    // (the scheduling barriers keep the loads in this order: mixed, a wait for
+    // the older step is a wait for all of them)
+    fetch(s0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(s1, kDwStep);
+    __builtin_amdgcn_sched_barrier(0);
+    stash(s0, 0, 0);
+    fetch(s0, 2 * kDwStep);
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+    for (int k0 = 0; k0 < rows; k0 += 2 * kDwStep) {
+        stash(s1, k0 + kDwStep, 1);
+        fetch(s1, k0 + 3 * kDwStep);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(0);
+        __syncthreads();
+        stash(s0, k0 + 2 * kDwStep, 0);
+        fetch(s0, k0 + 4 * kDwStep);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(1);
+        __syncthreads();
+    }
+    float *out = a.part + (int64_t)split * a.part_len + (l2 ? a.off[2] : l1 ? a.off[1] : a.off[0]);
+    for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < 2; ++j) {
+            const int col = n0 + wn + j * 32 + (lane & 31);
+            for (int v = 0; v < 16; ++v) {
+                const int row = m0 + wm + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+                if (row < K) out[(int64_t)row * N + col] = acc[i][j][v];
+            }
+        }
+}
+
+// Sums the partial gradients, always in the same order: the hidden layers'
+// weights over the row splits (one thread per parameter), the rest over the
+// row tiles (32 parameters x 8 groups of tiles per workgroup).
+struct GradSumArgs {
+    const float *wpart, *rpart;
+    int64_t wlen, rlen;         // parameters in a partial sum of each kind
+    int nsplit, ntile;
+    int64_t woff[3], wend[3];   // of each hidden layer's weights in `grad`, and running totals in a partial sum
+    int64_t roff[5], rend[5];   // of W4, b4, b1, b2, b3
+    unsigned wblocks;
+    float *grad;
+};
+
+__global__ void __launch_bounds__(256) mlp_grad_sum_kernel(GradSumArgs a) {
+    if (blockIdx.x < a.wblocks) {
+        const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+        if (i >= a.wlen) return;
+        float s = 0.f;
+#pragma unroll 4
+        for (int k = 0; k < a.nsplit; ++k) s += a.wpart[(int64_t)k * a.wlen + i];
+        int g = 0;
+        while (i >= a.wend[g]) ++g;
+        a.grad[a.woff[g] + i - (g ? a.wend[g - 1] : 0)] = s;
+        return;
+    }
+    __shared__ float red[8][32];
+    const int64_t i = (int64_t)(blockIdx.x - a.wblocks) * 32 + (threadIdx.x & 31);
+    const int grp = threadIdx.x >> 5;
+    float s = 0.f;
+    if (i < a.rlen)
+#pragma unroll 8
+        for (int k = grp; k < a.ntile; k += 8) s += a.rpart[(int64_t)k * a.rlen + i];
+    red[grp][threadIdx.x & 31] = s;
+    __syncthreads();
+    if (grp || i >= a.rlen) return;
+    s = 0.f;
+    for (int k = 0; k < 8; ++k) s += red[k][threadIdx.x & 31];
+    int g = 0;
+    while (i >= a.rend[g]) ++g;
+    a.grad[a.roff[g] + i - (g ? a.rend[g - 1] : 0)] = s;
 }
 
 // Wt[n][k] = W[k][n] for the three hidden-layer weight matrices.
@@ -499,28 +983,30 @@ __global__ void out_bwd_dx_kernel(const float *__restrict__ dz, const bf16 *__re
     dA[i] = bf2f(H[i]) > 0.f ? f2bf(s) : (bf16)0;
 }
 
-// dW[k][c] = sum_b H[b][k] dz[b][c] (one thread per (k, c), loop over b).
+// Partial sums over a tile of kSumRows rows, as mlp_train_rows_kernel leaves
+// them: the output layer's gradients dW4[k][c] = sum_b H[b][k] dz[b][c] and
+// db4[c], and the column sums of a hidden layer's dA.
+constexpr int kSumRows = 32;
+
 __global__ void out_bwd_dw_kernel(const bf16 *__restrict__ H, const float *__restrict__ dz, int64_t B, int hid,
-                                  int nout, float *__restrict__ dW) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= hid * nout) return;
+                                  int nout, float *__restrict__ part, int64_t part_len) {
+    const int64_t r0 = (int64_t)blockIdx.x * kSumRows, r1 = min(B, r0 + kSumRows);
+    const int i = blockIdx.y * blockDim.x + threadIdx.x;
+    if (i >= (hid + 1) * nout) return;
     const int k = i / nout, c = i - k * nout;
     float s = 0.f;
-    for (int64_t b = 0; b < B; ++b) s += bf2f(H[b * hid + k]) * dz[b * nout + c];
-    dW[i] = s;
+    for (int64_t b = r0; b < r1; ++b) s += (k < hid ? bf2f(H[b * hid + k]) : 1.f) * dz[b * nout + c];
+    part[blockIdx.x * part_len + i] = s;
 }
 
-// Column sums: db[c] = sum_b D[b][c] (BF16 or FP32 input).
-template <typename T>
-__global__ void colsum_kernel(const T *__restrict__ D, int64_t B, int n, float *__restrict__ db) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void colsum_kernel(const bf16 *__restrict__ D, int64_t B, int n, float *__restrict__ part,
+                              int64_t part_len) {
+    const int64_t r0 = (int64_t)blockIdx.x * kSumRows, r1 = min(B, r0 + kSumRows);
+    const int c = blockIdx.y * blockDim.x + threadIdx.x;
     if (c >= n) return;
     float s = 0.f;
-    for (int64_t b = 0; b < B; ++b) {
-        if constexpr (sizeof(T) == 2) s += bf2f(D[b * n + c]);
-        else s += D[b * n + c];
-    }
-    db[c] = s;
+    for (int64_t b = r0; b < r1; ++b) s += bf2f(D[b * n + c]);
+    part[blockIdx.x * part_len + c] = s;
 }
 
 // Adam on the FP32 master parameters; refreshes the BF16 copy.
@@ -599,6 +1085,8 @@ struct tqec_mlp {
     // fused inference (hidden width 512): fragment-ordered BF16 weights of the
     // four layers, rebuilt after every weight change
     bf16 *wf[4] = {nullptr, nullptr, nullptr, nullptr};
+    bf16 *wk[2] = {nullptr, nullptr};   // of the two inner hidden layers, for the backward pass
+    bf16 *w4 = nullptr;                 // output layer's rows, padded
     bool wf_stale = true;
     bool fused = true;             // forward / gate on the fused kernel where it applies
     int64_t zcap = 0;              // rows the logits buffer z holds
@@ -609,6 +1097,10 @@ struct tqec_mlp {
     bf16 *X = nullptr, *H1 = nullptr, *H2 = nullptr, *H3 = nullptr, *dA = nullptr, *dB = nullptr;
     float *z = nullptr, *dz = nullptr, *loss_parts = nullptr;
     int64_t loss_cap = 0;
+    // partial gradients: hidden weights per row split, the rest per row tile
+    float *wpart = nullptr, *rpart = nullptr;
+    size_t wpart_cap = 0, rpart_cap = 0;
+    bool train_attr = false;
 };
 
 namespace {
@@ -622,6 +1114,13 @@ int64_t param_count(int kin, int hid, int nout, int64_t off[8]) {
         o += sizes[i];
     }
     return o;
+}
+
+bool fused_ok(const tqec_mlp *p) { return p->hid == kFusedHid && p->nout <= 32 && p->kin <= kFusedHid; }
+
+// Partial sums of the loss that a training pass over B rows leaves.
+int64_t loss_blocks(const tqec_mlp *p, int64_t B) {
+    return fused_ok(p) ? B / kTrainRows : (B + 255) / 256;
 }
 
 int ensure_cap(tqec_mlp *p, int64_t B) {
@@ -639,7 +1138,7 @@ int ensure_cap(tqec_mlp *p, int64_t B) {
     TQM_HIP(hipMalloc((void **)&p->z, (size_t)B * p->nout * sizeof(float)));
     p->zcap = B;
     TQM_HIP(hipMalloc((void **)&p->dz, (size_t)B * p->nout * sizeof(float)));
-    const int64_t nb = (B + 255) / 256;
+    const int64_t nb = loss_blocks(p, B);
     if (p->loss_cap < nb) {
         if (p->loss_parts) (void)hipFree(p->loss_parts);
         TQM_HIP(hipMalloc((void **)&p->loss_parts, (size_t)nb * sizeof(float)));
@@ -649,13 +1148,45 @@ int ensure_cap(tqec_mlp *p, int64_t B) {
     return TQEC_OK;
 }
 
-template <bool AT, bool BT, int EPI>
 void gemm(const GemmArgs &a, hipStream_t st) {
     dim3 grid((a.N + BN - 1) / BN, (a.M + BM - 1) / BM);
-    hipLaunchKernelGGL((gemm_bf16_kernel<AT, BT, EPI>), grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL(gemm_bf16_kernel, grid, dim3(256), 0, st, a);
 }
 
-bool fused_ok(const tqec_mlp *p) { return p->hid == kFusedHid && p->nout <= 32 && p->kin <= kFusedHid; }
+int padded_classes(const tqec_mlp *p) { return p->nout <= 4 ? 4 : kTrainMaxOut; }
+
+// Fragment-ordered weights of the fused kernels, rebuilt after a weight change.
+int pack_weights(tqec_mlp *p, hipStream_t st) {
+    if (!p->wf_stale && p->wf[0]) return TQEC_OK;
+    const int kdim[4] = {p->kin, p->hid, p->hid, p->hid};
+    PackArgs a{};
+    int64_t end = 0;
+    for (int g = 0; g < 6; ++g) {
+        const int l = g < 4 ? g : g - 3;   // layers 1..4 forward, then 2 and 3 backward
+        const int npad = l < 3 ? p->hid : 32;
+        const int64_t n = (int64_t)kdim[l] * npad;
+        bf16 **dst = g < 4 ? &p->wf[g] : &p->wk[g - 4];
+        if (!*dst) TQM_HIP(hipMalloc((void **)dst, (size_t)n * sizeof(bf16)));
+        a.W[g] = p->wb + p->off[2 * l];
+        a.out[g] = *dst;
+        a.end[g] = end += n;
+        a.N[g] = l < 3 ? p->hid : p->nout;
+        a.tiles[g] = npad / 32;
+        a.kind[g] = g >= 4;
+    }
+    const int np = padded_classes(p);
+    if (!p->w4) TQM_HIP(hipMalloc((void **)&p->w4, (size_t)p->hid * np * sizeof(bf16)));
+    a.W[6] = p->wb + p->off[6];
+    a.out[6] = p->w4;
+    a.end[6] = end += (int64_t)p->hid * np;
+    a.N[6] = p->nout;
+    a.tiles[6] = np;
+    a.kind[6] = 2;
+    hipLaunchKernelGGL(pack_fused_kernel, dim3((unsigned)((end + 255) / 256)), dim3(256), 0, st, a);
+    TQM_HIP(hipGetLastError());
+    p->wf_stale = false;
+    return TQEC_OK;
+}
 
 // Logits only (no activations kept): the fused kernel, one workgroup per 128 rows.
 int forward_fused(tqec_mlp *p, const uint8_t *d_syn, int64_t B, hipStream_t st) {
@@ -673,17 +1204,8 @@ int forward_fused(tqec_mlp *p, const uint8_t *d_syn, int64_t B, hipStream_t st) 
                                     (int)lds));
         p->fused_attr = true;
     }
-    if (p->wf_stale || !p->wf[0]) {
-        const int kdim[4] = {p->kin, p->hid, p->hid, p->hid};
-        for (int l = 0; l < 4; ++l) {
-            const int npad = l < 3 ? p->hid : 32;
-            if (!p->wf[l]) TQM_HIP(hipMalloc((void **)&p->wf[l], (size_t)kdim[l] * npad * sizeof(bf16)));
-            const int64_t n = (int64_t)kdim[l] * npad;
-            hipLaunchKernelGGL(pack_fused_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                               p->wb + p->off[2 * l], kdim[l], l < 3 ? p->hid : p->nout, npad, p->wf[l]);
-        }
-        p->wf_stale = false;
-    }
+    int rc;
+    if ((rc = pack_weights(p, st))) return rc;
     const unsigned grid = (unsigned)((B + kFusedRows - 1) / kFusedRows);
     const float *b[4] = {p->w + p->off[1], p->w + p->off[3], p->w + p->off[5], p->w + p->off[7]};
     hipLaunchKernelGGL(mlp_fused_fwd_kernel<8>, dim3(grid), dim3(512), lds, st, d_syn, B, p->n_in, p->kin, p->wf[0],
@@ -751,55 +1273,158 @@ int forward(tqec_mlp *p, const uint8_t *d_syn, int64_t B, hipStream_t st, bool k
     return TQEC_OK;
 }
 
-// Gradients of the mean soft cross-entropy into p->g (FP32, flat layout).
-int backward(tqec_mlp *p, const float *d_q, int64_t B, hipStream_t st) {
+int grow(float **buf, size_t *cap, size_t need) {
+    if (*cap >= need) return TQEC_OK;
+    if (*buf) TQM_HIP(hipFree(*buf));
+    *buf = nullptr;
+    *cap = 0;
+    TQM_HIP(hipMalloc((void **)buf, need * sizeof(float)));
+    *cap = need;
+    return TQEC_OK;
+}
+
+int64_t row_part_len(const tqec_mlp *p) { return (int64_t)(p->hid + 1) * p->nout + 3 * (int64_t)p->hid; }
+
+// Weight gradients of the hidden layers from their inputs and dA1..dA3 (d[l]
+// the gradient at layer l + 1's pre-activation), then all partial sums into
+// `grad`.
+int weight_gradients(tqec_mlp *p, const bf16 *const d[3], int64_t B, int ntile, float *grad, hipStream_t st) {
+    DwArgs w{};
+    const bf16 *in[3] = {p->X, p->H1, p->H2};
+    const int kdim[3] = {p->kin, p->hid, p->hid};
+    GradSumArgs g{};
+    int tiles = 0;
+    int64_t len = 0;
+    for (int l = 0; l < 3; ++l) {
+        w.in[l] = in[l];
+        w.d[l] = d[l];
+        w.K[l] = kdim[l];
+        w.tile0[l] = tiles;
+        w.off[l] = len;
+        tiles += (kdim[l] + 127) / 128 * (p->hid / 128);
+        len += (int64_t)kdim[l] * p->hid;
+        g.woff[l] = p->off[2 * l];
+        g.wend[l] = len;
+    }
+    w.tile0[3] = tiles;
+    w.N = p->hid;
+    w.B = B;
+    w.part_len = len;
+    // one split per XCD, at least four steps of rows in each
+    int64_t split = std::max<int64_t>(1, std::min<int64_t>(8, B / (4 * kDwStep)));
+    w.rows = ((B + split - 1) / split + 31) / 32 * 32;
+    split = (B + w.rows - 1) / w.rows;
+    int rc;
+    if ((rc = grow(&p->wpart, &p->wpart_cap, (size_t)(split * len)))) return rc;
+    w.part = p->wpart;
+    w.nsplit = (int)split;
+    hipLaunchKernelGGL(mlp_dw_kernel, dim3((unsigned)(tiles * split)), dim3(256), 0, st, w);
+    g.wpart = p->wpart;
+    g.rpart = p->rpart;
+    g.wlen = len;
+    g.rlen = row_part_len(p);
+    g.nsplit = (int)split;
+    g.ntile = ntile;
+    const int64_t rn[5] = {(int64_t)p->hid * p->nout, p->nout, p->hid, p->hid, p->hid};
+    const int ri[5] = {6, 7, 1, 3, 5};
+    int64_t end = 0;
+    for (int i = 0; i < 5; ++i) {
+        g.roff[i] = p->off[ri[i]];
+        g.rend[i] = end += rn[i];
+    }
+    g.wblocks = (unsigned)((len + 255) / 256);
+    g.grad = grad;
+    hipLaunchKernelGGL(mlp_grad_sum_kernel, dim3(g.wblocks + (unsigned)((g.rlen + 31) / 32)), dim3(256), 0, st, g);
+    TQM_HIP(hipGetLastError());
+    return TQEC_OK;
+}
+
+// Forward and backward pass of a network that the fused kernels cover.
+int train_fused(tqec_mlp *p, const uint8_t *d_syn, const float *d_q, int64_t B, float *grad, hipStream_t st) {
+    int rc;
+    if ((rc = ensure_cap(p, B))) return rc;
+    if ((rc = pack_weights(p, st))) return rc;
+    const int64_t tiles = B / kTrainRows;
+    if ((rc = grow(&p->rpart, &p->rpart_cap, (size_t)(tiles * row_part_len(p))))) return rc;
+    if (!p->train_attr) {
+        TQM_HIP(hipFuncSetAttribute((const void *)mlp_train_rows_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    kTrainLds));
+        TQM_HIP(hipFuncSetAttribute((const void *)mlp_train_rows_kernel<kTrainMaxOut>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, kTrainLds));
+        p->train_attr = true;
+    }
+    TrainArgs a{};
+    a.syn = d_syn;
+    a.q = d_q;
+    a.B = B;
+    a.n_in = p->n_in;
+    a.kin = p->kin;
+    a.nout = p->nout;
+    for (int l = 0; l < 4; ++l) {
+        a.wf[l] = p->wf[l];
+        a.bias[l] = p->w + p->off[2 * l + 1];
+    }
+    a.wk[0] = p->wk[0];
+    a.wk[1] = p->wk[1];
+    a.w4 = p->w4;
+    a.X = p->X;
+    a.H1 = p->H1;
+    a.H2 = p->H2;
+    a.dA1 = p->H3;   // H3 itself never leaves the tile
+    a.dA2 = p->dB;
+    a.dA3 = p->dA;
+    a.part = p->rpart;
+    a.part_len = row_part_len(p);
+    a.loss_parts = p->loss_parts;
+    if (p->nout <= 4)
+        hipLaunchKernelGGL(mlp_train_rows_kernel<4>, dim3((unsigned)tiles), dim3(512), kTrainLds, st, a);
+    else
+        hipLaunchKernelGGL(mlp_train_rows_kernel<kTrainMaxOut>, dim3((unsigned)tiles), dim3(512), kTrainLds, st, a);
+    const bf16 *d[3] = {a.dA1, a.dA2, a.dA3};
+    return weight_gradients(p, d, B, (int)tiles, grad, st);
+}
+
+// Gradients of the mean soft cross-entropy into `grad` (FP32, flat layout),
+// layer by layer after forward().
+int backward(tqec_mlp *p, const float *d_q, int64_t B, float *grad, hipStream_t st) {
     const int64_t nb = (B + 255) / 256;
+    const int64_t tiles = (B + kSumRows - 1) / kSumRows, plen = row_part_len(p);
+    int rc;
+    if ((rc = grow(&p->rpart, &p->rpart_cap, (size_t)(tiles * plen)))) return rc;
     hipLaunchKernelGGL(xent_kernel, dim3((unsigned)nb), dim3(256), 0, st, p->z, d_q, B, p->nout, p->dz, p->loss_parts);
     // output layer
-    hipLaunchKernelGGL(out_bwd_dw_kernel, dim3((unsigned)((p->hid * p->nout + 255) / 256)), dim3(256), 0, st, p->H3,
-                       p->dz, B, p->hid, p->nout, p->g + p->off[6]);
-    hipLaunchKernelGGL((colsum_kernel<float>), dim3(1), dim3(64), 0, st, p->dz, B, p->nout, p->g + p->off[7]);
+    const int64_t no = (int64_t)(p->hid + 1) * p->nout;
+    hipLaunchKernelGGL(out_bwd_dw_kernel, dim3((unsigned)tiles, (unsigned)((no + 255) / 256)), dim3(256), 0, st, p->H3,
+                       p->dz, B, p->hid, p->nout, p->rpart, plen);
     const int64_t nh = B * p->hid;
     hipLaunchKernelGGL(out_bwd_dx_kernel, dim3((unsigned)((nh + 255) / 256)), dim3(256), 0, st, p->dz,
                        p->wb + p->off[6], p->H3, B, p->hid, p->nout, p->dA);
-    // hidden layers 3, 2, 1: dA holds dL/d(pre-activation) of layer l
+    // hidden layers 3, 2, 1: d[l] holds dL/d(pre-activation) of layer l + 1;
+    // H3 has been read when dA1 takes its place
     const bf16 *hin[3] = {p->X, p->H1, p->H2};
-    const int kdim[3] = {p->kin, p->hid, p->hid};
-    bf16 *cur = p->dA, *nxt = p->dB;
+    bf16 *d[3] = {p->H3, p->dB, p->dA};
     for (int l = 2; l >= 0; --l) {
-        // dW_l[K][N] = in_l^T [K][B] * dA [B][N]
-        GemmArgs w{};
-        w.A = hin[l];
-        w.B = cur;
-        w.M = kdim[l];
-        w.N = p->hid;
-        w.K = (int)B;
-        w.lda = kdim[l];
-        w.ldb = p->hid;
-        w.ldc = p->hid;
-        w.outf = p->g + p->off[2 * l];
-        gemm<true, false, kEpiF32>(w, st);
-        hipLaunchKernelGGL((colsum_kernel<bf16>), dim3((unsigned)((p->hid + 255) / 256)), dim3(256), 0, st, cur, B,
-                           p->hid, p->g + p->off[2 * l + 1]);
+        hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)tiles, (unsigned)((p->hid + 255) / 256)), dim3(256), 0, st, d[l],
+                           B, p->hid, p->rpart + no + (int64_t)l * p->hid, plen);
         if (l > 0) {
             // d in_l [B][K] = dA [B][N] * W_l^T (W_l stored [K][N]), masked by in_l > 0
             GemmArgs x{};
-            x.A = cur;
+            x.A = d[l];
             x.B = p->wb + p->off[2 * l];
             x.M = (int)B;
-            x.N = kdim[l];
+            x.N = p->hid;
             x.K = p->hid;
             x.lda = p->hid;
             x.ldb = p->hid;
-            x.ldc = kdim[l];
+            x.ldc = p->hid;
             x.mask = hin[l];
-            x.outb = nxt;
-            gemm<false, true, kEpiMaskBf16>(x, st);
-            std::swap(cur, nxt);
+            x.outb = d[l - 1];
+            gemm(x, st);
         }
     }
     TQM_HIP(hipGetLastError());
-    return TQEC_OK;
+    const bf16 *dc[3] = {d[0], d[1], d[2]};
+    return weight_gradients(p, dc, B, (int)tiles, grad, st);
 }
 
 // Training reduces over the batch inside the weight-gradient GEMM, whose K
@@ -890,11 +1515,15 @@ int tqec_mlp_gradients(tqec_mlp *p, const uint8_t *d_syn, const float *d_targets
     if ((rc = check_batch(p, B, true))) return rc;
     if (!d_syn || !d_targets) return fail(TQEC_ENULL, "null device pointer");
     hipStream_t st = (hipStream_t)stream;
-    if ((rc = forward(p, d_syn, B, st))) return rc;
-    if ((rc = backward(p, d_targets, B, st))) return rc;
-    if (d_grad) TQM_HIP(hipMemcpyAsync(d_grad, p->g, (size_t)p->nparams * 4, hipMemcpyDeviceToDevice, st));
+    float *grad = d_grad ? d_grad : p->g;
+    if (fused_ok(p)) {
+        if ((rc = train_fused(p, d_syn, d_targets, B, grad, st))) return rc;
+    } else {
+        if ((rc = forward(p, d_syn, B, st))) return rc;
+        if ((rc = backward(p, d_targets, B, grad, st))) return rc;
+    }
     if (h_loss) {
-        const int64_t nb = (B + 255) / 256;
+        const int64_t nb = loss_blocks(p, B);
         std::vector<float> parts(nb);
         TQM_HIP(hipMemcpyAsync(parts.data(), p->loss_parts, nb * 4, hipMemcpyDeviceToHost, st));
         TQM_HIP(hipStreamSynchronize(st));
@@ -966,7 +1595,7 @@ void tqec_mlp_destroy(tqec_mlp *p) {
     if (!p) return;
     void *bufs[] = {p->w,  p->g,  p->m,  p->v,  p->wb, p->X,  p->H1,         p->H2,    p->H3,
                     p->dA, p->dB, p->z,  p->dz, p->loss_parts, p->wt[0], p->wt[1], p->wt[2],
-                    p->wf[0], p->wf[1], p->wf[2], p->wf[3]};
+                    p->wf[0], p->wf[1], p->wf[2], p->wf[3], p->wk[0], p->wk[1], p->w4, p->wpart, p->rpart};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     delete p;
