@@ -353,9 +353,12 @@ void tqec_mixed_destroy(tqec_mixed *m);
 #define TQEC_SPEC_MFMA32 64        /* SPEC_F32 tiles of one syndrome (LDS or slab):
                                       GEMM-shaped steps (M, N >= 16, K >= 4, or
                                       M, N >= 32, K >= 2 per syndrome) on FP32
-                                      MFMA with FP32 operands;
+                                      MFMA with FP32 operands, contractions of 64 or
+                                      more terms into at most 256 outputs split over
+                                      the threads;
                                       within the FP32 tolerance, not bit-identical
-                                      (summation order)                              */
+                                      (summation order); the default of plans that do
+                                      not fit registers and have such steps          */
 
 /* Source of the plan-specialised kernel for a tile configuration
  * (inspection and offline compilation checks); `flags` as above, with the

@@ -21,9 +21,128 @@ namespace {
 size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 struct Layout {
-    size_t work = 0, tab = 0, mx = 0, ex = 0, syn = 0, low = 0, total = 0;
+    size_t work = 0, tab = 0, mx = 0, ex = 0, syn = 0, low = 0, red = 0, total = 0;
     size_t tab_entries = 0;
 };
+
+// x spread onto the given bit positions: bit t of x goes to bits[t].
+uint32_t pdep(uint32_t x, const std::vector<int> &bits) {
+    uint32_t r = 0;
+    for (size_t j = 0; j < bits.size(); ++j) r |= ((x >> j) & 1u) << bits[j];
+    return r;
+}
+
+// ---- steps with few outputs and a long contraction -----------------------
+//
+// One lane per output leaves most of a workgroup idle and makes each output a
+// serial chain of 2^nk multiply-adds (toric L=5 ends in 64 outputs of 2^18
+// terms: 38% of its time).  In the configurations that need not keep the
+// generic kernel's order of summation (mfma32), such a step gives every thread
+// a block of up to 64 outputs and a share of the contraction: the block's
+// operand values are loaded once per k, consecutive threads take consecutive
+// k, and the partial sums meet in a shuffle tree and, across waves, in LDS.
+// Measured: that step of toric L=5 24.3 -> 3.4 M cycles (its 16.8 MB per
+// syndrome at 5.6 TB/s over the chip, the rate of a large copy), 512 syndromes
+// 29.2 -> 20.9 ms with the smaller MFMA blocks of emit_outputs_mfma32; the
+// circuit-level d=3, 3-round plan 400 -> 358 us per 16,384.
+
+// Output bits held per thread, -1 when the step does not run this way.  The
+// block is as large as leaves each thread at least eight terms.
+int split_k_block(const StepDesc &st, const SpecCfg &cfg) {
+    if (!cfg.mfma32 || cfg.fp64 || cfg.glog != 0 || st.rc > 8 || st.nk < 6) return -1;
+    if ((1 << st.rc) > cfg.threads) return -1;
+    for (int rb = std::min(st.rc, 6); rb >= 0; --rb)
+        if ((int64_t)(cfg.threads >> (st.rc - rb)) * 8 <= (int64_t(1) << st.nk)) return rb;
+    return -1;
+}
+
+// LDS floats of the partial sums: one per output and wave of its threads.
+size_t split_k_entries(const CompiledPlan &cp, const SpecCfg &cfg) {
+    size_t n = 0;
+    for (const StepDesc &st : cp.steps) {
+        const int rb = split_k_block(st, cfg);
+        if (rb < 0) continue;
+        const int thr = cfg.threads >> (st.rc - rb);   // threads sharing a block
+        n = std::max(n, (size_t)std::max(1, thr / 64) << st.rc);
+    }
+    return n;
+}
+
+// ---- slab kernels: the smaller intermediates in LDS ----------------------
+//
+// A slab plan's steps are bound by memory traffic, and the widest few tensors
+// make the slab necessary while most of the traffic is in smaller ones, so as
+// many intermediates as fit live in LDS instead, each from the step that makes
+// it to the step that reads it.  The LDS of a CU is divided among the eight
+// waves (two per SIMD) that a slab kernel's registers allow.  Measured with
+// 256 threads (76 KB): circuit-level d=5, 2 rounds 2.79 -> 2.22 ms per 4,096
+// (it ran at 4.7 TB/s of HBM traffic, 34% of it in tensors of at most 2^13
+// entries), toric L=3 772 -> 594 us per 8,192; toric L=5, whose traffic is in
+// its 2^21-entry tensors, is unchanged.  Fewer workgroups with smaller slabs
+// in all (171 MB, less than the memory-side cache) changed nothing.
+struct Places {
+    std::vector<int64_t> lds;                // per step: output's LDS entry offset (per syndrome), -1 in the slab
+    std::vector<std::array<int, 2>> prod;    // per step: steps that made its operands, -1 for tables
+    int64_t entries = 0;                     // LDS entries per syndrome
+};
+
+constexpr size_t kSlabLds = 152 * 1024;      // of 160 KB per CU, the rest for scales and syndromes
+
+Places slab_places(const CompiledPlan &cp, const SpecCfg &cfg) {
+    const int ns = (int)cp.steps.size();
+    Places P;
+    P.lds.assign(ns, -1);
+    P.prod.assign(ns, {-1, -1});
+    std::vector<int> last(ns, ns);           // step that reads the output (the root: after the last)
+    for (int s = 0; s < ns; ++s)
+        for (int side = 0; side < 2; ++side) {
+            const OperandDesc &op = side ? cp.steps[s].b : cp.steps[s].a;
+            if (op.kind != kInter) continue;
+            for (int j = s - 1; j >= 0; --j)
+                if (cp.steps[j].c_off == op.off) {
+                    P.prod[s][side] = j;
+                    last[j] = s;
+                    break;
+                }
+        }
+    if (!cfg.slab || cfg.fp64) return P;
+    const int64_t room = (int64_t)(kSlabLds * std::min(cfg.threads, 512) / 512 / 4) >> cfg.glog;
+    std::vector<int> order(ns);
+    for (int s = 0; s < ns; ++s) order[s] = s;
+    int64_t best = 0;
+    for (int rule = 0; rule < 2; ++rule) {
+        // smallest tensors first, or shortest-lived first
+        std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+            const int rx = cp.steps[x].rc, ry = cp.steps[y].rc, lx = last[x] - x, ly = last[y] - y;
+            return rule == 0 ? std::make_pair(rx, lx) < std::make_pair(ry, ly) : std::make_pair(lx, -rx) < std::make_pair(ly, -ry);
+        });
+        std::vector<int64_t> at(ns, -1);
+        int64_t placed = 0, top = 0;
+        for (int s : order) {
+            const int64_t size = int64_t(1) << cp.steps[s].rc;
+            // lowest gap between the tensors that live at the same time
+            std::vector<std::pair<int64_t, int64_t>> busy;
+            for (int j = 0; j < ns; ++j)
+                if (at[j] >= 0 && j <= last[s] && s <= last[j]) busy.emplace_back(at[j], at[j] + (int64_t(1) << cp.steps[j].rc));
+            std::sort(busy.begin(), busy.end());
+            int64_t off = 0;
+            for (auto &b : busy) {
+                if (off + size <= b.first) break;
+                off = std::max(off, b.second);
+            }
+            if (off + size > room) continue;
+            at[s] = off;
+            placed += size;
+            top = std::max(top, off + size);
+        }
+        if (placed > best) {
+            best = placed;
+            P.lds = at;
+            P.entries = top;
+        }
+    }
+    return P;
+}
 
 Layout layout(const CompiledPlan &cp, const SpecCfg &cfg) {
     const size_t G = size_t(1) << cfg.glog;
@@ -33,6 +152,7 @@ Layout layout(const CompiledPlan &cp, const SpecCfg &cfg) {
     size_t off = 0;
     L.work = off;
     if (!cfg.slab) off += round_up((size_t)std::max<int64_t>(1, cp.ws_entries) * G * elem, 16);
+    else off += round_up((size_t)slab_places(cp, cfg).entries * G * elem, 16);
     L.tab = off;
     if (cfg.tab_lds) off += round_up(std::max<size_t>(1, L.tab_entries) * elem, 16);
     L.mx = off;
@@ -43,6 +163,9 @@ Layout layout(const CompiledPlan &cp, const SpecCfg &cfg) {
     off += round_up((size_t)std::max(1, cp.n_syn) * G, 4);
     L.low = off;
     if (!cfg.fp64) off += G * 4;
+    off = round_up(off, 16);
+    L.red = off;
+    off += split_k_entries(cp, cfg) * 4;
     L.total = round_up(off, 16);
     return L;
 }
@@ -64,9 +187,11 @@ std::string gather_expr(const OperandDesc &op) {
 }
 
 // Base pointer of an operand (fused_base).
-void emit_base(std::ostringstream &o, const char *name, const OperandDesc &op, size_t const_n) {
+// `lds`: entry offset of an intermediate that a slab kernel keeps in LDS, or -1.
+void emit_base(std::ostringstream &o, const char *name, const OperandDesc &op, size_t const_n, int64_t lds) {
     if (op.kind == kInter) {
-        o << "    const T *" << name << " = work + " << ((long long)op.off << 0) << " * G + g;\n";
+        o << "    const T *" << name << " = " << (lds >= 0 ? "lwork + " : "work + ")
+          << (long long)(lds >= 0 ? lds : op.off) << " * G + g;\n";
     } else if (op.kind == kConst) {
         o << "    const T *" << name << " = tab + " << (long long)op.off << ";\n";
     } else {
@@ -283,6 +408,8 @@ void emit_outputs(std::ostringstream &o, const StepDesc &st, int cstep, int bloc
     o << "    }\n";
 }
 
+void emit_outputs_split_k(std::ostringstream &o, const StepDesc &st, int threads, int rb);
+
 // Bits of `mask` (ascending).
 std::vector<int> bits_of(uint32_t mask) {
     std::vector<int> v;
@@ -300,6 +427,81 @@ std::string deposit(const std::string &x, const std::vector<int> &pos) {
         r += "(((" + x + ") >> " + std::to_string(t) + ") & 1u) << " + std::to_string(pos[t]);
     }
     return "(" + r + ")";
+}
+
+// The outputs of a step as described at split_k_block.  Thread t of the
+// workgroup belongs to block t / thr and takes the terms k = t % thr, + thr, ..
+// (thr = threads per block, so the k range of every thread ends inside 2^nk);
+// the block's bits are the step's exclusive output bits first, so that an A
+// value serves all B values of its k and the other way round.
+void emit_outputs_split_k(std::ostringstream &o, const StepDesc &st, int threads, int rb) {
+    const OperandDesc &A = st.a, &B = st.b;
+    const uint32_t am = source_mask(A), bm = source_mask(B);
+    const int rc = st.rc, thr = threads >> (rc - rb), waves = std::max(1, thr / 64);
+    std::vector<int> aonly, bonly, other, S;
+    for (int b = 0; b < rc; ++b) {
+        const bool ia = (am >> b) & 1u, ib = (bm >> b) & 1u;
+        (ia && !ib ? aonly : ib && !ia ? bonly : other).push_back(b);
+    }
+    size_t ia = 0, ib = 0, io = 0;
+    while ((int)S.size() < rb) {
+        if (ia < aonly.size() && (ia <= ib || ib >= bonly.size())) S.push_back(aonly[ia++]);
+        else if (ib < bonly.size()) S.push_back(bonly[ib++]);
+        else S.push_back(other[io++]);
+    }
+    std::vector<int> R;
+    uint32_t sm = 0;
+    for (int b : S) sm |= 1u << b;
+    for (int b = 0; b < rc; ++b)
+        if (!((sm >> b) & 1u)) R.push_back(b);
+    auto combos = [&](uint32_t mask) {
+        std::vector<int> bits;
+        for (int b : S)
+            if ((mask >> b) & 1u) bits.push_back(b);
+        std::vector<uint32_t> v;
+        for (uint32_t t = 0; t < (1u << bits.size()); ++t) v.push_back(pdep(t, bits));
+        return v;
+    };
+    const std::vector<uint32_t> ca = combos(am), cb = combos(bm);
+    auto single = [](const OperandDesc &op) { return op.kind == kInter ? 1u << op.nsingle : 1u; };
+    const std::string ga = gather_expr(A), gb = gather_expr(B);
+    o << "    {\n      float *red = reinterpret_cast<float *>(smem + RED);\n";
+    o << "      const unsigned blk = (unsigned)tid / " << thr << "u, kl = (unsigned)tid % " << thr << "u;\n";
+    o << "      const unsigned rb = " << (R.empty() ? std::string("0u") : deposit("blk", R)) << ";\n";
+    for (size_t x = 0; x < ca.size(); ++x)
+        o << "      const unsigned ar" << x << " = " << subst_c(ga, "(rb | " + std::to_string(ca[x]) + "u)") << ";\n";
+    for (size_t y = 0; y < cb.size(); ++y)
+        o << "      const unsigned br" << y << " = " << subst_c(gb, "(rb | " + std::to_string(cb[y]) + "u)") << ";\n";
+    for (uint32_t t = 0; t < (1u << rb); ++t) o << "      float acc" << t << " = 0.f;\n";
+    // two terms per iteration in flight (each thread has at least eight)
+    o << "      #pragma unroll 2\n      for (unsigned k = kl; k < " << (1u << st.nk) << "u; k += " << thr << "u) {\n";
+    auto loads = [&](const OperandDesc &op, const char *base, const char *r, const char *v, size_t n) {
+        for (size_t x = 0; x < n; ++x) {
+            const std::string idx = std::string(r) + std::to_string(x) + " | (k << " + std::to_string(op.kshift) + ")";
+            o << "        float " << v << x << " = " << base << "[" << idx << "];\n";
+            for (uint32_t q = 1; q < single(op); ++q)
+                o << "        " << v << x << " += " << base << "[" << idx << " | " << (q << op.sshift) << "u];\n";
+        }
+    };
+    loads(A, "pa", "ar", "va", ca.size());
+    loads(B, "pb", "br", "vb", cb.size());
+    std::vector<uint32_t> outs;
+    for (uint32_t t = 0; t < (1u << rb); ++t) {
+        const uint32_t c = pdep(t, S);
+        outs.push_back(c);
+        const size_t x = std::find(ca.begin(), ca.end(), c & am) - ca.begin();
+        const size_t y = std::find(cb.begin(), cb.end(), c & bm) - cb.begin();
+        o << "        acc" << t << " = fmaf(va" << x << ", vb" << y << ", acc" << t << ");\n";
+    }
+    o << "      }\n";
+    for (uint32_t t = 0; t < (1u << rb); ++t) {
+        for (int w = 1; w < std::min(thr, 64); w <<= 1) o << "      acc" << t << " += __shfl_xor(acc" << t << ", " << w << ");\n";
+        o << "      if ((kl & 63u) == 0u) red[((kl >> 6) << " << rc << ") | rb | " << outs[t] << "u] = acc" << t << ";\n";
+    }
+    o << "      __syncthreads();\n";
+    o << "      if (tid < " << (1 << rc) << ") {\n        float x = red[tid];\n";
+    for (int w = 1; w < waves; ++w) o << "        x += red[" << (w << rc) << " + tid];\n";
+    o << "        x = ldexpf(x, shift);\n        lmax = x > lmax ? x : lmax;\n        pc[tid] = x;\n      }\n    }\n";
 }
 
 // GEMM-shaped step on BF16 MFMA: per syndrome, C[i, j] = sum_k A[i, k] B[k, j]
@@ -358,6 +560,15 @@ void emit_outputs_mfma(std::ostringstream &o, const StepDesc &st, int threads) {
     o << "        }\n      }\n    }\n";
 }
 
+// Operand bit that output bit u feeds, or -1.
+int seg_image(const OperandDesc &op, int u) {
+    for (int i = 0; i < op.nseg; ++i) {
+        const Seg &g = op.seg[i];
+        if (g.width > 0 && u >= g.src && u < g.src + g.width) return g.dst + (u - g.src);
+    }
+    return -1;
+}
+
 // Exclusive output bits of a step: those feeding only A and only B.
 void mfma_side_bits(const StepDesc &st, std::vector<int> &aon, std::vector<int> &bon) {
     const uint32_t am = source_mask(st.a), bm = source_mask(st.b);
@@ -374,8 +585,16 @@ void mfma_side_bits(const StepDesc &st, std::vector<int> &aon, std::vector<int> 
 // one more B-only bit: 4 x 2 tiles, the best of 2 x 2, 4 x 2 and 2 x 4 on
 // toric L=5; 4 x 4 spills), so every operand value a lane loads feeds rb (or
 // ra) MFMAs.  The k loop takes ku instructions' worth of contracted values
-// per iteration and loads the next iteration's operands before issuing its
-// own MFMAs (at one or two waves per SIMD few other waves hide the loads).
+// per iteration; a group's registers are loaded again for the next iteration as
+// soon as its MFMAs have been issued, and the last iteration of a block loads
+// the first values of the wave's next block, so that loads stay in flight
+// across the block's stores (at one or two waves per SIMD few other waves hide
+// them, and a wait for loads behind stores is a wait for the stores too).  The
+// wave's last block loads its own first values once more, unused.  Measured
+// against one wait per iteration for all of its loads: the circuit-level d=3,
+// 3-round plan 357 -> 330 us per 16,384, d=5 with 2 rounds 2.91 -> 2.80 ms per
+// 4,096, toric L=5 20.0 -> 19.7 ms per 512 (its widest step runs at 50 of 64
+// multiply-adds per cycle and workgroup, the FP32 MFMA rate).
 // Layouts (wave64), with T the tile edge (64 / T contracted values per
 // instruction):
 // lane l holds A[l % T][l / T] and B[l / T][l % T]; T = 32: D[v] =
@@ -393,7 +612,11 @@ void emit_outputs_mfma32(std::ostringstream &o, const StepDesc &st, int threads)
     const int tbits = big ? 5 : 4;                 // tile edge 2^tbits
     const unsigned tedge = 1u << tbits, kq = 64u / tedge;   // k values per instruction
     const std::vector<int> ai(aon.begin(), aon.begin() + tbits), bj(bon.begin(), bon.begin() + tbits);
-    const int xa = std::min<int>(2, (int)aon.size() - tbits), xb = std::min<int>(1, (int)bon.size() - tbits);
+    // a block shrinks while there are fewer blocks than waves: at 4 x 2 tiles a
+    // 128 x 64 step is one block, and three of four waves would idle
+    const int nwaves = threads / 64;
+    int xa = std::min<int>(2, (int)aon.size() - tbits), xb = std::min<int>(1, (int)bon.size() - tbits);
+    while (xa + xb > 0 && (1 << (st.rc - 2 * tbits - xa - xb)) < nwaves) (xa >= 2 * xb ? xa : xb) -= 1;
     const std::vector<int> a2(aon.begin() + tbits, aon.begin() + tbits + xa);
     const std::vector<int> b2(bon.begin() + tbits, bon.begin() + tbits + xb);
     std::vector<int> rest;
@@ -406,65 +629,75 @@ void emit_outputs_mfma32(std::ostringstream &o, const StepDesc &st, int threads)
     }
     const int ra = 1 << xa, rb = 1 << xb;
     const unsigned ntiles = 1u << rest.size();
-    const int nwaves = threads / 64;
     const unsigned nkk = 1u << st.nk;
     const unsigned ku = std::min(4u, nkk / kq);   // instructions' k groups per loop iteration
     const unsigned kstep = kq * ku;
     const std::string tm = std::to_string(tedge - 1) + "u", lsh = std::to_string(tbits);
     const char *acc_t = big ? "f32x16" : "f32x4";
     const char *mfma = big ? "__builtin_amdgcn_mfma_f32_32x32x2f32" : "__builtin_amdgcn_mfma_f32_16x16x4f32";
-    const std::string ga = gather_expr(A), gb = gather_expr(B);
-    auto ld = [&](const OperandDesc &op, const char *base, const std::string &idx, const std::string &k) {
-        const std::string e = idx + " | ((" + k + ") << " + std::to_string(op.kshift) + ")";
-        if (op.kind == kInter) return std::string(base) + "[(" + e + ") << GLOG]";
-        return std::string(base) + "[" + e + "]";
+    // Operand bits that output bits feed (those that feed the other side only
+    // drop out), and the operand index made from them.
+    auto image = [](const OperandDesc &op, const std::vector<int> &bits) {
+        std::vector<int> v;
+        for (int c : bits) v.push_back(seg_image(op, c));
+        return v;
+    };
+    auto spread = [](const std::string &x, const std::vector<int> &pos) {
+        std::string r;
+        for (size_t t = 0; t < pos.size(); ++t)
+            if (pos[t] >= 0)
+                r += std::string(r.empty() ? "" : " | ") + "(((" + x + ") >> " + std::to_string(t) + ") & 1u) << " +
+                     std::to_string(pos[t]);
+        return r.empty() ? std::string("0u") : "(" + r + ")";
+    };
+    // place of a block's first operand values (the lane's row or column and its
+    // contracted value within a group); the values of the block's other tiles
+    // and groups lie at constant distances
+    const std::string lane = "(unsigned)(l & " + tm + ")", kl = "((unsigned)(l >> " + lsh + ") << ";
+    auto offsets = [&](const std::string &t) {
+        return "          tb = " + deposit(t, rest) + ";\n          qa = pa + (" + spread(t, image(A, rest)) + " | " +
+               spread(lane, image(A, ai)) + " | " + kl + std::to_string(A.kshift) + "));\n          qb = pb + (" +
+               spread(t, image(B, rest)) + " | " + spread(lane, image(B, bj)) + " | " + kl + std::to_string(B.kshift) +
+               "));\n";
+    };
+    auto load = [&](unsigned u) {
+        for (int x = 0; x < ra; ++x)
+            o << "          a" << u << "_" << x << " = qa[" << (pdep(x, image(A, a2)) + ((kq * u) << A.kshift)) << "];\n";
+        for (int y = 0; y < rb; ++y)
+            o << "          b" << u << "_" << y << " = qb[" << (pdep(y, image(B, b2)) + ((kq * u) << B.kshift)) << "];\n";
+        // in this order, group by group: a wait for the oldest group is then not
+        // a wait for all
+        o << "          __builtin_amdgcn_sched_barrier(0);\n";
     };
     o << "    {\n";
     o << "      const int l = tid & 63, w = tid >> 6;\n";
+    o << "      if (w < " << ntiles << ") {\n";
+    o << "      unsigned tb;\n      const T *qa, *qb;\n      float a0_0";
+    for (unsigned u = 0; u < ku; ++u) {
+        for (int x = 0; x < ra; ++x)
+            if (u || x) o << ", a" << u << "_" << x;
+        for (int y = 0; y < rb; ++y) o << ", b" << u << "_" << y;
+    }
+    o << ";\n          " << offsets("(unsigned)w");
+    for (unsigned u = 0; u < ku; ++u) load(u);
     o << "      #pragma unroll 1\n";
     o << "      for (unsigned t = (unsigned)w; t < " << ntiles << "u; t += " << nwaves << "u) {\n";
-    o << "        const unsigned tb = " << deposit("t", rest) << ";\n";
-    for (int x = 0; x < ra; ++x)
-        o << "        const unsigned ar" << x << " = "
-          << subst_c(ga, "(tb | " + deposit("(unsigned)(l & " + tm + ")", ai) + " | " +
-                             deposit(std::to_string(x) + "u", a2) + ")")
-          << ";\n";
-    for (int y = 0; y < rb; ++y)
-        o << "        const unsigned br" << y << " = "
-          << subst_c(gb, "(tb | " + deposit("(unsigned)(l & " + tm + ")", bj) + " | " +
-                             deposit(std::to_string(y) + "u", b2) + ")")
-          << ";\n";
+    o << "        const unsigned tc = tb;\n";
     for (int x = 0; x < ra; ++x)
         for (int y = 0; y < rb; ++y) o << "        " << acc_t << " acc" << x << "_" << y << " = {};\n";
-    auto loads = [&](const std::string &kbase, const char *pre, bool decl) {
-        for (unsigned u = 0; u < ku; ++u) {
-            const std::string k = kbase + " + " + std::to_string(kq * u) + "u";
-            for (int x = 0; x < ra; ++x)
-                o << "          " << (decl ? "float " : "") << pre << "a" << u << "_" << x << " = "
-                  << ld(A, "pa", "ar" + std::to_string(x), k) << ";\n";
-            for (int y = 0; y < rb; ++y)
-                o << "          " << (decl ? "float " : "") << pre << "b" << u << "_" << y << " = "
-                  << ld(B, "pb", "br" + std::to_string(y), k) << ";\n";
-        }
-    };
-    o << "        {\n";
-    loads("(unsigned)(l >> " + lsh + ")", "n", true);
     o << "        #pragma unroll 1\n";
-    o << "        for (unsigned kb = (unsigned)(l >> " << lsh << "); kb < " << nkk << "u; kb += " << kstep << "u) {\n";
+    o << "        for (unsigned kb = " << kstep << "u; kb <= " << nkk << "u; kb += " << kstep << "u) {\n";
+    o << "          if (kb < " << nkk << "u) {\n";
+    o << "            qa += " << (kstep << A.kshift) << ";\n            qb += " << (kstep << B.kshift) << ";\n";
+    o << "          } else {\n          const unsigned tn = t + " << nwaves << "u < " << ntiles << "u ? t + " << nwaves
+      << "u : t;\n          " << offsets("tn") << "          }\n";
     for (unsigned u = 0; u < ku; ++u) {
-        for (int x = 0; x < ra; ++x) o << "          const float a" << u << "_" << x << " = na" << u << "_" << x << ";\n";
-        for (int y = 0; y < rb; ++y) o << "          const float b" << u << "_" << y << " = nb" << u << "_" << y << ";\n";
-    }
-    // the same for every lane (kb differs across the wave by l >> tbits < kq <= kstep): uniform
-    o << "          if (kb + " << kstep << "u < " << nkk << "u) {\n";
-    loads("kb + " + std::to_string(kstep) + "u", "n", false);
-    o << "          }\n";
-    for (unsigned u = 0; u < ku; ++u)
         for (int x = 0; x < ra; ++x)
             for (int y = 0; y < rb; ++y)
                 o << "          acc" << x << "_" << y << " = " << mfma << "(a" << u << "_" << x << ", b" << u << "_" << y
                   << ", acc" << x << "_" << y << ", 0, 0, 0);\n";
-    o << "        }\n";
+        load(u);
+    }
     o << "        }\n";
     for (int x = 0; x < ra; ++x)
         for (int y = 0; y < rb; ++y) {
@@ -474,7 +707,7 @@ void emit_outputs_mfma32(std::ostringstream &o, const StepDesc &st, int threads)
                 o << "          const unsigned i = 8u * (unsigned)(v >> 2) + 4u * (unsigned)(l >> 5) + (unsigned)(v & 3);\n";
             else
                 o << "          const unsigned i = 4u * (unsigned)(l >> 4) + (unsigned)v;\n";
-            o << "          const unsigned c = tb | " << deposit("i", ai) << " | " << deposit(std::to_string(x) + "u", a2)
+            o << "          const unsigned c = tc | " << deposit("i", ai) << " | " << deposit(std::to_string(x) + "u", a2)
               << " | " << deposit("(unsigned)(l & " + tm + ")", bj) << " | " << deposit(std::to_string(y) + "u", b2)
               << ";\n";
             o << "          const float x = ldexpf(acc" << x << "_" << y << "[v], shift);\n";
@@ -482,12 +715,18 @@ void emit_outputs_mfma32(std::ostringstream &o, const StepDesc &st, int threads)
             o << "          pc[c << GLOG] = x;\n";
             o << "        }\n";
         }
-    o << "      }\n    }\n";
+    o << "      }\n      }\n    }\n";
 }
 
 void emit_step(std::ostringstream &o, const StepDesc &st, int s, size_t const_n, int cstep, bool fp64, int unroll,
-               const SpecCfg *mfma_cfg, bool opaque_tid = false) {
+               const SpecCfg *mfma_cfg, const Places &places, bool opaque_tid = false) {
     const OperandDesc &A = st.a, &B = st.b;
+    int64_t lds[2] = {-1, -1};
+    for (int side = 0; side < 2; ++side)
+        if (places.prod[s][side] >= 0) lds[side] = places.lds[places.prod[s][side]];
+    const int64_t lc = places.lds[s];
+    const std::string pc = (lc >= 0 ? "lwork + " + std::to_string(lc) : "work + " + std::to_string((long long)st.c_off)) +
+                           " * G + g;\n";
     o << "  { // step " << s << ": rank " << st.rc << ", contracted " << st.nk << "\n";
     if (opaque_tid)
         // the step's own copy of the thread index, opaque to the optimiser:
@@ -499,9 +738,9 @@ void emit_step(std::ostringstream &o, const StepDesc &st, int s, size_t const_n,
              "    (void)g; (void)c0; (void)lane;\n";
     if (fp64) {
         // generic FP64 step: no scaling, the folded constant exponents restored per entry
-        emit_base(o, "pa", A, const_n);
-        emit_base(o, "pb", B, const_n);
-        o << "    T *pc = work + " << (long long)st.c_off << " * G + g;\n";
+        emit_base(o, "pa", A, const_n, lds[0]);
+        emit_base(o, "pb", B, const_n, lds[1]);
+        o << "    T *pc = " << pc;
         emit_outputs(o, st, cstep, unroll, true);
         o << "  }\n";
         o << "  __syncthreads();\n";
@@ -527,14 +766,20 @@ void emit_step(std::ostringstream &o, const StepDesc &st, int s, size_t const_n,
         if (B.kind == kInter) cond += std::string(cond.empty() ? "" : " || ") + "nb < -100";
         if (!cond.empty()) o << "    if (" << cond << ") lowf[g] = 1;\n";
     }
-    emit_base(o, "pa", A, const_n);
-    emit_base(o, "pb", B, const_n);
-    o << "    T *pc = work + " << (long long)st.c_off << " * G + g;\n";
+    emit_base(o, "pa", A, const_n, lds[0]);
+    emit_base(o, "pb", B, const_n, lds[1]);
+    o << "    T *pc = " << pc;
     o << "    T lmax = 0;\n";
+    // a slab's steps of one or two contracted labels wait on memory: more
+    // outputs per lane block put more loads in flight (circuit-level d=5, 2
+    // rounds 3.18 -> 2.91 ms per 4,096 against blocks of 4)
+    if (opaque_tid && st.nk <= 2) unroll = std::max(unroll, st.nk <= 1 ? 16 : 8);
     if (mfma_cfg && spec_step_uses_mfma(st, *mfma_cfg))
         emit_outputs_mfma(o, st, mfma_cfg->threads);
     else if (mfma_cfg && spec_step_uses_mfma32(st, *mfma_cfg))
         emit_outputs_mfma32(o, st, mfma_cfg->threads);
+    else if (mfma_cfg && split_k_block(st, *mfma_cfg) >= 0)
+        emit_outputs_split_k(o, st, mfma_cfg->threads, split_k_block(st, *mfma_cfg));
     else
         emit_outputs(o, st, cstep, unroll, false);
     o << "    for (int w = G; w < 64; w <<= 1) { const float other = __shfl_xor(lmax, w); lmax = other > lmax ? other : lmax; }\n";
@@ -560,14 +805,6 @@ struct RLay {
     int pos[2] = {-1, -1};   // tensor index bit held by lane bit t (-1: replicated along t)
 };
 
-int seg_image(const OperandDesc &op, int u) {
-    for (int i = 0; i < op.nseg; ++i) {
-        const Seg &g = op.seg[i];
-        if (g.width > 0 && u >= g.src && u < g.src + g.width) return g.dst + (u - g.src);
-    }
-    return -1;
-}
-
 uint32_t gather_host(uint32_t c, const OperandDesc &op) {
     uint32_t r = 0;
     for (int i = 0; i < op.nseg; ++i) {
@@ -591,12 +828,6 @@ std::vector<int> reg_bits(const RLay &l, int rank) {
 uint32_t pext(uint32_t x, const std::vector<int> &bits) {
     uint32_t r = 0;
     for (size_t j = 0; j < bits.size(); ++j) r |= ((x >> bits[j]) & 1u) << j;
-    return r;
-}
-
-uint32_t pdep(uint32_t x, const std::vector<int> &bits) {
-    uint32_t r = 0;
-    for (size_t j = 0; j < bits.size(); ++j) r |= ((x >> j) & 1u) << bits[j];
     return r;
 }
 
@@ -1436,9 +1667,10 @@ void emit_tile_fn(std::ostringstream &o, const CompiledPlan &cp, const SpecCfg &
     o << "  using T = " << tn << ";\n";
     o << "  constexpr int G = " << (1 << cfg.glog) << ", GLOG = " << cfg.glog << ", NT = " << cfg.threads
       << ", CSTEP = " << (cfg.threads >> cfg.glog) << ", NBITS = " << std::max(1, cp.n_syn) << ", NOUT = "
-      << (1 << cp.n_out) << ", NSLOTS = " << std::max(1, cp.n_slots) << ";\n";
+      << (1 << cp.n_out) << ", NSLOTS = " << std::max(1, cp.n_slots) << ", RED = " << L.red << ";\n  (void)RED;\n";
+    const Places places = slab_places(cp, cfg);
     if (cfg.slab)
-        o << "  T *work = slabw;\n";
+        o << "  T *work = slabw;\n  T *lwork = reinterpret_cast<T *>(smem + " << L.work << ");\n  (void)lwork;\n";
     else
         o << "  T *work = reinterpret_cast<T *>(smem + " << L.work << ");\n";
     if (!cfg.fp64) {
@@ -1470,7 +1702,7 @@ void emit_tile_fn(std::ostringstream &o, const CompiledPlan &cp, const SpecCfg &
     o << "  __syncthreads();\n";
     for (int s = 0; s < nsteps; ++s)
         emit_step(o, cp.steps[s], s, const_n, cfg.threads >> cfg.glog, cfg.fp64, std::max(1, cfg.unroll),
-                  ((cfg.mfma || cfg.mfma32) && !cfg.fp64) ? &cfg : nullptr, cfg.slab);
+                  ((cfg.mfma || cfg.mfma32) && !cfg.fp64) ? &cfg : nullptr, places, cfg.slab);
     o << "  if (tid < G) {\n"
          "    const long long q = b0 + tid;\n"
          "    if (q < count) {\n"
@@ -1482,7 +1714,11 @@ void emit_tile_fn(std::ostringstream &o, const CompiledPlan &cp, const SpecCfg &
     o << "      T best = 0, second = -1;\n"
          "      int bi = 0;\n"
          "      for (int j = 0; j < NOUT; ++j) {\n";
-    o << "        const T x = work[(" << (long long)cp.root_off << " + j) * G + g];\n";
+    int64_t root_lds = -1;
+    for (int s = 0; s < nsteps; ++s)
+        if (cp.steps[s].is_root) root_lds = places.lds[s];
+    o << "        const T x = " << (root_lds >= 0 ? "lwork" : "work") << "[("
+      << (long long)(root_lds >= 0 ? root_lds : cp.root_off) << " + j) * G + g];\n";
     o << "        if (mar) mar[b * NOUT + j] = ldexp((double)x, e);\n"
          "        if (j == 0 || x > best) {\n"
          "          if (j > 0) second = best;\n"

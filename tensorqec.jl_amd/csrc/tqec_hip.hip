@@ -1325,10 +1325,44 @@ bool spec_fits(const tqec_plan *p, const SpecCfg &c) {
 
 // Default before tuning: the register-resident FP32 kernel when the plan's
 // live tensors fit a quad's registers (256 threads, tables in global memory,
-// two waves per SIMD when the live set leaves room); else the largest tile whose LDS
+// two waves per SIMD when the live set leaves room); else, for FP32 plans with
+// GEMM-shaped steps, one syndrome per workgroup with those steps on FP32 MFMA,
+// in LDS or from a slab (choose_gemm); else the largest tile whose LDS
 // image (tables included when they fit) lets three workgroups share a CU
 // (else two, else one), 16 threads per syndrome within [64, 128], blocks of
 // 4 outputs per lane; else per-workgroup slabs, 256 threads, blocks of 4.
+//
+// One syndrome per workgroup is what MFMA steps need, and it beats larger
+// tiles on every plan with such steps that was measured: circuit-level d=3
+// with 3 rounds (24 KB of LDS) 330 us per 16,384 syndromes instead of 834 in
+// tiles of 2, d=9 (37 KB) 1.18 instead of 1.33 ms, toric L=3 (slab) 594 us per
+// 8,192 instead of 2,080 in tiles of 16, circuit-level d=5 with 2 rounds
+// (slab) 2.2 ms per 4,096 instead of 11.1 in tiles of 4.  Two waves per SIMD
+// (at most 256 registers) let one wave's MFMAs cover the other's loads; an LDS
+// plan takes as many threads as bring its workgroups per CU to four or more
+// waves (64 threads were faster than 128 or 256 at four and six workgroups).
+bool choose_gemm(const tqec_plan *p, SpecCfg &out) {
+    SpecCfg c;
+    c.glog = 0;
+    c.threads = 64;
+    c.tab_lds = false;
+    c.unroll = 4;
+    c.mfma32 = true;
+    c.waves = 2;
+    if (!spec_plan_uses_mfma32(p->cp, c)) return false;
+    const size_t lds = spec_lds_bytes(p->cp, c);
+    if (lds <= p->lds_limit) {
+        const size_t per_cu = p->lds_limit / std::max<size_t>(lds, 1);
+        c.threads = per_cu >= 4 ? 64 : per_cu >= 2 ? 128 : 256;
+    } else {
+        c.slab = true;
+        c.threads = 256;
+    }
+    if (!spec_fits(p, c)) return false;
+    out = c;
+    return true;
+}
+
 SpecCfg choose_spec(const tqec_plan *p, bool fp64 = false) {
     if (spec_reg_supported(p->cp)) {
         // every tensor of a syndrome fits a quad's registers: no LDS intermediates
@@ -1341,6 +1375,8 @@ SpecCfg choose_spec(const tqec_plan *p, bool fp64 = false) {
         c.waves = (!fp64 && spec_reg_peak(p->cp) <= 200) ? 2 : 0;
         if (spec_fits(p, c)) return c;
     }
+    SpecCfg gemm;
+    if (!fp64 && choose_gemm(p, gemm)) return gemm;
     for (int div : {3, 2, 1}) {
         for (int gl = 6; gl >= 0; --gl) {
             for (bool tab : {true, false}) {
@@ -1365,14 +1401,6 @@ SpecCfg choose_spec(const tqec_plan *p, bool fp64 = false) {
         c.fp64 = fp64;
         c.slab = true;
         c.unroll = 4;
-        // GEMM-shaped steps of one-syndrome FP32 slabs on FP32 MFMA (toric L=5:
-        // 2.2x; circuit-level d=5, 2 rounds: 1.08x after tuning)
-        SpecCfg m = c;
-        m.mfma32 = true;
-        c.mfma32 = spec_plan_uses_mfma32(p->cp, m);   // false for FP64 and for tiles of several syndromes
-        // two waves per SIMD (at most 256 registers) let one wave's MFMAs
-        // cover the other's operand loads: toric L=5 1.4x over one wave
-        if (c.mfma32) c.waves = 2;
         const size_t bytes = spec_slab_entries(p->cp, c) * (fp64 ? 8 : 4);
         if ((bytes <= (size_t(4) << 20) || gl == 0) && spec_lds_bytes(p->cp, c) <= p->lds_limit) return c;
     }
@@ -1424,19 +1452,19 @@ int spec_get(tqec_plan *p, int dev, const SpecCfg &cfg, SpecKernel **out) {
         return set_error(TQEC_EDEVICE, std::string("hipModuleGetFunction: ") + hipGetErrorString(e));
     }
     k.blocks = p->n_cu * resident_per_cu(k.lds, cfg.threads, p->lds_limit);
+    if (cfg.reg || cfg.slab) {
+        // register-bound: the runtime's occupancy of the compiled kernel
+        int per_cu = 0;
+        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k.fn, cfg.threads, 0) == hipSuccess &&
+            per_cu > 0)
+            k.blocks = p->n_cu * per_cu;
+    }
     if (cfg.slab) {
         // the kernel loops over tiles in as many workgroups as run: fewer of
         // them when their slabs would not fit the budget (plans of width 2^23:
         // 72 MB per workgroup)
         const size_t per = spec_slab_entries(p->cp, cfg) * (cfg.fp64 ? 8 : 4);
         if (per) k.blocks = (int)std::max<size_t>((size_t)p->n_cu, std::min<size_t>((size_t)k.blocks, kSpecSlabTotal / per));
-    }
-    if (cfg.reg) {
-        // register-bound: the runtime's occupancy of the compiled kernel
-        int per_cu = 0;
-        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k.fn, cfg.threads, 0) == hipSuccess &&
-            per_cu > 0)
-            k.blocks = p->n_cu * per_cu;
     }
     p->spec[key] = k;
     *out = &p->spec[key];
