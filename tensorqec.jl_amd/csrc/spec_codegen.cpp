@@ -1231,12 +1231,23 @@ bool reg_static_scales(const CompiledPlan &cp, const RegPlan &rp, RegScale &rs, 
     return true;
 }
 
+// The register-resident kernel is one straight line of code, cut into chunks:
+// the terms of one contracted value of one step.  A chunk's table values are
+// loaded several chunks before its multiply-adds (emit_reg_chunks).
+constexpr int kPrefetch32 = 24, kPrefetch64 = 8;   // table values in flight
+
+struct RegChunk {
+    std::string loads;   // the step's table addresses (first chunk) and this chunk's table values
+    int values = 0;      // table values loaded
+    std::string body;
+};
+
 // One step of the register-resident kernel.  FP32 with `rs`: the static
 // exponents and shifts of reg_static_scales; FP32 without: per-tensor
 // power-of-two scaling from each operand's maximum (the generic FP32
 // kernel's); FP64 (`fp64`): no scaling, the constant exponents folded out of
 // table data restored per entry (the generic FP64 kernel's).
-bool emit_reg_step(std::ostringstream &o, const CompiledPlan &cp, const RegPlan &rp, int s, size_t const_n,
+bool emit_reg_step(std::vector<RegChunk> &out, const CompiledPlan &cp, const RegPlan &rp, int s, size_t const_n,
                    bool fp64, const RegScale *rs, std::string &err) {
     const StepDesc &st = cp.steps[s];
     const RLay &LC = rp.lay[s];
@@ -1246,43 +1257,42 @@ bool emit_reg_step(std::ostringstream &o, const CompiledPlan &cp, const RegPlan 
     const char *T = fp64 ? "double" : "float";
     const char *zero = fp64 ? "0.0" : "0.f";
     const bool dyn = !fp64 && !rs;
-    if (dyn) o << "    float m" << s << ";\n    int e" << s << ";\n";
-    o << "    " << T;
-    for (uint32_t r = 0; r < nreg; ++r) o << (r ? ", " : " ") << "x" << s << "_" << r;
-    o << ";\n";
-    o << "    { // step " << s << ": rank " << st.rc << ", contracted " << st.nk << ", " << nreg
-      << " registers per lane";
-    if (rs) o << "; bound 2^" << (int)std::ceil(rs->pre[s]) << " before a shift of " << rs->shift[s] << ", exponent "
-              << rs->E[s];
-    o << "\n";
+    const std::string S = std::to_string(s);
     const char *ab[2] = {"a", "b"};
+    std::ostringstream first, addr;
+    first << "    // step " << s << ": rank " << st.rc << ", contracted " << st.nk << ", " << nreg << " registers per lane";
+    if (rs) first << "; bound 2^" << (int)std::ceil(rs->pre[s]) << " before a shift of " << rs->shift[s] << ", exponent "
+                  << rs->E[s];
+    first << "\n    " << T;
+    for (uint32_t r = 0; r < nreg; ++r) first << (r ? ", " : " ") << "x" << s << "_" << r << " = " << zero;
+    first << ";\n";
     for (int side = 0; side < 2 && dyn; ++side) {
         const OperandDesc &op = side ? st.b : st.a;
         const int p = rp.prod[side][s];
         if (op.kind == kInter)
-            o << "      const int n" << ab[side] << " = (m" << p << " > 0.f) ? ilogbf(m" << p << ") : 0, e" << ab[side]
-              << " = e" << p << " + n" << ab[side] << ";\n";
+            first << "    const int n" << ab[side] << S << " = (m" << p << " > 0.f) ? ilogbf(m" << p << ") : 0, e" << ab[side]
+                  << S << " = e" << p << " + n" << ab[side] << S << ";\n";
         else
-            o << "      const int n" << ab[side] << " = 0, e" << ab[side] << " = " << op.cexp << ";\n";
+            first << "    const int n" << ab[side] << S << " = 0, e" << ab[side] << S << " = " << op.cexp << ";\n";
     }
-    if (dyn) o << "      const int shift = -(na + nb);\n";
     if (dyn) {
+        first << "    const int shift" << S << " = -(na" << S << " + nb" << S << ");\n";
         std::string cond;
-        if (st.a.kind == kInter) cond += "na < -100";
-        if (st.b.kind == kInter) cond += std::string(cond.empty() ? "" : " || ") + "nb < -100";
-        if (!cond.empty()) o << "      if (" << cond << ") lowf = 1;\n";
+        if (st.a.kind == kInter) cond += "na" + S + " < -100";
+        if (st.b.kind == kInter) cond += std::string(cond.empty() ? "" : " || ") + "nb" + S + " < -100";
+        if (!cond.empty()) first << "    if (" << cond << ") lowf = 1;\n";
     }
     bool has_lane_off[2] = {false, false};
     for (int side = 0; side < 2; ++side) {
         const OperandDesc &op = side ? st.b : st.a;
         if (op.kind == kInter) continue;
         if (op.kind == kConst) {
-            o << "      const " << T << " *p" << ab[side] << " = tab + " << (long long)op.off << ";\n";
+            addr << "    const " << T << " *p" << ab[side] << S << " = tab + " << (long long)op.off << ";\n";
         } else {
-            o << "      const unsigned v" << ab[side] << " = 0u";
-            for (int j = 0; j < op.nev; ++j) o << " | (s" << op.ev_bit[j] << " << " << j << ")";
-            o << ";\n      const " << T << " *p" << ab[side] << " = tab + " << (long long)(const_n + (size_t)op.off) << " + (v"
-              << ab[side] << " << " << op.rank << ");\n";
+            addr << "    const unsigned v" << ab[side] << S << " = 0u";
+            for (int j = 0; j < op.nev; ++j) addr << " | (s" << op.ev_bit[j] << " << " << j << ")";
+            addr << ";\n    const " << T << " *p" << ab[side] << S << " = tab + " << (long long)(const_n + (size_t)op.off)
+                 << " + (v" << ab[side] << S << " << " << op.rank << ");\n";
         }
         std::string lo;
         for (int t = 0; t < 2; ++t) {
@@ -1295,30 +1305,33 @@ bool emit_reg_step(std::ostringstream &o, const CompiledPlan &cp, const RegPlan 
                   std::to_string(sh) + ")";
         }
         if (!lo.empty()) {
-            o << "      const unsigned l" << ab[side] << " = " << lo << ";\n";
+            addr << "    const unsigned l" << ab[side] << S << " = " << lo << ";\n";
             has_lane_off[side] = true;
         }
     }
-    o << "      " << T;
-    for (uint32_t r = 0; r < nreg; ++r) o << (r ? ", " : " ") << "acc" << r << " = " << zero;
-    o << ";\n";
     int ntmp = 0;
     for (uint32_t k = 0; k < nkk; ++k) {
-        o << "      {\n";
+        RegChunk chunk;
+        std::ostringstream o, ld;
+        if (k == 0) {
+            o << first.str();
+            ld << addr.str();
+        }
         std::vector<std::pair<std::string, std::string>> cache;   // expression -> temporary
-        auto value = [&](int side, uint32_t cst, std::string &out) -> bool {
+        auto temp = [&]() { return "f" + S + "_" + std::to_string(ntmp++); };
+        auto value = [&](int side, uint32_t cst, std::string &name) -> bool {
             const OperandDesc &op = side ? st.b : st.a;
             const uint32_t idx = gather_host(cst, op) | (k << op.kshift);
             std::string expr;
             if (op.kind != kInter) {
-                expr = std::string("p") + ab[side] + "[" + (has_lane_off[side] ? std::string("l") + ab[side] + " + " : "") +
-                       std::to_string(idx) + "u]";
+                expr = std::string("p") + ab[side] + S + "[" +
+                       (has_lane_off[side] ? std::string("l") + ab[side] + S + " + " : "") + std::to_string(idx) + "u]";
             } else {
                 const int p = rp.prod[side][s];
                 if (op.nsingle == 0) {
                     if (!reg_fetch(op, LC, rp.lay[p], p, idx, expr, err)) return false;
                     if (expr.compare(0, 3, "QP(") != 0) {
-                        out = expr;
+                        name = expr;
                         return true;
                     }
                 } else {
@@ -1333,58 +1346,47 @@ bool emit_reg_step(std::ostringstream &o, const CompiledPlan &cp, const RegPlan 
                     }
                     for (auto &c : cache)
                         if (c.first == expr) {
-                            out = c.second;
+                            name = c.second;
                             return true;
                         }
-                    const std::string nm = "f" + std::to_string(ntmp++);
-                    o << "        " << T << " " << nm << " = " << zero << ";\n";
-                    for (auto &t1 : terms) o << "        " << nm << " += " << t1 << ";\n";
+                    const std::string nm = temp();
+                    o << "    " << T << " " << nm << " = " << zero << ";\n";
+                    for (auto &t1 : terms) o << "    " << nm << " += " << t1 << ";\n";
                     cache.emplace_back(expr, nm);
-                    out = nm;
+                    name = nm;
                     return true;
                 }
             }
             for (auto &c : cache)
                 if (c.first == expr) {
-                    out = c.second;
+                    name = c.second;
                     return true;
                 }
-            const std::string nm = "f" + std::to_string(ntmp++);
-            o << "        const " << T << " " << nm << " = " << expr << ";\n";
+            const std::string nm = temp();
+            if (op.kind != kInter) ++chunk.values;
+            (op.kind != kInter ? ld : o) << "    const " << T << " " << nm << " = " << expr << ";\n";
             cache.emplace_back(expr, nm);
-            out = nm;
+            name = nm;
             return true;
         };
         for (uint32_t r = 0; r < nreg; ++r) {
             const uint32_t cst = pdep(r, RB);
             std::string va, vb;
             if (!value(0, cst, va) || !value(1, cst, vb)) return false;
-            o << "        acc" << r << " = " << (fp64 ? "fma(" : "fmaf(") << va << ", " << vb << ", acc" << r << ");\n";
+            o << "    x" << s << "_" << r << " = " << (fp64 ? "fma(" : "fmaf(") << va << ", " << vb << ", x" << s << "_" << r
+              << ");\n";
         }
-        o << "      }\n";
+        chunk.loads = ld.str();
+        chunk.body = o.str();
+        out.push_back(chunk);
     }
-    if (fp64) {
-        const int cexp = st.a.cexp + st.b.cexp;
-        for (uint32_t r = 0; r < nreg; ++r) {
-            o << "      x" << s << "_" << r << " = ";
-            if (cexp != 0)
-                o << "ldexp(acc" << r << ", " << cexp << ");\n";
-            else
-                o << "acc" << r << ";\n";
-        }
-        o << "    }\n";
-        return true;
-    }
-    if (rs) {
-        const int sh = rs->shift[s];
-        for (uint32_t r = 0; r < nreg; ++r) {
-            o << "      x" << s << "_" << r << " = ";
-            if (sh != 0)
-                o << "ldexpf(acc" << r << ", " << -sh << ");\n";
-            else
-                o << "acc" << r << ";\n";
-        }
-        o << "    }\n";
+    std::ostringstream o;
+    const int sh = fp64 ? st.a.cexp + st.b.cexp : rs ? -rs->shift[s] : 0;
+    if (!dyn) {
+        if (sh != 0)
+            for (uint32_t r = 0; r < nreg; ++r)
+                o << "    x" << s << "_" << r << " = " << (fp64 ? "ldexp(x" : "ldexpf(x") << s << "_" << r << ", " << sh << ");\n";
+        out.back().body += o.str();
         return true;
     }
     // Entries are >= 0 or NaN, and NaN-ignoring fmaxf over them equals the
@@ -1392,8 +1394,8 @@ bool emit_reg_step(std::ostringstream &o, const CompiledPlan &cp, const RegPlan 
     // free); a tree of three-input maxima halves the instructions.
     std::vector<std::string> mx;
     for (uint32_t r = 0; r < nreg; ++r) {
-        o << "      x" << s << "_" << r << " = ldexpf(acc" << r << ", shift);\n";
-        mx.push_back("x" + std::to_string(s) + "_" + std::to_string(r));
+        o << "    x" << s << "_" << r << " = ldexpf(x" << s << "_" << r << ", shift" << S << ");\n";
+        mx.push_back("x" + S + "_" + std::to_string(r));
     }
     mx.push_back("0.f");
     int nm = 0;
@@ -1404,8 +1406,8 @@ bool emit_reg_step(std::ostringstream &o, const CompiledPlan &cp, const RegPlan 
                 nx.push_back(mx[i]);
                 continue;
             }
-            const std::string t = "mx" + std::to_string(nm++);
-            o << "      const float " << t << " = ";
+            const std::string t = "mx" + S + "_" + std::to_string(nm++);
+            o << "    const float " << t << " = ";
             if (i + 2 < mx.size())
                 o << "fmaxf(fmaxf(" << mx[i] << ", " << mx[i + 1] << "), " << mx[i + 2] << ");\n";
             else
@@ -1414,29 +1416,196 @@ bool emit_reg_step(std::ostringstream &o, const CompiledPlan &cp, const RegPlan 
         }
         mx.swap(nx);
     }
-    o << "      float lmax = " << mx[0] << ";\n";
-    o << "      lmax = fmaxf(QP(lmax, 177), lmax);\n      lmax = fmaxf(QP(lmax, 78), lmax);\n";
-    o << "      m" << s << " = lmax;\n      e" << s << " = ea + eb;\n    }\n";
+    o << "    float m" << S << " = " << mx[0] << ";\n";
+    o << "    m" << S << " = fmaxf(QP(m" << S << ", 177), m" << S << ");\n    m" << S << " = fmaxf(QP(m" << S << ", 78), m" << S
+      << ");\n";
+    o << "    const int e" << S << " = ea" << S << " + eb" << S << ";\n";
+    out.back().body += o.str();
     return true;
 }
 
-void emit_tile_fn(std::ostringstream &o, const CompiledPlan &cp, const SpecCfg &cfg, const std::string &name,
-                  bool noinline = false);
-
-// FP64 configuration of the register-resident kernel's inline re-check: one
-// syndrome at a time over the whole workgroup, intermediates in LDS.
-SpecCfg inline_recheck_cfg(const SpecCfg &cfg) {
-    SpecCfg c;
-    c.glog = 0;
-    c.threads = cfg.threads;
-    c.tab_lds = false;
-    c.fp64 = true;
-    return c;
+// The chunks in order, each one's table values loaded as many chunks ahead as
+// keeps at most `budget` of them in flight: at two waves per SIMD nothing else
+// hides a load, and left to itself the compiler loads a chunk's values right
+// in front of it, one wait per 60 multiply-adds.  The scheduling barriers keep
+// the loads where they are put.  Measured with emit_reg_syndrome on the d=7
+// plan: FP32 64.2 -> 55.0 us per 65,536 rows and 20.9 -> 15.0 us for one tile
+// (budgets of 8 to 24 agree within 2%, 32 and more spill: 70 us), FP64 117 ->
+// 99 us.  Two waves per SIMD (223 registers) then wait 21% of their time and
+// issue a multiply-add every 3.9 cycles; the SIMD's own limit is 2.25.
+void emit_reg_chunks(std::ostringstream &o, const std::vector<RegChunk> &chunks, int budget) {
+    size_t next = 0;
+    int flight = 0;
+    for (size_t i = 0; i < chunks.size(); ++i) {
+        bool any = false;
+        while (next < chunks.size() && (next <= i || flight + chunks[next].values <= budget)) {
+            o << chunks[next].loads;
+            any = any || chunks[next].values > 0;
+            flight += chunks[next++].values;
+        }
+        if (any) o << "    __builtin_amdgcn_sched_barrier(0);\n";
+        o << chunks[i].body;
+        flight -= chunks[i].values;
+    }
 }
 
-// LDS a workgroup of the register-resident kernel may spend on its inline
-// FP64 re-check (beyond it, the separate re-check kernel runs instead).
+// Syndrome bits of row b as s0, s1, ..: words as wide as the rows' alignment
+// allows, all loads at once (a load of its own per bit under `valid ? :` cost a
+// branch and a wait each, 5 us of the d=7 kernel's 21 us for one tile).
+void emit_reg_syndrome(std::ostringstream &o, const CompiledPlan &cp, const std::vector<char> &used) {
+    const int nb = std::max(1, cp.n_syn);
+    const int w = nb % 16 == 0 ? 16 : nb % 8 == 0 ? 8 : nb % 4 == 0 ? 4 : 1;
+    const int words = (nb + 3) / 4;
+    o << "    unsigned sw[" << words << "];\n";
+    const char *bytes = "    {\n"
+                        "#pragma unroll\n"
+                        "      for (int i = 0; i < NBITS; ++i) sw[i >> 2] = (i & 3 ? sw[i >> 2] : 0u) | ((unsigned)row[i] << (8 * (i & 3)));\n"
+                        "    }\n";
+    if (w == 1) {
+        o << bytes;
+    } else {
+        const char *type = w == 16 ? "uint4" : w == 8 ? "uint2" : "unsigned";
+        o << "    if (((unsigned long long)syn & " << (w - 1) << "ull) == 0ull) {\n";
+        for (int i = 0; i < nb / w; ++i) {
+            o << "      const " << type << " w" << i << " = reinterpret_cast<const " << type << " *>(row)[" << i << "];\n";
+            const char *part[4] = {".x", ".y", ".z", ".w"};
+            for (int c = 0; c < w / 4; ++c) o << "      sw[" << i * (w / 4) + c << "] = w" << i << (w == 4 ? "" : part[c]) << ";\n";
+        }
+        o << "    } else\n" << bytes;
+    }
+    for (int j = 0; j < cp.n_syn; ++j)
+        if (used[j]) o << "    const unsigned s" << j << " = (sw[" << j / 4 << "] >> " << 8 * (j % 4) << ") & 1u;\n";
+}
+
+// ---- inline FP64 re-check of the register-resident FP32 kernel ------------
+//
+// The rows a tile flags are re-contracted by its waves, one row per wave: a
+// row's latency is what counts (a batch of more than a few hundred rows has
+// one in its last tiles nearly always), so its table slices are fetched to LDS
+// all at once and the steps need no workgroup barrier.  A workgroup of 256
+// threads that stepped through one row with a barrier and a table load from L2
+// per step took 8.5 us for a row of the d=7 code and 3.5 us at d=3; this takes
+// 7.3 and under 1 us, and several rows of a tile run side by side (65,536 rows
+// of d=3 with 1,002 of them re-checked: 13.6 -> 9.9 us).
+
+// LDS a workgroup may spend on it (beyond it, the separate kernel runs instead).
 constexpr size_t kInlineRecheckLds = 48 * 1024;
+
+struct Recheck {
+    bool tables = false;                  // table slices staged in LDS
+    std::vector<std::array<int, 2>> at;   // per step: LDS entry of its operands' slices, -1 for intermediates
+    int entries = 0;                      // doubles per row: intermediates, then slices
+    int rows = 0;                         // rows at a time (0: not inline)
+};
+
+Recheck recheck_plan(const CompiledPlan &cp, const SpecCfg &cfg) {
+    Recheck r;
+    if (!cfg.reg || cfg.fp64 || cp.ws_entries <= 0) return r;
+    int64_t top = cp.ws_entries;
+    for (const StepDesc &st : cp.steps) {
+        std::array<int, 2> at = {-1, -1};
+        for (int side = 0; side < 2; ++side) {
+            const OperandDesc &op = side ? st.b : st.a;
+            if (op.kind == kInter) continue;
+            at[side] = (int)top;
+            top += int64_t(1) << op.rank;
+        }
+        r.at.push_back(at);
+    }
+    r.tables = (size_t)top * 8 <= kInlineRecheckLds;
+    const int64_t e = r.tables ? top : cp.ws_entries;
+    if ((size_t)e * 8 > kInlineRecheckLds) return r;
+    r.entries = (int)e;
+    r.rows = (int)std::min<size_t>((size_t)cfg.threads / 64, kInlineRecheckLds / ((size_t)e * 8));
+    return r;
+}
+
+// recheck64: one row by one wave, the generic FP64 kernel's arithmetic.
+void emit_recheck_fn(std::ostringstream &o, const CompiledPlan &cp, const Recheck &r) {
+    const int nb = std::max(1, cp.n_syn);
+    const size_t const_n = cp.const_pool.size();
+    o << "__device__ __attribute__((noinline)) void recheck64(const unsigned char *__restrict__ row, long long b,\n"
+         "    const double *__restrict__ tab, double *__restrict__ mar, int *__restrict__ cls,\n"
+         "    unsigned char *__restrict__ ties, double tie_tol, double *work) {\n"
+         "  using T = double;\n  constexpr int GLOG = 0, NOUT = "
+      << (1 << cp.n_out) << ";\n  const int c0 = threadIdx.x & 63;\n";
+    // the row's bits, uniform over the wave
+    for (int w = 0; w * 64 < nb; ++w)
+        o << "  const unsigned long long m" << w << " = __ballot(c0 < " << std::min(64, nb - 64 * w) << " && (row[" << 64 * w
+          << " + min(c0, " << std::min(64, nb - 64 * w) - 1 << ")] & 1));\n";
+    auto base = [&](const OperandDesc &op) {
+        if (op.kind == kConst) return "tab + " + std::to_string((long long)op.off);
+        std::string v = "0u";
+        for (int j = 0; j < op.nev; ++j)
+            v += " | (((unsigned)(m" + std::to_string(op.ev_bit[j] / 64) + " >> " + std::to_string(op.ev_bit[j] % 64) + ") & 1u) << " +
+                 std::to_string(j) + ")";
+        return "tab + " + std::to_string((long long)(const_n + (size_t)op.off)) + " + ((" + v + ") << " +
+               std::to_string(op.rank) + ")";
+    };
+    if (r.tables) {
+        // slices in groups of loads small enough for registers
+        std::ostringstream ld, stg;
+        int n = 0;
+        auto flush = [&]() {
+            o << "  {\n" << ld.str() << stg.str() << "  }\n";
+            ld.str("");
+            stg.str("");
+            n = 0;
+        };
+        for (size_t s = 0; s < cp.steps.size(); ++s)
+            for (int side = 0; side < 2; ++side) {
+                const OperandDesc &op = side ? cp.steps[s].b : cp.steps[s].a;
+                if (r.at[s][side] < 0) continue;
+                const int size = 1 << op.rank;
+                ld << "    const double *t" << s << "_" << side << " = " << base(op) << ";\n";
+                for (int i = 0; i < size; i += 64) {
+                    const std::string nm = "d" + std::to_string(s) + "_" + std::to_string(side) + "_" + std::to_string(i);
+                    ld << "    const double " << nm << " = t" << s << "_" << side << "["
+                       << (size < 64 ? "min(c0, " + std::to_string(size - 1) + ")" : "c0 + " + std::to_string(i)) << "];\n";
+                    stg << "    " << (size < 64 ? "if (c0 < " + std::to_string(size) + ") " : "") << "work["
+                        << r.at[s][side] + i << " + c0] = " << nm << ";\n";
+                    ++n;
+                }
+                if (n >= 32) flush();
+            }
+        if (n) flush();
+    }
+    const char *sync = "  __threadfence_block();\n  __builtin_amdgcn_wave_barrier();\n";
+    o << sync;
+    for (size_t s = 0; s < cp.steps.size(); ++s) {
+        const StepDesc &st = cp.steps[s];
+        o << "  { // step " << s << "\n";
+        for (int side = 0; side < 2; ++side) {
+            const OperandDesc &op = side ? st.b : st.a;
+            o << "    const T *p" << (side ? "b" : "a") << " = ";
+            if (op.kind == kInter) o << "work + " << (long long)op.off << ";\n";
+            else if (r.tables) o << "work + " << r.at[s][side] << ";\n";
+            else o << base(op) << ";\n";
+        }
+        o << "    T *pc = work + " << (long long)st.c_off << ";\n";
+        emit_outputs(o, st, 64, 4, true);
+        o << "  }\n" << sync;
+    }
+    o << "  if (c0 == 0) {\n"
+         "    double best = 0, second = -1;\n"
+         "    int bi = 0;\n"
+         "    for (int j = 0; j < NOUT; ++j) {\n"
+         "      const double x = work["
+      << (long long)cp.root_off << " + j];\n"
+         "      if (mar) mar[b * NOUT + j] = x;\n"
+         "      if (j == 0 || x > best) {\n"
+         "        if (j > 0) second = best;\n"
+         "        best = x;\n"
+         "        bi = j;\n"
+         "      } else if (x > second) {\n"
+         "        second = x;\n"
+         "      }\n"
+         "    }\n"
+         "    if (cls) cls[b] = bi;\n"
+         "    const bool low = NOUT > 1 && second >= 0 && best - second <= tie_tol * best;\n"
+         "    if (ties) ties[b] = low ? 1 : 0;\n"
+         "  }\n" << sync << "}\n\n";
+}
 
 std::string reg_source(const CompiledPlan &cp, const SpecCfg &cfg, std::string &err) {
     RegPlan rp;
@@ -1470,10 +1639,10 @@ std::string reg_source(const CompiledPlan &cp, const SpecCfg &cfg, std::string &
              "__builtin_amdgcn_mov_dpp(__double2loint(x), (c), 0xf, 0xf, false))\n";
     else
         o << "#define QP(x, c) __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), (c), 0xf, 0xf, false))\n";
-    const bool inl = spec_reg_inline_recheck(cp, cfg);
-    const SpecCfg c64 = inline_recheck_cfg(cfg);
+    const Recheck rck = recheck_plan(cp, cfg);
+    const bool inl = rck.rows > 0;
     // a call of its own, so that its registers do not crowd the FP32 program's
-    if (inl) emit_tile_fn(o, cp, c64, "recheck64", true);
+    if (inl) emit_recheck_fn(o, cp, rck);
     o << "extern \"C\" __global__ void __launch_bounds__(" << cfg.threads;
     if (cfg.waves > 0) o << ", " << cfg.waves;
     o << ") " << spec_kernel_name(cfg) << "(\n"
@@ -1490,7 +1659,8 @@ std::string reg_source(const CompiledPlan &cp, const SpecCfg &cfg, std::string &
         // rows this tile flags for the FP64 re-check, done by the whole
         // workgroup at the end of the tile
         o << "  __shared__ int flagged[G];\n";
-        o << "  __shared__ __attribute__((aligned(16))) unsigned char smem64[" << layout(cp, c64).total << "];\n";
+        o << "  __shared__ double work64[" << rck.rows << "][" << rck.entries << "];\n"
+             "  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);\n";
     }
     if (cfg.tab_lds) {
         o << "  __shared__ " << T << " tab[" << std::max<size_t>(1, tab_n) << "];\n";
@@ -1513,18 +1683,21 @@ std::string reg_source(const CompiledPlan &cp, const SpecCfg &cfg, std::string &
          "   if (t < ntiles) {\n"
          "    const long long qi = t * G + (threadIdx.x >> 2);\n"
          "    const bool valid = qi < count;\n"
-         "    const long long b = valid ? (list ? (long long)list[qi] : qi) : 0ll;\n"
+         "    // lanes beyond the last row read it again and store nothing\n"
+         "    const long long qc = valid ? qi : count - 1;\n"
+         "    const long long b = list ? (long long)list[qc] : qc;\n"
          "    const unsigned char *row = syn + b * NBITS;\n";
     std::vector<char> used(std::max(1, cp.n_syn), 0);
     for (const StepDesc &st : cp.steps)
         for (const OperandDesc *op : {&st.a, &st.b})
             if (op->kind == kSliced)
                 for (int j = 0; j < op->nev; ++j) used[op->ev_bit[j]] = 1;
-    for (int j = 0; j < cp.n_syn; ++j)
-        if (used[j]) o << "    const unsigned s" << j << " = valid ? (unsigned)(row[" << j << "] & 1u) : 0u;\n";
+    emit_reg_syndrome(o, cp, used);
     if (dyn) o << "    int lowf = 0;\n";
+    std::vector<RegChunk> chunks;
     for (int s = 0; s < (int)cp.steps.size(); ++s)
-        if (!emit_reg_step(o, cp, rp, s, const_n, fp64, stat ? &rsc : nullptr, err)) return "";
+        if (!emit_reg_step(chunks, cp, rp, s, const_n, fp64, stat ? &rsc : nullptr, err)) return "";
+    emit_reg_chunks(o, chunks, fp64 ? kPrefetch64 : kPrefetch32);
     // every lane gathers the root's entries; the quad's lane 0 finishes the row
     const RLay &LR = rp.lay[rp.root];
     const std::vector<int> RR = reg_bits(LR, cp.steps[rp.root].rc);
@@ -1590,12 +1763,13 @@ std::string reg_source(const CompiledPlan &cp, const SpecCfg &cfg, std::string &
          "   }\n"
          "   __syncthreads();\n";
     if (inl)
-        // at most G flagged rows (one per valid row of the tile), re-contracted
-        // in FP64 one after the other by the whole workgroup
+        // at most G flagged rows (one per valid row of the tile)
         o << "   const int nf = seg_n;\n"
-             "   for (int i = 0; i < nf; ++i)\n"
-             "     recheck64(syn, nf, flagged, i, gtab64, mar, cls, ties, nullptr, nullptr, 0, tie_tol, recheck_tol, "
-             "smem64, nullptr, 0u);\n"
+             "   if (wave < "
+          << rck.rows << ")\n"
+             "     for (int i = wave; i < nf; i += "
+          << rck.rows << ")\n"
+             "       recheck64(syn + (long long)flagged[i] * NBITS, flagged[i], gtab64, mar, cls, ties, tie_tol, work64[wave]);\n"
              "   if (threadIdx.x == 0 && rcount) rcount[t] = nf;\n"
              "   __syncthreads();\n";
     else
@@ -1608,7 +1782,7 @@ std::string reg_source(const CompiledPlan &cp, const SpecCfg &cfg, std::string &
 }  // namespace
 
 bool spec_reg_inline_recheck(const CompiledPlan &cp, const SpecCfg &cfg) {
-    return cfg.reg && !cfg.fp64 && cp.ws_entries > 0 && layout(cp, inline_recheck_cfg(cfg)).total <= kInlineRecheckLds;
+    return recheck_plan(cp, cfg).rows > 0;
 }
 
 size_t spec_lds_bytes(const CompiledPlan &cp, const SpecCfg &cfg) {
@@ -1653,13 +1827,12 @@ namespace {
 // whole step program, as a device function: the body of the generic fused
 // kernel's tile with every descriptor value substituted.  Starts and ends
 // with a workgroup barrier.
-void emit_tile_fn(std::ostringstream &o, const CompiledPlan &cp, const SpecCfg &cfg, const std::string &name,
-                  bool noinline) {
+void emit_tile_fn(std::ostringstream &o, const CompiledPlan &cp, const SpecCfg &cfg, const std::string &name) {
     const Layout L = layout(cp, cfg);
     const size_t const_n = cp.const_pool.size();
     const int nsteps = (int)cp.steps.size();
     const char *tn = cfg.fp64 ? "double" : "float";
-    o << "__device__ " << (noinline ? "__attribute__((noinline))" : "__forceinline__") << " void " << name << "(\n"
+    o << "__device__ __forceinline__ void " << name << "(\n"
       << "    const unsigned char *__restrict__ syn, long long count, const int *__restrict__ list, long long b0,\n"
       << "    const " << tn << " *__restrict__ tab, double *__restrict__ mar, int *__restrict__ cls,\n"
       << "    unsigned char *__restrict__ ties, int *rl, int *rcount, long long rcap, double tie_tol,\n"
