@@ -54,8 +54,10 @@ extern "C" {
 /* Execution modes of tqec_decode_batch*. */
 #define TQEC_MODE_PLAIN_F64 0 /* one batched kernel per plan step, FP64,
                                  intermediates in HBM                     */
-#define TQEC_MODE_FUSED_F64 1 /* whole plan per workgroup tile, FP64,
-                                 intermediates in LDS                     */
+#define TQEC_MODE_FUSED_F64 1 /* whole plan per launch, FP64, intermediates
+                                 in LDS: a wave per one to eight syndromes
+                                 where eight waves share a CU's LDS, else
+                                 (or where pinned) workgroup tiles        */
 #define TQEC_MODE_WIDE_F32 3  /* plain layout (intermediates in HBM) in FP32
                                  with per-tensor power-of-two scaling;
                                  low-margin syndromes re-contracted by the
@@ -139,8 +141,8 @@ typedef struct tqec_stats {
     int64_t plain_ws_entries;  /* per-syndrome HBM workspace, in entries  */
     int64_t fused_lds_entries; /* per-syndrome LDS footprint, in entries  */
     int32_t n_out;          /* number of logical classes = 2^n_out        */
-    int32_t fused_tile_f64; /* syndromes per workgroup, FUSED_F64         */
-    int32_t fused_tile_f32; /* syndromes per workgroup, FUSED_F32         */
+    int32_t fused_tile_f64; /* syndromes per workgroup tile, FUSED_F64    */
+    int32_t fused_tile_f32; /* syndromes per workgroup tile, FUSED_F32    */
     int64_t const_entries;  /* folded syndrome-independent operand data    */
     int64_t table_entries;  /* tabulated operand data (all bit patterns)   */
     int32_t tabulate_bits;  /* subtrees on at most this many syndrome bits
@@ -405,7 +407,9 @@ int tqec_plan_autotune(tqec_plan *plan, int32_t mode, const uint8_t *d_syndromes
                        int32_t *tile, int32_t *threads);
 
 /* Pin the tile configuration of a fused mode (tile: syndromes per workgroup,
- * a power of two <= 64; threads: 64, 128 or 256). */
+ * a power of two <= 64; threads: 64, 128 or 256).  For FUSED_F64 and FUSED_F32
+ * a tile of one syndrome and one wave (1, 64) is the wave executor, where the
+ * plan suits it; the autotuner reports that choice in the same way. */
 int tqec_plan_set_tile(tqec_plan *plan, int32_t mode, int32_t tile, int32_t threads);
 
 /* Kernel timing with HIP events recorded on the call's stream (off by

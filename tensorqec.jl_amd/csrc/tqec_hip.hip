@@ -38,6 +38,7 @@
 #include "plan.hpp"
 #include "plan_compile.hpp"
 #include "spec_codegen.hpp"
+#include "wave_tile.hpp"
 #include "tqec_hip.h"
 
 using namespace tqec;
@@ -482,7 +483,8 @@ __device__ void fused_tile(const FusedArgs &args, int64_t b0, int64_t count, uin
     __syncthreads();
 }
 
-// Persistent single-plan kernel: workgroups stride over the tiles.
+// Persistent single-plan kernel: workgroups stride over the tiles.  Serves
+// plans too wide for the wave executor, and tiles pinned by the caller.
 template <typename T, bool SCALE>
 __global__ void __launch_bounds__(256) fused_kernel(FusedArgs args) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -797,6 +799,7 @@ struct DeviceData {
     StepDesc *steps = nullptr;
     double *cpool64 = nullptr, *spool64 = nullptr;
     float *cpool32 = nullptr, *spool32 = nullptr;
+    uint32_t *wdesc = nullptr, *went = nullptr;   // wave executor: WavePlan::desc, WavePlan::ent
 };
 
 struct Workspace {
@@ -859,6 +862,8 @@ struct tqec_plan {
     std::map<int, DeviceData> dev;
     std::map<std::pair<int, hipStream_t>, Workspace> ws;
     FusedCfg f64, f32;
+    bool tiled64 = false, tiled32 = false;   // a workgroup tile was chosen (autotune, set_tile) over the wave executor
+    WavePlan wave;
     bool cfg_done = false;
     bool timing = false;
     size_t lds_limit = 0;
@@ -905,6 +910,12 @@ int ensure_device(tqec_plan *p, int device, DeviceData **out) {
         both.insert(both.end(), cp.sliced_pool.begin(), cp.sliced_pool.end());
         if ((rc = upload<float>(both, &dd.tab32))) return rc;
         if ((rc = upload<double>(both, &dd.tab64))) return rc;
+    }
+    if (cp.semiring == TQEC_SEMIRING_SUM && p->wave.ok) {
+        TQ_HIP(hipMalloc((void **)&dd.wdesc, p->wave.desc.size() * sizeof(uint32_t)));
+        TQ_HIP(hipMemcpy(dd.wdesc, p->wave.desc.data(), p->wave.desc.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+        TQ_HIP(hipMalloc((void **)&dd.went, p->wave.ent.size() * sizeof(uint32_t)));
+        TQ_HIP(hipMemcpy(dd.went, p->wave.ent.data(), p->wave.ent.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     }
     if (cp.semiring == TQEC_SEMIRING_MAX) {
         TQ_HIP(hipMalloc((void **)&dd.msteps, std::max<size_t>(1, cp.map_steps.size()) * sizeof(MapStep)));
@@ -963,6 +974,59 @@ FusedCfg choose_fused(const CompiledPlan &cp, size_t elem, bool scale, size_t ld
     return FusedCfg();
 }
 
+// Launch shape of the wave executor for n syndromes.
+struct WaveCfg {
+    int glog = -1;      // -1: the plan keeps the workgroup tiles
+    int waves = 4;      // per workgroup
+    size_t lds = 0;
+    int blocks = 0;
+};
+
+WaveDims wave_dims(const tqec_plan *p, int glog) {
+    WaveDims d;
+    d.nsteps = p->wave.nsteps;
+    d.nops = p->wave.nops;
+    d.nent = p->wave.nops ? (int)p->wave.ent.size() : 0;
+    d.ws = (int)p->cp.ws_entries;
+    d.nslots = p->cp.n_slots;
+    d.nbits = p->cp.n_syn;
+    d.glog = glog;
+    return d;
+}
+
+// The wave executor serves every plan of which eight waves share a CU's LDS
+// (below that too few waves are in flight to hide its latencies).  A wave
+// takes one syndrome while that still leaves every CU at most 16 tiles, and
+// from there on twice as many as long as eight waves fit; steps whose outputs
+// fill less than half a wave's lanes are doubled up from 4 tiles per CU.
+// Measured (FP32 call with its FP64 re-check, us, workgroup tile -> G = 1 / 2
+// / 4 / 8): d=7, 1 row 648 -> 38 / 47 / 67 / -; 3,000 rows 670 -> 53 / 60 / 86
+// / -; 8,000 rows 677 -> 123 / 111 / 145 / -; 65,536 rows 5671 -> 960 / 863 /
+// 1115 / -.  d=5, 1 row 264 -> 19 / 19 / 21 / 27; 65,536 rows 707 -> 287 / 184
+// / 136 / 211.  d=3, 3,000 rows 135 -> 20 / 20 / 18 / 20; 65,536 rows 146 ->
+// 143 / 77 / 46 / 35.  Four waves per workgroup share the descriptors: one
+// wave per workgroup leaves room for fewer (d=7, 3,000 rows: 75 us).
+WaveCfg choose_wave(const tqec_plan *p, int elem, int64_t n) {
+    WaveCfg c;
+    if (!p->wave.ok) return c;
+    const auto lds4 = [&](int glog) {
+        const WaveDims d = wave_dims(p, glog);
+        return (size_t)d.desc_bytes() + 4 * (size_t)d.wave_bytes(elem);
+    };
+    if (lds4(0) > p->lds_limit / 2) return c;
+    const auto tiles = [&](int glog) { return (n + (1 << glog) - 1) >> glog; };
+    c.glog = 0;
+    while (c.glog < kWaveMaxGlog && lds4(c.glog + 1) <= p->lds_limit / 2 &&
+           (tiles(c.glog) > 16 * (int64_t)p->n_cu ||
+            (tiles(c.glog) > 4 * (int64_t)p->n_cu && (p->wave.mean_outputs << c.glog) <= 32)))
+        ++c.glog;
+    c.waves = (int)std::max<int64_t>(1, std::min<int64_t>(4, tiles(c.glog) / p->n_cu));
+    const WaveDims d = wave_dims(p, c.glog);
+    c.lds = (size_t)d.desc_bytes() + (size_t)c.waves * d.wave_bytes(elem);
+    c.blocks = p->n_cu * resident_per_cu(c.lds, c.waves * 64, p->lds_limit);
+    return c;
+}
+
 int configure(tqec_plan *p) {
     if (p->cfg_done) return TQEC_OK;
     int dev;
@@ -979,6 +1043,10 @@ int configure(tqec_plan *p) {
     TQ_HIP(hipFuncSetAttribute((const void *)fused_kernel<double, false>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     TQ_HIP(hipFuncSetAttribute((const void *)fused_kernel<float, true>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    TQ_HIP(hipFuncSetAttribute((const void *)wave_kernel<double, false>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    TQ_HIP(hipFuncSetAttribute((const void *)wave_kernel<float, true>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     p->cfg_done = true;
     return TQEC_OK;
@@ -1151,6 +1219,41 @@ FusedArgs base_args(tqec_plan *p, DeviceData *dd, const uint8_t *d_syn, int64_t 
     return a;
 }
 
+// Launch the wave executor over n syndromes, or those listed (at most n).
+int launch_wave(tqec_plan *p, DeviceData *dd, const WaveCfg &c, bool f32, const uint8_t *d_syn, int64_t n,
+                const int32_t *list, const int32_t *list_count, double *d_mar, int32_t *d_cls, uint8_t *d_tie,
+                int32_t *rl, int32_t *rcount, int64_t rcap, hipStream_t stream) {
+    const CompiledPlan &cp = p->cp;
+    WaveArgs a;
+    a.d = wave_dims(p, c.glog);
+    a.desc = dd->wdesc;
+    a.ent = dd->went;
+    a.tab = f32 ? (const void *)dd->tab32 : (const void *)dd->tab64;
+    a.syn = d_syn;
+    a.n = n;
+    a.nout = 1 << cp.n_out;
+    a.root_off = (int)cp.root_off;
+    a.root_slot = cp.root_slot;
+    a.list = list;
+    a.list_count = list_count;
+    a.marginals = d_mar;
+    a.classes = d_cls;
+    a.ties = d_tie;
+    a.tie_tol = p->tie_tol;
+    a.recheck_tol = p->recheck_tol;
+    a.recheck_list = rl;
+    a.recheck_count = rcount;
+    a.recheck_cap = rcap;
+    const int64_t tiles = (n + (1 << c.glog) - 1) >> c.glog;
+    const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>((tiles + c.waves - 1) / c.waves, c.blocks));
+    if (f32)
+        hipLaunchKernelGGL((wave_kernel<float, true>), dim3(grid), dim3(64 * c.waves), c.lds, stream, a);
+    else
+        hipLaunchKernelGGL((wave_kernel<double, false>), dim3(grid), dim3(64 * c.waves), c.lds, stream, a);
+    TQ_HIP(hipGetLastError());
+    return TQEC_OK;
+}
+
 int prepare_recheck(Workspace &w, int64_t n, hipStream_t stream);
 int enqueue_recheck(tqec_plan *p, DeviceData *dd, Workspace &w, const uint8_t *d_syn, int64_t n, double *d_mar,
                     int32_t *d_cls, uint8_t *d_tie, hipStream_t stream);
@@ -1174,7 +1277,14 @@ int run_fused(tqec_plan *p, DeviceData *dd, Workspace &w, const uint8_t *d_syn, 
         const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(ntiles, c64.blocks));
         int rc0;
         if ((rc0 = record(p, w, 0, stream))) return rc0;
-        hipLaunchKernelGGL((fused_kernel<double, false>), dim3(grid), dim3(c64.threads), c64.lds, stream, a);
+        const WaveCfg wc = p->tiled64 ? WaveCfg() : choose_wave(p, sizeof(double), n);
+        if (wc.glog >= 0) {
+            if ((rc0 = launch_wave(p, dd, wc, false, d_syn, n, in_list, in_count, d_mar, d_cls, d_tie, nullptr, nullptr,
+                                   0, stream)))
+                return rc0;
+        } else {
+            hipLaunchKernelGGL((fused_kernel<double, false>), dim3(grid), dim3(c64.threads), c64.lds, stream, a);
+        }
         if ((rc0 = record(p, w, 1, stream))) return rc0;
         TQ_HIP(hipGetLastError());
         return TQEC_OK;
@@ -1196,7 +1306,14 @@ int run_fused(tqec_plan *p, DeviceData *dd, Workspace &w, const uint8_t *d_syn, 
     const int64_t ntiles = (n + (1 << c32.glog) - 1) >> c32.glog;
     const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(ntiles, c32.blocks));
     if ((rc = record(p, w, 0, stream))) return rc;
-    hipLaunchKernelGGL((fused_kernel<float, true>), dim3(grid), dim3(c32.threads), c32.lds, stream, a);
+    const WaveCfg wc = p->tiled32 ? WaveCfg() : choose_wave(p, sizeof(float), n);
+    if (wc.glog >= 0) {
+        if ((rc = launch_wave(p, dd, wc, true, d_syn, n, in_list, in_count, d_mar, d_cls, d_tie, w.list, w.count,
+                              w.list_cap, stream)))
+            return rc;
+    } else {
+        hipLaunchKernelGGL((fused_kernel<float, true>), dim3(grid), dim3(c32.threads), c32.lds, stream, a);
+    }
     if ((rc = record(p, w, 1, stream))) return rc;
     return enqueue_recheck(p, dd, w, d_syn, n, d_mar, d_cls, d_tie, stream);
 }
@@ -1256,7 +1373,14 @@ int enqueue_recheck(tqec_plan *p, DeviceData *dd, Workspace &w, const uint8_t *d
     const unsigned rgrid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(
         (n + (1 << c64.glog) - 1) >> c64.glog, c64.blocks));
     if ((rc = record(p, w, 2, stream))) return rc;
-    hipLaunchKernelGGL((fused_kernel<double, false>), dim3(rgrid), dim3(c64.threads), c64.lds, stream, r);
+    const WaveCfg wc = p->tiled64 ? WaveCfg() : choose_wave(p, sizeof(double), n);
+    if (wc.glog >= 0) {
+        if ((rc = launch_wave(p, dd, wc, false, d_syn, n, w.list, w.count, d_mar, d_cls, d_tie, nullptr, nullptr, 0,
+                              stream)))
+            return rc;
+    } else {
+        hipLaunchKernelGGL((fused_kernel<double, false>), dim3(rgrid), dim3(c64.threads), c64.lds, stream, r);
+    }
     if ((rc = record(p, w, 3, stream))) return rc;
     w.count_on_device = true;   // read on demand by tqec_last_recheck_count
     TQ_HIP(hipGetLastError());
@@ -2109,6 +2233,7 @@ int tqec_plan_create(const tqec_plan_desc *desc, tqec_plan **out) {
     try {
         rc = compile_plan(desc, p->cp, err);
         if (rc == TQEC_OK && p->cp.semiring == TQEC_SEMIRING_SUM) spec_reg_prepare(p->cp);
+        if (rc == TQEC_OK && p->cp.semiring == TQEC_SEMIRING_SUM) p->wave = wave_plan(p->cp);
     } catch (const std::bad_alloc &) {
         return set_error(TQEC_ENOMEM, "out of host memory while compiling the plan");
     } catch (const std::exception &e) {
@@ -2150,6 +2275,8 @@ void tqec_plan_destroy(tqec_plan *p) {
         if (d.tab32) (void)hipFree(d.tab32);
         if (d.tab64) (void)hipFree(d.tab64);
         (void)hipFree(d.steps);
+        if (d.wdesc) (void)hipFree(d.wdesc);
+        if (d.went) (void)hipFree(d.went);
         if (d.msteps) (void)hipFree(d.msteps);
         if (d.mlabels) (void)hipFree(d.mlabels);
         (void)hipFree(d.cpool64);
@@ -2371,14 +2498,21 @@ int tqec_plan_autotune(tqec_plan *p, int32_t mode, const uint8_t *d_syn, int64_t
     TQ_HIP(hipEventCreate(&e1));
     const bool saved_timing = p->timing;
     p->timing = false;
+    const FusedCfg before = cfg;
     FusedCfg best = cfg;
     float best_ms = 1e30f;
     const size_t elem = f32 ? sizeof(float) : sizeof(double);
-    for (int gl = 0; gl <= 6; ++gl) {
-        if (fused_lds_bytes(p->cp, gl, elem, f32) > p->lds_limit) break;
+    // the wave executor first (tile -1), as what stays if no tile is faster
+    bool &tiled = f32 ? p->tiled32 : p->tiled64;
+    const bool tiled_before = tiled;
+    bool best_tiled = tiled;
+    for (int gl = choose_wave(p, (int)elem, n).glog >= 0 ? -1 : 0; gl <= 6; ++gl) {
+        if (gl >= 0 && fused_lds_bytes(p->cp, gl, elem, f32) > p->lds_limit) break;
         for (int thr : {64, 128, 256}) {
-            if (thr < (1 << gl)) continue;
-            cfg = make_cfg(p->cp, gl, thr, elem, f32, p->lds_limit, p->n_cu);
+            if (gl < 0 && thr > 64) continue;
+            if (thr < (1 << std::max(gl, 0))) continue;
+            tiled = gl >= 0;
+            cfg = gl < 0 ? before : make_cfg(p->cp, gl, thr, elem, f32, p->lds_limit, p->n_cu);
             float ms = 0;
             for (int rep = 0; rep < 2 && rc == TQEC_OK; ++rep) {
                 if ((rc = record_or(hipEventRecord(e0, st)))) break;
@@ -2392,17 +2526,21 @@ int tqec_plan_autotune(tqec_plan *p, int32_t mode, const uint8_t *d_syn, int64_t
             if (ms < best_ms) {
                 best_ms = ms;
                 best = cfg;
+                best_tiled = tiled;
             }
         }
         if (rc) break;
     }
     cfg = best;
+    tiled = rc ? tiled_before : best_tiled;
     p->timing = saved_timing;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc;
-    if (tile) *tile = 1 << best.glog;
-    if (threads) *threads = best.threads;
+    // one syndrome and one wave stands for the wave executor, also for
+    // tqec_plan_set_tile
+    if (tile) *tile = best_tiled ? 1 << best.glog : 1;
+    if (threads) *threads = best_tiled ? best.threads : 64;
     return TQEC_OK;
 }
 
@@ -2602,6 +2740,8 @@ int tqec_plan_set_tile(tqec_plan *p, int32_t mode, int32_t tile, int32_t threads
     if (fused_lds_bytes(p->cp, gl, elem, f32) > p->lds_limit)
         return set_error(TQEC_EUNSUPPORTED, "tile does not fit in LDS");
     (f32 ? p->f32 : p->f64) = make_cfg(p->cp, gl, threads, elem, f32, p->lds_limit, p->n_cu);
+    // one syndrome and one wave: the wave executor where the plan suits it
+    (f32 ? p->tiled32 : p->tiled64) = !(gl == 0 && threads == 64);
     return TQEC_OK;
 }
 
