@@ -168,6 +168,14 @@ int tqec_plan_stats(const tqec_plan *plan, tqec_stats *out);
  */
 int tqec_decode_batch(tqec_plan *plan, const uint8_t *syndromes, int64_t n, int32_t mode,
                       double *marginals, int32_t *classes, uint8_t *tie_flags, void *stream);
+/* As tqec_decode_batch, with the error patterns of a CSS code (host buffers
+ * of n x nq bytes) recovered on the device in the same call; the matrices are
+ * those of tqec_recovery_create_css, a byte per entry, logicals 0/1, at most
+ * 2,048 qubits and 15 logical pairs (else TQEC_EUNSUPPORTED, nothing done). */
+int tqec_decode_css_batch(tqec_plan *plan, const uint8_t *syndromes, int64_t n, int32_t mode, double *marginals,
+                          int32_t *classes, uint8_t *ties, int32_t nq, int32_t nsx, int32_t nsz, const uint8_t *Rx,
+                          const uint8_t *Rz, int32_t k, const uint8_t *lx, const uint8_t *lz, uint8_t *err_x,
+                          uint8_t *err_z, void *stream);
 
 /* Same with device pointers; enqueues on `stream` and returns. */
 int tqec_decode_batch_device(tqec_plan *plan, const uint8_t *d_syndromes, int64_t n, int32_t mode,

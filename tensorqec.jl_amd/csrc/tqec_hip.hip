@@ -39,6 +39,7 @@
 #include "plan_compile.hpp"
 #include "spec_codegen.hpp"
 #include "wave_tile.hpp"
+#include "recover_rows.hpp"
 #include "tqec_hip.h"
 
 using namespace tqec;
@@ -815,7 +816,9 @@ struct Workspace {
     int32_t *segc = nullptr;        // register-resident kernel: re-check rows per tile segment
     int64_t segc_cap = 0;
     int64_t count_nseg = 0;         // > 0: the last call's re-check count is the sum of segc[0 .. count_nseg)
-    uint8_t *d_syn = nullptr; size_t d_syn_bytes = 0;   // staging for the host API
+    void *h_stage = nullptr; size_t h_stage_bytes = 0;  // host API: pinned inputs and outputs of one call
+    void *d_stage = nullptr; size_t d_stage_bytes = 0;  // their device copies
+    uint8_t *d_syn = nullptr; size_t d_syn_bytes = 0;   // host API calls beyond kStageBytes
     double *d_mar = nullptr; size_t d_mar_bytes = 0;
     int32_t *d_cls = nullptr; size_t d_cls_bytes = 0;
     uint8_t *d_tie = nullptr; size_t d_tie_bytes = 0;
@@ -1969,6 +1972,104 @@ int decode_device(tqec_plan *p, const uint8_t *d_syn, int64_t n, int mode, doubl
     return set_error(TQEC_EINVAL, "unknown mode " + std::to_string(mode));
 }
 
+// Error-pattern recovery asked for with a host batch (tqec_decode_css_batch).
+struct HostRecovery {
+    RowsDims d;
+    const uint8_t *Rx, *Rz, *lx, *lz;
+    uint8_t *ex, *ez;
+};
+
+// Host calls up to this size go through pinned staging: one copy each way
+// instead of one per array out of pageable memory, and no copy of the
+// re-check count (read when asked for).  With the patterns recovered in the
+// same call, d=7 from Python: 3,000 rows 3103 -> 120 us (numpy's products
+// 2.5 ms of it); one d=5 row 119 -> 53 us.  Kernels that read and write the
+// pinned memory itself are no faster for a few rows (54 us).
+constexpr size_t kStageBytes = size_t(8) << 20;
+
+int grow_pinned(void **ptr, size_t *cap, size_t need) {
+    if (*cap >= need) return TQEC_OK;
+    if (*ptr) TQ_HIP(hipHostFree(*ptr));
+    *ptr = nullptr;
+    *cap = 0;
+    need = (need + 65535) & ~size_t(65535);
+    TQ_HIP(hipHostMalloc(ptr, need));
+    *cap = need;
+    return TQEC_OK;
+}
+
+// Decode a host batch and, when asked, recover its error patterns.
+int decode_host(tqec_plan *p, const uint8_t *syn, int64_t n, int32_t mode, double *mar, int32_t *cls, uint8_t *tie,
+                const HostRecovery *rec, void *stream) {
+    if (!p) return set_error(TQEC_ENULL, "null plan");
+    if (n < 0) return set_error(TQEC_EINVAL, "negative batch size");
+    if (n > 0 && !syn) return set_error(TQEC_ENULL, "null syndrome pointer");
+    if (n > (int64_t(1) << 31) - 1) return set_error(TQEC_EINVAL, "batch too large (max 2^31-1)");
+    if (mode < 0 || mode > TQEC_MODE_SPEC_BF16) return set_error(TQEC_EINVAL, "unknown mode " + std::to_string(mode));
+    if (p->cp.semiring != TQEC_SEMIRING_SUM)
+        return set_error(TQEC_EINVAL, "a max-product plan is decoded by tqec_map_decode_batch");
+    std::lock_guard<std::mutex> lk(p->mu);
+    hipStream_t st = (hipStream_t)stream;
+    int dev;
+    TQ_HIP(hipGetDevice(&dev));
+    Workspace &w = p->ws[std::make_pair(dev, st)];
+    w.device = dev;
+    if (n == 0) return TQEC_OK;
+    const int nout = 1 << p->cp.n_out;
+    int rc;
+    const auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+    // [matrices | syndromes | marginals | classes | ex | ez | ties], inputs first
+    const size_t mat_b = rec ? up((size_t)rec->d.bytes()) : 0, syn_b = (size_t)n * p->cp.n_syn;
+    const size_t mar_b = mar ? (size_t)n * nout * sizeof(double) : 0, cls_b = cls ? (size_t)n * sizeof(int32_t) : 0;
+    const size_t err_b = rec ? (size_t)n * rec->d.nq : 0, tie_b = tie ? (size_t)n : 0;
+    const size_t o_syn = mat_b, o_mar = up(o_syn + syn_b), o_cls = o_mar + up(mar_b), o_ex = o_cls + up(cls_b);
+    const size_t o_ez = o_ex + up(err_b), o_tie = o_ez + up(err_b), total = o_tie + up(tie_b);
+    const bool staged = total <= kStageBytes;
+    char *h = nullptr, *d;
+    if (staged || rec) {
+        if ((rc = grow_pinned(&w.h_stage, &w.h_stage_bytes, staged ? total : mat_b))) return rc;
+        h = (char *)w.h_stage;
+    }
+    if (rec && !rows_pack(rec->d, rec->Rx, rec->Rz, rec->lx, rec->lz, h))
+        return set_error(TQEC_EUNSUPPORTED, "logical operators must be 0/1");
+    if (staged) {
+        if ((rc = grow((char **)&w.d_stage, &w.d_stage_bytes, total))) return rc;
+        d = (char *)w.d_stage;
+    } else {
+        if ((rc = grow((char **)&w.d_syn, &w.d_syn_bytes, total))) return rc;
+        d = (char *)w.d_syn;
+    }
+    if (staged) {
+        std::memcpy(h + o_syn, syn, syn_b);
+        TQ_HIP(hipMemcpyAsync(d, h, o_syn + syn_b, hipMemcpyHostToDevice, st));
+    } else {
+        if (rec) TQ_HIP(hipMemcpyAsync(d, h, mat_b, hipMemcpyHostToDevice, st));
+        TQ_HIP(hipMemcpyAsync(d + o_syn, syn, syn_b, hipMemcpyHostToDevice, st));
+    }
+    const uint8_t *d_syn = (const uint8_t *)(d + o_syn);
+    int32_t *d_cls = cls ? (int32_t *)(d + o_cls) : nullptr;
+    if ((rc = decode_device(p, d_syn, n, mode, mar ? (double *)(d + o_mar) : nullptr, d_cls,
+                            tie ? (uint8_t *)(d + o_tie) : nullptr, st, nullptr)))
+        return rc;
+    if (rec) {
+        const unsigned grid = (unsigned)std::min<int64_t>((n + 3) / 4, (int64_t)p->n_cu * 8);
+        hipLaunchKernelGGL(recover_rows_kernel, dim3(grid), dim3(256), 0, st, rec->d, (const uint64_t *)d, d_syn,
+                           (const int32_t *)d_cls, n, (uint8_t *)(d + o_ex), (uint8_t *)(d + o_ez));
+        TQ_HIP(hipGetLastError());
+    }
+    if (staged) TQ_HIP(hipMemcpyAsync(h + o_mar, d + o_mar, total - o_mar, hipMemcpyDeviceToHost, st));
+    const struct { void *to; size_t off, bytes; } outs[] = {{mar, o_mar, mar_b}, {cls, o_cls, cls_b}, {tie, o_tie, tie_b},
+        {rec ? rec->ex : nullptr, o_ex, err_b}, {rec ? rec->ez : nullptr, o_ez, err_b}};
+    if (!staged)
+        for (const auto &o : outs)
+            if (o.bytes) TQ_HIP(hipMemcpyAsync(o.to, d + o.off, o.bytes, hipMemcpyDeviceToHost, st));
+    TQ_HIP(hipStreamSynchronize(st));
+    if (staged)
+        for (const auto &o : outs)
+            if (o.bytes) std::memcpy(o.to, h + o.off, o.bytes);
+    return TQEC_OK;
+}
+
 // Mixed-code executor state.  Each of two call slots owns the per-call
 // tables (header, batch table, counters, batch clocks) and a pinned host
 // staging copy of header + batch table, so a call can be staged while the
@@ -2256,6 +2357,8 @@ void tqec_plan_destroy(tqec_plan *p) {
         if (w.count) (void)hipFree(w.count);
         if (w.segc) (void)hipFree(w.segc);
         if (w.host_count) (void)hipHostFree(w.host_count);
+        if (w.h_stage) (void)hipHostFree(w.h_stage);
+        if (w.d_stage) (void)hipFree(w.d_stage);
         if (w.d_syn) (void)hipFree(w.d_syn);
         if (w.d_mar) (void)hipFree(w.d_mar);
         if (w.d_cls) (void)hipFree(w.d_cls);
@@ -2407,42 +2510,20 @@ int tqec_decode_batch_device_noalloc(tqec_plan *p, const uint8_t *d_syn, int64_t
 
 int tqec_decode_batch(tqec_plan *p, const uint8_t *syn, int64_t n, int32_t mode, double *mar, int32_t *cls,
                       uint8_t *tie, void *stream) {
-    if (!p) return set_error(TQEC_ENULL, "null plan");
-    if (n < 0) return set_error(TQEC_EINVAL, "negative batch size");
-    if (n > 0 && !syn) return set_error(TQEC_ENULL, "null syndrome pointer");
-    if (n > (int64_t(1) << 31) - 1) return set_error(TQEC_EINVAL, "batch too large (max 2^31-1)");
-    if (mode < 0 || mode > TQEC_MODE_SPEC_BF16) return set_error(TQEC_EINVAL, "unknown mode " + std::to_string(mode));
-    if (p->cp.semiring != TQEC_SEMIRING_SUM)
-        return set_error(TQEC_EINVAL, "a max-product plan is decoded by tqec_map_decode_batch");
-    std::lock_guard<std::mutex> lk(p->mu);
-    hipStream_t st = (hipStream_t)stream;
-    int dev;
-    TQ_HIP(hipGetDevice(&dev));
-    Workspace &w = p->ws[std::make_pair(dev, st)];
-    w.device = dev;
-    if (n == 0) return TQEC_OK;
-    const int nout = 1 << p->cp.n_out;
-    int rc;
-    if ((rc = grow(&w.d_syn, &w.d_syn_bytes, (size_t)n * std::max(1, p->cp.n_syn)))) return rc;
-    if (mar && (rc = grow(&w.d_mar, &w.d_mar_bytes, (size_t)n * nout * sizeof(double)))) return rc;
-    if (cls && (rc = grow(&w.d_cls, &w.d_cls_bytes, (size_t)n * sizeof(int32_t)))) return rc;
-    if (tie && (rc = grow(&w.d_tie, &w.d_tie_bytes, (size_t)n))) return rc;
-    TQ_HIP(hipMemcpyAsync(w.d_syn, syn, (size_t)n * p->cp.n_syn, hipMemcpyHostToDevice, st));
-    Workspace *wp = nullptr;
-    if ((rc = decode_device(p, w.d_syn, n, mode, mar ? w.d_mar : nullptr, cls ? w.d_cls : nullptr,
-                            tie ? w.d_tie : nullptr, st, &wp)))
-        return rc;
-    if (mar) TQ_HIP(hipMemcpyAsync(mar, w.d_mar, (size_t)n * nout * sizeof(double), hipMemcpyDeviceToHost, st));
-    if (cls) TQ_HIP(hipMemcpyAsync(cls, w.d_cls, (size_t)n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    if (tie) TQ_HIP(hipMemcpyAsync(tie, w.d_tie, (size_t)n, hipMemcpyDeviceToHost, st));
-    TQ_HIP(hipStreamSynchronize(st));
-    if (wp && wp->count_on_device && wp->host_count) {
-        int64_t m;
-        if ((rc = read_recheck_count(*wp, &m))) return rc;
-        wp->last_recheck = m;
-        wp->count_on_device = false;
-    }
-    return TQEC_OK;
+    return decode_host(p, syn, n, mode, mar, cls, tie, nullptr, stream);
+}
+
+int tqec_decode_css_batch(tqec_plan *p, const uint8_t *syn, int64_t n, int32_t mode, double *mar, int32_t *cls,
+                          uint8_t *tie, int32_t nq, int32_t nsx, int32_t nsz, const uint8_t *Rx, const uint8_t *Rz,
+                          int32_t k, const uint8_t *lx, const uint8_t *lz, uint8_t *err_x, uint8_t *err_z,
+                          void *stream) {
+    if (!p || !cls || !err_x || !err_z || (nsz > 0 && !Rx) || (nsx > 0 && !Rz) || (k > 0 && (!lx || !lz)))
+        return set_error(TQEC_ENULL, "null argument");
+    if (nq <= 0 || nsx < 0 || nsz < 0 || k < 0) return set_error(TQEC_EINVAL, "negative or empty sizes");
+    if (nsx + nsz != p->cp.n_syn) return set_error(TQEC_EINVAL, "check counts differ from the plan's syndrome bits");
+    if ((nq + 63) / 64 > kRowsMaxChunks || k > 15) return set_error(TQEC_EUNSUPPORTED, "recovery sizes out of range");
+    HostRecovery r{RowsDims{nq, nsx, nsz, k}, Rx, Rz, lx, lz, err_x, err_z};
+    return decode_host(p, syn, n, mode, mar, cls, tie, &r, stream);
 }
 
 int tqec_last_recheck_count(tqec_plan *p, void *stream, int64_t *count) {

@@ -295,8 +295,10 @@ def decode_batch(ct, syndromes, mode: Optional[str] = None, want_marginals: bool
             return decode_batch_dem(ct, syndromes, mode, want_marginals, error_patterns)
         raise TypeError(f"unsupported compiled decoder {type(ct)}")
     rows = _syndrome_rows(ct, syndromes)
-    mar, cls, tie = ct.hip.decode(rows, mode or ct.mode, want_marginals)
-    ep = css_error_patterns(ct, rows, cls) if error_patterns else None
+    if not error_patterns:
+        return BatchResult(*ct.hip.decode(rows, mode or ct.mode, want_marginals), None)
+    mar, cls, tie, ex, ez = ct.hip.decode(rows, mode or ct.mode, want_marginals, (ct.pure_x, ct.pure_z, ct.lx, ct.lz))
+    ep = css_error_patterns(ct, rows, cls) if ex is None else CSSErrorPattern(ex, ez)
     return BatchResult(mar, cls, tie, ep)
 
 

@@ -111,6 +111,10 @@ EXPORTS = [
     ("tqec_plan_stats", ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(Stats)]),
     ("tqec_decode_batch", ctypes.c_int,
      [ctypes.c_void_p, _u8p, ctypes.c_int64, ctypes.c_int32, _f64p, _i32p, _u8p, ctypes.c_void_p]),
+    ("tqec_decode_css_batch", ctypes.c_int,
+     [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p,
+      ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p,
+      ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]),
     ("tqec_decode_batch_device", ctypes.c_int,
      [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p,
       ctypes.c_void_p, ctypes.c_void_p]),
@@ -308,8 +312,13 @@ class HipPlan:
     def set_tolerances(self, tie_tol: float, recheck_tol: float) -> None:
         check(load().tqec_plan_set_tolerances(self._h, float(tie_tol), float(recheck_tol)))
 
-    def decode(self, syndromes: np.ndarray, mode="fused_f32", want_marginals=True) -> Tuple:
-        """Host-buffer batch decode: returns (marginals or None, classes, ties)."""
+    def decode(self, syndromes: np.ndarray, mode="fused_f32", want_marginals=True, recovery=None) -> Tuple:
+        """Host-buffer batch decode: returns (marginals or None, classes, ties).
+
+        With ``recovery=(pure_x, pure_z, lx, lz)`` (uint8 matrices as of
+        ``css_error_patterns``) the X and Z error patterns follow, recovered
+        on the device in the same call; both None when that call does not
+        serve these matrices."""
         m = MODES[mode] if isinstance(mode, str) else int(mode)
         s = np.ascontiguousarray(np.asarray(syndromes, dtype=np.uint8))
         if s.ndim == 1:
@@ -321,10 +330,24 @@ class HipPlan:
         mar = np.empty((B, nout), dtype=np.float64) if want_marginals else None
         cls = np.empty(B, dtype=np.int32)
         tie = np.empty(B, dtype=np.uint8)
-        check(load().tqec_decode_batch(self._h, _ptr(s, _u8p), B, m,
-                                       _ptr(mar, _f64p) if mar is not None else None,
-                                       _ptr(cls, _i32p), _ptr(tie, _u8p), None))
-        return mar, cls, tie
+        if recovery is not None:
+            rx, rz, lx, lz = recovery
+            nq, k = rx.shape[0], lx.shape[0]
+            if (rx.dtype == rz.dtype == lx.dtype == lz.dtype == np.uint8 and rx.ndim == rz.ndim == 2
+                    and lx.shape == lz.shape == (k, nq) and rz.shape[0] == nq
+                    and rx.shape[1] + rz.shape[1] == self.n_syn and B and nq):
+                rx, rz, lx, lz = (np.ascontiguousarray(x) for x in recovery)
+                ex, ez = np.empty((B, nq), dtype=np.uint8), np.empty((B, nq), dtype=np.uint8)
+                rc = load().tqec_decode_css_batch(
+                    self._h, s.ctypes.data, B, m, mar.ctypes.data if mar is not None else None, cls.ctypes.data,
+                    tie.ctypes.data, nq, rz.shape[1], rx.shape[1], rx.ctypes.data, rz.ctypes.data, k, lx.ctypes.data,
+                    lz.ctypes.data, ex.ctypes.data, ez.ctypes.data, None)
+                if rc != TQEC_EUNSUPPORTED:
+                    check(rc)
+                    return mar, cls, tie, ex, ez
+        pm = _ptr(mar, _f64p) if mar is not None else None
+        check(load().tqec_decode_batch(self._h, _ptr(s, _u8p), B, m, pm, _ptr(cls, _i32p), _ptr(tie, _u8p), None))
+        return (mar, cls, tie) if recovery is None else (mar, cls, tie, None, None)
 
     def decode_device(self, d_syn: int, n: int, mode, d_mar: int, d_cls: int, d_tie: int, stream: int = 0) -> None:
         """Device-pointer decode (integers are device addresses); enqueues only."""
