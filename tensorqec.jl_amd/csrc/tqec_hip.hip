@@ -852,6 +852,7 @@ struct SpecKernel {
     SpecCfg cfg;
     size_t lds = 0;
     int blocks = 0;
+    bool inline_recheck = false;   // spec_reg_inline_recheck of cfg
 };
 
 }  // namespace
@@ -1572,6 +1573,7 @@ int spec_get(tqec_plan *p, int dev, const SpecCfg &cfg, SpecKernel **out) {
     SpecKernel k;
     k.cfg = cfg;
     k.lds = spec_lds_bytes(p->cp, cfg);
+    k.inline_recheck = spec_reg_inline_recheck(p->cp, cfg);
     TQ_HIP(hipModuleLoadData(&k.mod, code.data()));
     const hipError_t e = hipModuleGetFunction(&k.fn, k.mod, spec_kernel_name(cfg));
     if (e != hipSuccess) {
@@ -1730,7 +1732,7 @@ int run_spec(tqec_plan *p, DeviceData *dd, Workspace &w, const uint8_t *d_syn, i
     int rc;
     if ((rc = spec_get(p, w.device, cfg, &k))) return rc;
     // the register-resident kernel may re-check its flagged rows itself
-    const bool inline_rc = spec_reg_inline_recheck(p->cp, cfg);
+    const bool inline_rc = k->inline_recheck;
     if (!inline_rc && (rc = spec_recheck_kernel(p, w.device, &k64))) return rc;
     if ((rc = grow((char **)&w.spec_slab, &w.spec_slab_bytes,
                    std::max(spec_slab_need(p, k, n), k64 ? spec_slab_need(p, k64, n) : size_t(0)))))
@@ -2473,7 +2475,7 @@ int tqec_decode_batch_device_noalloc(tqec_plan *p, const uint8_t *d_syn, int64_t
         return spec_launch(p, nullptr, 0, k, dd, d_syn, n, nullptr, nullptr, d_mar, d_cls, d_tie, nullptr, nullptr, 0,
                            p->tie_tol, p->recheck_tol, st);
     int32_t *list = scr, *counts = scr + kNoAllocRows;
-    if (cfg.reg && spec_reg_inline_recheck(p->cp, cfg)) {
+    if (cfg.reg && k->inline_recheck) {
         // flagged rows are re-contracted in FP64 inside the kernel; only the
         // per-tile counts go to the scratch
         const int32_t G = 1 << cfg.glog;
