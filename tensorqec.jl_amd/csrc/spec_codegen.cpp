@@ -2124,6 +2124,248 @@ std::string spec_map_source(const CompiledPlan &cp, int glog, int threads) {
     return o.str();
 }
 
+namespace {
+
+// Largest table set that a workgroup of the wave max-product kernel copies to LDS.
+constexpr size_t kMapTabLds = 16 * 1024;
+
+// Records of a wave at most (64 bits each, two vector registers for 64 of
+// them), and blocks of outputs of one step among which the backtrace selects.
+constexpr int kMapMaxRecords = 512, kMapMaxBlocks = 8;
+
+// Records of a step: bits eliminated times 64-entry blocks of (output, syndrome).
+int map_blocks(const StepDesc &st, int glog) { return std::max(1, (1 << st.rc) >> (6 - glog)); }
+
+struct MapWaveLayout {
+    size_t tab = 0;                      // bytes at the start of the workgroup's LDS
+    size_t syn = 0, total = 0;           // per wave
+    std::vector<int> rec_at;             // first 64-bit record of each step
+    int nrec = 0, max_blocks = 1;
+};
+
+MapWaveLayout map_wave_layout(const CompiledPlan &cp, int glog) {
+    MapWaveLayout L;
+    const size_t tab = (cp.const_pool.size() + cp.sliced_pool.size()) * 8;
+    if (tab <= kMapTabLds) L.tab = round_up(tab, 16);
+    for (const StepDesc &st : cp.steps) {
+        L.rec_at.push_back(L.nrec);
+        L.nrec += map_blocks(st, glog) * (st.nk + st.a.nsingle + st.b.nsingle);
+        L.max_blocks = std::max(L.max_blocks, map_blocks(st, glog));
+    }
+    const size_t words = (size_t)(cp.n_vars + 31) / 32;
+    L.syn = round_up(((size_t)std::max<int64_t>(1, cp.ws_entries) * 8) << glog, 16);
+    // the syndrome's bytes, later the configuration's words
+    L.total = round_up(L.syn + (std::max((size_t)std::max(1, cp.n_syn), words * 4) << glog), 16);
+    return L;
+}
+
+}  // namespace
+
+// A d=5 plan has 75 steps of 9 outputs on average: a workgroup tile spends its
+// time on 75 barriers, a table load from global memory before each, and a
+// backtrace by 16 of 256 threads.  A wave takes as many syndromes as leave its
+// lanes an output each on average; fewer where eight waves would not share the
+// LDS.  us, workgroup tile -> G = 2 / 4 / 8 per wave: 16,384 rows 47 -> 52 / 29
+// / 23, 65,536 rows 162 -> 170 / 108 / 82 (d=3, 65,536 rows, G = 4 / 8 / 16: 23
+// / 14 / 11).  Two waves per SIMD: with one (all the registers the compiler
+// wants) 31 us instead of 23.
+bool spec_map_wave_cfg(const CompiledPlan &cp, size_t lds_limit, int &glog, int &waves) {
+    if (cp.steps.empty()) return false;
+    int64_t outputs = 0;
+    for (const StepDesc &st : cp.steps) {
+        outputs += int64_t(1) << st.rc;
+        if (st.nk + st.a.nsingle + st.b.nsingle > 16 || st.rc > 16) return false;
+    }
+    const int64_t mean = outputs / (int64_t)cp.steps.size();
+    for (glog = 4; glog > 0 && (mean << glog) > 80; --glog) {}
+    for (;; --glog) {
+        if (glog < 0) return false;
+        const MapWaveLayout L = map_wave_layout(cp, glog);
+        if (L.nrec > kMapMaxRecords || L.max_blocks > kMapMaxBlocks) continue;
+        for (waves = 4; waves >= 1; waves >>= 1)
+            if (8 / waves * (L.tab + (size_t)waves * L.total) <= lds_limit) return true;
+    }
+}
+
+std::string spec_map_wave_source(const CompiledPlan &cp, int glog, int waves) {
+    const int G = 1 << glog, lanes = 64 >> glog, cl = 6 - glog, nt = waves * 64;
+    const int ns = (int)cp.steps.size();
+    const int words = (cp.n_vars + 31) / 32;
+    const size_t const_n = cp.const_pool.size(), tab_n = const_n + cp.sliced_pool.size();
+    const MapWaveLayout W = map_wave_layout(cp, glog);
+    std::ostringstream o;
+    o << "// plan-specialised max-product (TNMAP) kernel, a wave per " << G << " syndromes (generated)\n";
+    // the LDS holds two waves per SIMD at least: registers for as many
+    o << "extern \"C\" __global__ void __launch_bounds__(" << nt << ", 2) tqec_map_spec(\n"
+         "    const unsigned char *__restrict__ syn, long long n, const double *__restrict__ cpool,\n"
+         "    const double *__restrict__ spool, unsigned char *__restrict__ config, int n_config,\n"
+         "    double *__restrict__ logp) {\n";
+    o << "  constexpr int G = " << G << ", GLOG = " << glog << ", LANES = " << lanes << ", NBITS = " << cp.n_syn
+      << ";\n";
+    o << "  __shared__ __attribute__((aligned(16))) unsigned char smem[" << W.tab + (size_t)waves * W.total << "];\n";
+    o << "  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);\n"
+         "  const int g = lane & (G - 1), c0 = lane >> GLOG;\n";
+    o << "  unsigned char *mine = smem + " << W.tab << " + wave * " << W.total << ";\n"
+         "  double *work = reinterpret_cast<double *>(mine) + g;\n"
+         "  unsigned char *synl = mine + " << W.syn << ";\n"
+         "  unsigned *cfgw = reinterpret_cast<unsigned *>(synl);\n";
+    if (W.tab) {
+        o << "  double *tab = reinterpret_cast<double *>(smem);\n"
+             "  for (int i = threadIdx.x; i < " << const_n << "; i += " << nt << ") tab[i] = cpool[i];\n"
+             "  for (int i = threadIdx.x; i < " << tab_n - const_n << "; i += " << nt << ") tab[" << const_n
+          << " + i] = spool[i];\n"
+             "  const double *tc = tab, *ts = tab + " << const_n << ";\n"
+             "  __syncthreads();\n";
+    } else {
+        o << "  const double *tc = cpool, *ts = spool;\n";
+    }
+    const char *fence = "__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, \"wavefront\"); __builtin_amdgcn_wave_barrier();\n";
+    o << "  const long long ntiles = (n + G - 1) >> GLOG;\n"
+         "  for (long long t = (long long)blockIdx.x * " << waves << " + wave; t < ntiles; t += (long long)gridDim.x * "
+      << waves << ") {\n"
+         "    const long long q = (t << GLOG) + g;\n"
+         "    const bool valid = q < n;\n"
+         "    // lanes beyond the last row read it again and store nothing\n"
+         "    const long long b = valid ? q : n - 1;\n"
+         "    for (int i = c0; i < NBITS; i += LANES) synl[(i << GLOG) + g] = syn[b * NBITS + i] & 1u;\n    " << fence;
+    // arg-max records: uniform 64-bit words, a bit per (output, syndrome); the
+    // compiler keeps those beyond the scalar registers in vector lanes
+    for (int r = 0; r < W.nrec; ++r) o << "    unsigned long long r" << r << ";\n";
+    for (int s = 0; s < ns; ++s) {
+        const StepDesc &st = cp.steps[s];
+        const int nb = st.nk + st.a.nsingle + st.b.nsingle;
+        o << "    { // step " << s << ": rank " << st.rc << ", eliminated " << nb << "\n";
+        for (int side = 0; side < 2; ++side) {
+            const OperandDesc &op = side ? st.b : st.a;
+            const char *nm = side ? "pb" : "pa";
+            if (op.kind == kInter) {
+                o << "      const double *" << nm << " = work + " << ((long long)op.off << glog) << ";\n";
+            } else if (op.kind == kConst) {
+                o << "      const double *" << nm << " = tc + " << (long long)op.off << ";\n";
+            } else {
+                o << "      unsigned v" << nm << " = 0u;\n";
+                for (int j = 0; j < op.nev; ++j)
+                    o << "      v" << nm << " |= (unsigned)synl[(" << op.ev_bit[j] << " << GLOG) + g] << " << j << ";\n";
+                o << "      const double *" << nm << " = ts + " << (long long)op.off << " + (v" << nm << " << " << op.rank
+                  << ");\n";
+            }
+        }
+        // every output keeps the first maximum over (k, sa, sb), as the generic kernel
+        const int nk = 1 << st.nk, na = 1 << st.a.nsingle, nbn = 1 << st.b.nsingle;
+        const int terms = nk * (na + nbn), blocks = map_blocks(st, glog);
+        const int cexp = st.a.cexp + st.b.cexp;
+        const std::string ga = gather_expr(st.a), gb = gather_expr(st.b);
+        const unsigned cmask = (1u << st.rc) - 1u;
+        // outputs of a chunk: loads first, then comparisons, then stores
+        const int chunk = std::max(1, std::min(blocks, 32 / std::max(1, terms)));
+        const bool flat = terms <= 64;
+        for (int x0 = 0; x0 < blocks; x0 += chunk) {
+            const int x1 = std::min(blocks, x0 + chunk);
+            o << "      {\n";
+            for (int x = x0; x < x1; ++x) {
+                const std::string X = std::to_string(x);
+                o << "      const unsigned oc" << X << " = ((unsigned)c0 | " << ((unsigned)x << cl) << "u) & " << cmask
+                  << "u;\n";
+                o << "      const double *a" << X << " = pa + ((" << subst_c(ga, "oc" + X) << ")"
+                  << (st.a.kind == kInter ? " << GLOG" : "") << ");\n";
+                o << "      const double *b" << X << " = pb + ((" << subst_c(gb, "oc" + X) << ")"
+                  << (st.b.kind == kInter ? " << GLOG" : "") << ");\n";
+                o << "      double best" << X << " = -1.0;\n      unsigned bi" << X << " = 0u;\n";
+                if (!flat) continue;
+                for (int k = 0; k < nk; ++k) {
+                    for (int qa = 0; qa < na; ++qa)
+                        o << "      const double u" << X << "_" << k << "_" << qa << " = a" << X << "["
+                          << ((((unsigned)qa << st.a.sshift) | ((unsigned)k << st.a.kshift))
+                              << (st.a.kind == kInter ? glog : 0))
+                          << "];\n";
+                    for (int qb = 0; qb < nbn; ++qb)
+                        o << "      const double w" << X << "_" << k << "_" << qb << " = b" << X << "["
+                          << ((((unsigned)qb << st.b.sshift) | ((unsigned)k << st.b.kshift))
+                              << (st.b.kind == kInter ? glog : 0))
+                          << "];\n";
+                }
+            }
+            for (int x = x0; x < x1; ++x) {
+                const std::string X = std::to_string(x);
+                if (flat) {
+                    for (int k = 0; k < nk; ++k)
+                        for (int qa = 0; qa < na; ++qa)
+                            for (int qb = 0; qb < nbn; ++qb)
+                                o << "      { const double v = u" << X << "_" << k << "_" << qa << " * w" << X << "_" << k
+                                  << "_" << qb << "; if (v > best" << X << ") { best" << X << " = v; bi" << X << " = "
+                                  << (unsigned)(k | (qa << st.nk) | (qb << (st.nk + st.a.nsingle))) << "u; } }\n";
+                } else {
+                    const auto idx = [&](const char *qn, const OperandDesc &op) {
+                        return std::string("(((unsigned)") + qn + " << " + std::to_string(op.sshift) + ") | ((unsigned)k << " +
+                               std::to_string(op.kshift) + "))" + (op.kind == kInter ? " << GLOG" : "");
+                    };
+                    o << "      for (int k = 0; k < " << nk << "; ++k)\n        for (int qa = 0; qa < " << na
+                      << "; ++qa) {\n          const double va = a" << X << "[" << idx("qa", st.a) << "];\n"
+                      << "          for (int qb = 0; qb < " << nbn << "; ++qb) {\n            const double v = va * b" << X
+                      << "[" << idx("qb", st.b) << "];\n            if (v > best" << X << ") { best" << X << " = v; bi" << X
+                      << " = (unsigned)k | ((unsigned)qa << " << st.nk << ") | ((unsigned)qb << " << st.nk + st.a.nsingle
+                      << "); }\n          }\n        }\n";
+                }
+                if (cexp != 0) o << "      best" << X << " = ldexp(best" << X << ", " << cexp << ");\n";
+            }
+            for (int x = x0; x < x1; ++x) {
+                const std::string X = std::to_string(x);
+                o << "      work[(" << (long long)st.c_off << " + oc" << X << ") << GLOG] = best" << X << ";\n";
+                for (int j = 0; j < nb; ++j)
+                    o << "      r" << W.rec_at[s] + x * nb + j << " = __ballot((bi" << X << " >> " << j << ") & 1u);\n";
+            }
+            o << "      }\n";
+        }
+        o << "    }\n    " << fence;
+    }
+    // backtrace: every lane of a syndrome follows it, from the root down, with
+    // a register per label; a step's record is bit (output, syndrome) of its block
+    std::vector<char> known(std::max(1, cp.n_vars), 0);
+    for (int s = ns - 1; s >= 0; --s) {
+        const StepDesc &st = cp.steps[s];
+        const MapStep &ms = cp.map_steps[s];
+        const int32_t *lab = cp.map_labels.data() + ms.off;
+        const int nb = st.nk + st.a.nsingle + st.b.nsingle, blocks = map_blocks(st, glog);
+        if (!nb) continue;
+        for (int j = 0; j < nb; ++j)
+            if (!known[lab[ms.nc + j]]) {
+                known[lab[ms.nc + j]] = 1;
+                o << "    unsigned L" << lab[ms.nc + j] << " = 0u;\n";
+            }
+        o << "    {\n      unsigned c = 0u;\n";
+        for (int j = 0; j < ms.nc; ++j)
+            if (known[lab[j]]) o << "      c |= L" << lab[j] << " << " << j << ";\n";
+        o << "      const unsigned at = ((c & " << lanes - 1 << "u) << GLOG) | (unsigned)g;\n";
+        // 32-bit halves: no variable 64-bit shifts (a kernel made of those gave
+        // wrong bits now and then)
+        const bool low = (int64_t(1) << (st.rc + glog)) <= 32;
+        for (int j = 0; j < nb; ++j)
+            for (int x = 0; x < blocks; ++x) {
+                const std::string r = "r" + std::to_string(W.rec_at[s] + x * nb + j);
+                o << "      ";
+                if (blocks > 1) o << "if ((c >> " << cl << ") == " << x << "u) ";
+                o << "L" << lab[ms.nc + j] << " |= __builtin_amdgcn_ubfe(";
+                if (low) o << "(unsigned)" << r;
+                else o << "at < 32u ? (unsigned)" << r << " : (unsigned)(" << r << " >> 32)";
+                o << ", at" << (low ? "" : " & 31u") << ", 1u);\n";
+            }
+        o << "    }\n";
+    }
+    for (int w = 0; w < words; ++w) {
+        o << "    cfgw[" << (w << glog) << " + g] = 0u";
+        for (int v = 32 * w; v < std::min(cp.n_vars, 32 * w + 32); ++v)
+            if (known[v]) o << " | (L" << v << " << " << (v & 31) << ")";
+        o << ";\n";
+    }
+    o << "    " << fence;
+    o << "    if (valid)\n"
+         "      for (int v = c0; v < n_config; v += LANES)\n"
+         "        config[b * n_config + v] = (unsigned char)((cfgw[((v >> 5) << GLOG) + g] >> (v & 31)) & 1u);\n"
+         "    if (valid && c0 == 0 && logp) logp[b] = log(work[" << ((long long)cp.root_off << glog) << "]);\n    "
+      << fence << "  }\n}\n";
+    return o.str();
+}
+
 size_t spec_mixed_lds_bytes(const std::vector<MixedSpecPlan> &plans) {
     size_t m = 16;
     for (const MixedSpecPlan &q : plans) {

@@ -121,6 +121,15 @@ std::string spec_mixed_source(const std::vector<MixedSpecPlan> &plans, int threa
 // backtrace's label words in registers).  Bit-identical to it.
 std::string spec_map_source(const CompiledPlan &cp, int glog, int threads);
 
+// The same kernel with `waves` wavefronts per workgroup that each own
+// 2^glog syndromes: no workgroup barrier between steps, tables in LDS,
+// arg-max records as ballot masks in registers, the backtrace in registers.
+// Bit-identical.
+// spec_map_wave_cfg chooses glog and waves; false where eight waves do not
+// share `lds_limit`.
+bool spec_map_wave_cfg(const CompiledPlan &cp, size_t lds_limit, int &glog, int &waves);
+std::string spec_map_wave_source(const CompiledPlan &cp, int glog, int waves);
+
 inline const char *spec_kernel_name(const SpecCfg &cfg) {
     return cfg.fp64 ? "tqec_spec_f64" : (cfg.mfma ? "tqec_spec_bf16" : "tqec_spec_f32");
 }

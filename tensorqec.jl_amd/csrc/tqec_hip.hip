@@ -2712,9 +2712,15 @@ int tqec_map_decode_batch_device(tqec_plan *p, const uint8_t *d_syn, int64_t n, 
     const int64_t ntiles = (n + (1 << gl) - 1) >> gl;
     const int per_cu = resident_per_cu(lds, threads, p->lds_limit);
     const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(ntiles, (int64_t)p->n_cu * per_cu));
+    // the generated kernel: a wave per syndromes where it fits, else a workgroup tile
+    int wgl = -1, waves = 0, wthreads = threads;
+    if (p->map_spec) {
+        if (spec_map_wave_cfg(cp, p->lds_limit, wgl, waves)) wthreads = 64 * waves;
+        else wgl = -1;
+    }
     if (p->map_spec) {
         // plan-specialised max-product kernel (hiprtc, cached per device and tile)
-        const auto key = std::make_tuple(dev, gl, threads, 0, 0, 1, 1 << 20);
+        const auto key = std::make_tuple(dev, wgl >= 0 ? wgl : gl, wthreads, 0, 0, 1, 1 << 20);
         auto it = p->spec.find(key);
         if (it == p->spec.end()) {
             // a plan whose generated kernel cannot be built (hiprtc or module
@@ -2725,7 +2731,7 @@ int tqec_map_decode_batch_device(tqec_plan *p, const uint8_t *d_syn, int64_t n, 
             SpecKernel k;
             k.lds = lds;
             std::string why;
-            if (spec_code(spec_map_source(cp, gl, threads), code)) {
+            if (spec_code(wgl >= 0 ? spec_map_wave_source(cp, wgl, waves) : spec_map_source(cp, gl, threads), code)) {
                 why = "hiprtc: " + g_last_error;
             } else {
                 hipError_t e = hipModuleLoadData(&k.mod, code.data());
@@ -2734,6 +2740,12 @@ int tqec_map_decode_batch_device(tqec_plan *p, const uint8_t *d_syn, int64_t n, 
                     if (e != hipSuccess) (void)hipModuleUnload(k.mod);
                 }
                 if (e != hipSuccess) why = std::string("module load: ") + hipGetErrorString(e);
+                int per = 0;
+                if (e == hipSuccess && wgl >= 0 &&
+                    hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per, k.fn, wthreads, 0) == hipSuccess && per > 0)
+                    k.blocks = p->n_cu * per;
+                else
+                    k.blocks = p->n_cu * per_cu;
             }
             if (why.empty()) {
                 it = p->spec.emplace(key, k).first;
@@ -2744,7 +2756,9 @@ int tqec_map_decode_batch_device(tqec_plan *p, const uint8_t *d_syn, int64_t n, 
         }
     }
     if (p->map_spec) {
-        auto it = p->spec.find(std::make_tuple(dev, gl, threads, 0, 0, 1, 1 << 20));
+        auto it = p->spec.find(std::make_tuple(dev, wgl >= 0 ? wgl : gl, wthreads, 0, 0, 1, 1 << 20));
+        const int64_t groups = wgl >= 0 ? (((n + (1 << wgl) - 1) >> wgl) + waves - 1) / waves : ntiles;
+        const unsigned sgrid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(groups, it->second.blocks));
         const unsigned char *a_syn = d_syn;
         long long a_n = (long long)n;
         const double *a_cp = dd->cpool64, *a_sp = dd->spool64;
@@ -2752,7 +2766,7 @@ int tqec_map_decode_batch_device(tqec_plan *p, const uint8_t *d_syn, int64_t n, 
         int a_nc = n_config;
         double *a_lp = d_logp;
         void *args[] = {&a_syn, &a_n, &a_cp, &a_sp, &a_cfg, &a_nc, &a_lp};
-        TQ_HIP(hipModuleLaunchKernel(it->second.fn, grid, 1, 1, (unsigned)threads, 1, 1, 0, (hipStream_t)stream, args,
+        TQ_HIP(hipModuleLaunchKernel(it->second.fn, sgrid, 1, 1, (unsigned)wthreads, 1, 1, 0, (hipStream_t)stream, args,
                                      nullptr));
         return TQEC_OK;
     }
