@@ -88,6 +88,13 @@ struct SamplerArgs {
     unsigned long long *errm;   // [ceil(n / 64)][2 nvar] (2 j: x, 2 j + 1: z) or [..][nvar]
 };
 
+// Bit i of a mask, by its 32-bit half: kernels with 64-bit shifts by a
+// register have returned wrong bits now and then.
+__device__ __forceinline__ uint32_t mask_bit(unsigned long long m, int i) {
+    const uint32_t w = i < 32 ? (uint32_t)m : (uint32_t)(m >> 32);
+    return (w >> (i & 31)) & 1u;
+}
+
 // Rows of `width` bytes of samples [0, rows) out to `out`, byte c of a sample
 // being its bit of mask at(c).  Four bytes per store where `out` allows it.
 template <typename At>
@@ -101,7 +108,7 @@ __device__ __forceinline__ void store_bits(uint8_t *__restrict__ out, int rows, 
             uint32_t v = 0;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                v |= (uint32_t)((at(c) >> i) & 1ull) << (8 * e);
+                v |= mask_bit(at(c), i) << (8 * e);
                 if (++c == width) {
                     c = 0;
                     ++i;
@@ -112,7 +119,7 @@ __device__ __forceinline__ void store_bits(uint8_t *__restrict__ out, int rows, 
     }
     for (int f = done + t0; f < total; f += nt) {
         const int i = f / width;
-        out[f] = (uint8_t)((at(f - i * width) >> i) & 1ull);
+        out[f] = (uint8_t)mask_bit(at(f - i * width), i);
     }
 }
 
@@ -165,7 +172,7 @@ __global__ void __launch_bounds__(256) sample_kernel(SamplerArgs a) {
     store_bits(a.syn + b0 * a.nsyn, rows, a.nsyn, [&](int c) { return row[c]; });
     if (a.cls && (int)threadIdx.x < rows) {
         uint32_t c = 0;
-        for (int l = 0; l < a.nlog; ++l) c |= (uint32_t)((row[a.nsyn + l] >> threadIdx.x) & 1ull) << l;
+        for (int l = 0; l < a.nlog; ++l) c |= mask_bit(row[a.nsyn + l], threadIdx.x) << l;
         a.cls[b0 + threadIdx.x] = (int32_t)c;
     }
     if (a.err) {
