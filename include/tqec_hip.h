@@ -314,7 +314,7 @@ int tqec_mixed_set_graph(tqec_mixed *m, int32_t enable);
 int tqec_mixed_set_order(tqec_mixed *m, int32_t order);
 /* Kernel of the executor: the generic interpreter of the step descriptors
  * (default), or one kernel generated from every plan's specialised code
- * (each plan's current SPEC_F32 tile, 128 threads, compiled with hiprtc
+ * (each plan's current SPEC_F32 tile, 256 threads, compiled with hiprtc
  * here; results bit-identical).  Waits for calls in flight. */
 #define TQEC_MIXED_KERNEL_GENERIC 0
 #define TQEC_MIXED_KERNEL_SPEC 1

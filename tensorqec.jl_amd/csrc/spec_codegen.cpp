@@ -1823,11 +1823,14 @@ size_t spec_slab_entries(const CompiledPlan &cp, const SpecCfg &cfg) {
 
 namespace {
 
+// `opaque`: hide the thread id from the compiler, so that nothing computed
+// from it is moved out of the loop that calls the function.
 // One tile of G syndromes (rows b0.., or list entries b0..) through the
 // whole step program, as a device function: the body of the generic fused
 // kernel's tile with every descriptor value substituted.  Starts and ends
 // with a workgroup barrier.
-void emit_tile_fn(std::ostringstream &o, const CompiledPlan &cp, const SpecCfg &cfg, const std::string &name) {
+void emit_tile_fn(std::ostringstream &o, const CompiledPlan &cp, const SpecCfg &cfg, const std::string &name,
+                  bool opaque = false) {
     const Layout L = layout(cp, cfg);
     const size_t const_n = cp.const_pool.size();
     const int nsteps = (int)cp.steps.size();
@@ -1852,7 +1855,9 @@ void emit_tile_fn(std::ostringstream &o, const CompiledPlan &cp, const SpecCfg &
         o << "  int *lowf = reinterpret_cast<int *>(smem + " << L.low << ");\n";
     }
     o << "  unsigned char *synl = smem + " << L.syn << ";\n";
-    o << "  const int tid = threadIdx.x;\n  const int g = tid & (G - 1);\n  const int c0 = tid >> GLOG;\n"
+    o << "  int tid = threadIdx.x;\n";
+    if (opaque) o << "  asm volatile(\"\" : \"+v\"(tid));\n";
+    o << "  const int g = tid & (G - 1);\n  const int c0 = tid >> GLOG;\n"
          "  const int lane = tid & 63;\n  (void)lane; (void)c0; (void)tag_base; (void)rl; (void)rcount; (void)rcap;\n"
          "  (void)recheck_tol; (void)NSLOTS;\n";
     o << "  if (!list) {\n"
@@ -2204,7 +2209,7 @@ std::string spec_map_wave_source(const CompiledPlan &cp, int glog, int waves) {
       << ";\n";
     o << "  __shared__ __attribute__((aligned(16))) unsigned char smem[" << W.tab + (size_t)waves * W.total << "];\n";
     o << "  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);\n"
-         "  const int g = lane & (G - 1), c0 = lane >> GLOG;\n";
+         "  int g = lane & (G - 1), c0 = lane >> GLOG;\n";
     o << "  unsigned char *mine = smem + " << W.tab << " + wave * " << W.total << ";\n"
          "  double *work = reinterpret_cast<double *>(mine) + g;\n"
          "  unsigned char *synl = mine + " << W.syn << ";\n"
@@ -2376,7 +2381,7 @@ size_t spec_mixed_lds_bytes(const std::vector<MixedSpecPlan> &plans) {
 }
 
 std::string spec_mixed_source(const std::vector<MixedSpecPlan> &plans, int threads, size_t slab32_entries,
-                              size_t slab64_entries) {
+                              size_t slab64_entries, int cus) {
     std::ostringstream o;
     o << "// mixed-code kernel: plan-specialised tiles of " << plans.size() << " plans (generated)\n";
     bool any_mfma = false;
@@ -2389,10 +2394,16 @@ std::string spec_mixed_source(const std::vector<MixedSpecPlan> &plans, int threa
          "struct MCounters { unsigned long long next_tile; unsigned long long next_recheck; int rl_count; int pad;\n"
          "                   unsigned long long t_start; };\n\n";
     for (size_t i = 0; i < plans.size(); ++i) {
-        emit_tile_fn(o, *plans[i].cp, plans[i].f32, "p" + std::to_string(i) + "_f32");
-        emit_tile_fn(o, *plans[i].cp, plans[i].f64, "p" + std::to_string(i) + "_f64");
+        emit_tile_fn(o, *plans[i].cp, plans[i].f32, "p" + std::to_string(i) + "_f32", true);
+        emit_tile_fn(o, *plans[i].cp, plans[i].f64, "p" + std::to_string(i) + "_f64", true);
     }
-    o << "extern \"C\" __global__ void __launch_bounds__(" << threads << ") tqec_mixed_spec(\n"
+    // Three workgroups of 256 threads per CU: many tiles run 1.6 times as fast
+    // as with one, which is what the compiler's own choice of registers allows
+    // once it has moved every plan's address arithmetic out of the tile loop
+    // (the tile functions hide their thread id to keep it inside; else 300
+    // registers spill).
+    o << "extern \"C\" __global__ void __launch_bounds__(" << threads << ", " << (threads == 256 ? 3 : 1)
+      << ") tqec_mixed_spec(\n"
          "    const MBatch *__restrict__ batches, const MHeader *__restrict__ hdr, MCounters *ctr,\n"
          "    unsigned long long *t_done, const float *const *tabs32, const double *const *tabs64, float *slab32,\n"
          "    double *slab64) {\n";
@@ -2400,7 +2411,10 @@ std::string spec_mixed_source(const std::vector<MixedSpecPlan> &plans, int threa
     o << "  __shared__ long long grab;\n  __shared__ int loc_n;\n  __shared__ int loc_rows[64];\n";
     o << "  float *s32 = slab32 ? slab32 + (unsigned long long)blockIdx.x * " << slab32_entries << "ull : nullptr;\n";
     o << "  double *s64 = slab64 ? slab64 + (unsigned long long)blockIdx.x * " << slab64_entries << "ull : nullptr;\n";
+    // few tiles: one workgroup per CU takes them, rather than any of three
     o << "  const int nb = hdr->nbatches;\n  const long long ntiles = hdr->ntiles;\n"
+         "  if (ntiles <= "
+      << 2 * cus << " && blockIdx.x >= " << cus << ") return;\n"
          "  unsigned tag = 1;\n  bool first = true;\n"
          "  if (threadIdx.x == 0) loc_n = 0;\n"
          "  for (;;) {\n"

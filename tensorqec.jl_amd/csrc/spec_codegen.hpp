@@ -109,10 +109,11 @@ struct MixedSpecPlan {
 // MixedCounters *, unsigned long long *t_done, const float *const *tabs32,
 // const double *const *tabs64, float *slab32, double *slab64)` with the
 // batch table, header and counters of the mixed executor (tqec_hip.hip);
-// slabs hold slab32_entries / slab64_entries per workgroup.
+// slabs hold slab32_entries / slab64_entries per workgroup; `cus` workgroups
+// alone take up to twice as many tiles.
 size_t spec_mixed_lds_bytes(const std::vector<MixedSpecPlan> &plans);
 std::string spec_mixed_source(const std::vector<MixedSpecPlan> &plans, int threads, size_t slab32_entries,
-                              size_t slab64_entries);
+                              size_t slab64_entries, int cus);
 // Max-product (TNMAP) plan: kernel `tqec_map_spec(const unsigned char *syn,
 // long long n, const double *cpool, const double *spool, unsigned char
 // *config, int n_config, double *logp)`, G = 2^glog syndromes per

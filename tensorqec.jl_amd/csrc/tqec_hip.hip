@@ -2120,7 +2120,7 @@ struct tqec_mixed {
     bool spec = false;
     hipModule_t spec_mod = nullptr;
     hipFunction_t spec_fn = nullptr;
-    int spec_threads = 128, spec_blocks = 0;
+    int spec_threads = 256, spec_blocks = 0;
     std::vector<int> spec_glog, spec_slab;   // per plan: FP32 tile, slab flags (bit 0 FP32, bit 1 FP64)
     const void **d_tabs32 = nullptr, **d_tabs64 = nullptr;
     float *spec_slab32 = nullptr;
@@ -2225,8 +2225,13 @@ int mixed_spec_layout(const std::vector<tqec_plan *> &plans, int nt, size_t lds_
         if (tuned) {
             c = p->spec_cfg;
         } else {
-            // the default tile of the largest size whose LDS image fits the budget
-            c.glog = 6;
+            // 32 syndromes, or as many as fit the budget, in blocks of 4
+            // outputs.  24 batches of 6,800 rows, five codes, us (tiles of
+            // 64 / 32 / 16): 128 threads 116 (one output at a time), 83 / 83 /
+            // 85 (blocks of 4), 256 threads 59 / 61 / 72; 16 leaves most time
+            // to the slab plan's tiles, 64 to a few tiles of the widest LDS plan.
+            c.glog = 5;
+            c.unroll = 4;
             c.threads = nt;
             c.tab_lds = false;
             while (c.glog > 0 && spec_lds_bytes(p->cp, c) > budget) --c.glog;
@@ -3305,14 +3310,17 @@ int tqec_mixed_set_kernel(tqec_mixed *m, int32_t kind) {
     const size_t lds = spec_mixed_lds_bytes(sp) + 8 + 4 + 256;
     if (lds > lds_limit) return set_error(TQEC_EUNSUPPORTED, "the plans' tiles exceed the LDS");
     std::vector<char> code;
-    if ((rc = spec_code(spec_mixed_source(sp, nt, std::max<size_t>(s32, 1), std::max<size_t>(s64, 1)), code))) return rc;
+    if ((rc = spec_code(spec_mixed_source(sp, nt, std::max<size_t>(s32, 1), std::max<size_t>(s64, 1), n_cu), code))) return rc;
     TQ_HIP(hipModuleLoadData(&m->spec_mod, code.data()));
     hipError_t e = hipModuleGetFunction(&m->spec_fn, m->spec_mod, "tqec_mixed_spec");
     if (e != hipSuccess) {
         mixed_free_spec(m);
         return set_error(TQEC_EDEVICE, std::string("hipModuleGetFunction: ") + hipGetErrorString(e));
     }
-    m->spec_blocks = n_cu * resident_per_cu(lds, nt, lds_limit);
+    int per_cu = resident_per_cu(lds, nt, lds_limit), occ = 0;
+    if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&occ, m->spec_fn, nt, 0) == hipSuccess && occ > 0)
+        per_cu = std::min(per_cu, occ);
+    m->spec_blocks = n_cu * per_cu;
     if (const size_t per = s32 * sizeof(float) + s64 * sizeof(double))
         m->spec_blocks = (int)std::max<size_t>((size_t)n_cu, std::min<size_t>((size_t)m->spec_blocks, kMixedSlabTotal / per));
     std::vector<const void *> t32(m->plans.size()), t64(m->plans.size());
@@ -3360,7 +3368,7 @@ int tqec_mixed_spec_source(tqec_plan *const *plans, int32_t n_plans, int32_t thr
     int rc;
     // gfx950: 160 KiB of LDS per workgroup
     if ((rc = mixed_spec_layout(v, threads, size_t(160) << 10, sp, glog, slabf, s32, s64))) return rc;
-    const std::string src = spec_mixed_source(sp, threads, std::max<size_t>(s32, 1), std::max<size_t>(s64, 1));
+    const std::string src = spec_mixed_source(sp, threads, std::max<size_t>(s32, 1), std::max<size_t>(s64, 1), 256);
     if (len) *len = src.size();
     if (buf && cap > 0) {
         const size_t k = std::min(cap - 1, src.size());
