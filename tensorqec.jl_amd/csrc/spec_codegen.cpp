@@ -2172,8 +2172,10 @@ MapWaveLayout map_wave_layout(const CompiledPlan &cp, int glog) {
 // lanes an output each on average; fewer where eight waves would not share the
 // LDS.  us, workgroup tile -> G = 2 / 4 / 8 per wave: 16,384 rows 47 -> 52 / 29
 // / 23, 65,536 rows 162 -> 170 / 108 / 82 (d=3, 65,536 rows, G = 4 / 8 / 16: 23
-// / 14 / 11).  Two waves per SIMD: with one (all the registers the compiler
-// wants) 31 us instead of 23.
+// / 14 / 11).  Three waves per SIMD, and the lane id hidden in the group loop:
+// the compiler otherwise moves the address arithmetic of all steps out of it,
+// and with all the registers it wants for that (one wave per SIMD) the 23 us
+// are 31; a d=7 plan takes 151 us per 16,384 rows instead of 215.
 bool spec_map_wave_cfg(const CompiledPlan &cp, size_t lds_limit, int &glog, int &waves) {
     if (cp.steps.empty()) return false;
     int64_t outputs = 0;
@@ -2200,18 +2202,15 @@ std::string spec_map_wave_source(const CompiledPlan &cp, int glog, int waves) {
     const MapWaveLayout W = map_wave_layout(cp, glog);
     std::ostringstream o;
     o << "// plan-specialised max-product (TNMAP) kernel, a wave per " << G << " syndromes (generated)\n";
-    // the LDS holds two waves per SIMD at least: registers for as many
-    o << "extern \"C\" __global__ void __launch_bounds__(" << nt << ", 2) tqec_map_spec(\n"
+    o << "extern \"C\" __global__ void __launch_bounds__(" << nt << ", 3) tqec_map_spec(\n"
          "    const unsigned char *__restrict__ syn, long long n, const double *__restrict__ cpool,\n"
          "    const double *__restrict__ spool, unsigned char *__restrict__ config, int n_config,\n"
          "    double *__restrict__ logp) {\n";
     o << "  constexpr int G = " << G << ", GLOG = " << glog << ", LANES = " << lanes << ", NBITS = " << cp.n_syn
       << ";\n";
     o << "  __shared__ __attribute__((aligned(16))) unsigned char smem[" << W.tab + (size_t)waves * W.total << "];\n";
-    o << "  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);\n"
-         "  int g = lane & (G - 1), c0 = lane >> GLOG;\n";
+    o << "  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);\n";
     o << "  unsigned char *mine = smem + " << W.tab << " + wave * " << W.total << ";\n"
-         "  double *work = reinterpret_cast<double *>(mine) + g;\n"
          "  unsigned char *synl = mine + " << W.syn << ";\n"
          "  unsigned *cfgw = reinterpret_cast<unsigned *>(synl);\n";
     if (W.tab) {
@@ -2228,6 +2227,10 @@ std::string spec_map_wave_source(const CompiledPlan &cp, int glog, int waves) {
     o << "  const long long ntiles = (n + G - 1) >> GLOG;\n"
          "  for (long long t = (long long)blockIdx.x * " << waves << " + wave; t < ntiles; t += (long long)gridDim.x * "
       << waves << ") {\n"
+         "    int lane = threadIdx.x & 63;\n"
+         "    asm volatile(\"\" : \"+v\"(lane));   // keeps address arithmetic inside the loop\n"
+         "    const int g = lane & (G - 1), c0 = lane >> GLOG;\n"
+         "    double *work = reinterpret_cast<double *>(mine) + g;\n"
          "    const long long q = (t << GLOG) + g;\n"
          "    const bool valid = q < n;\n"
          "    // lanes beyond the last row read it again and store nothing\n"
