@@ -1260,7 +1260,8 @@ bool emit_reg_step(std::vector<RegChunk> &out, const CompiledPlan &cp, const Reg
     const std::string S = std::to_string(s);
     const char *ab[2] = {"a", "b"};
     std::ostringstream first, addr;
-    first << "    // step " << s << ": rank " << st.rc << ", contracted " << st.nk << ", " << nreg << " registers per lane";
+    // the step program is a scope of its own, which the first step opens
+    first << (s == 0 ? "    { // step " : "    // step ") << s << ": rank " << st.rc << ", contracted " << st.nk << ", " << nreg << " registers per lane";
     if (rs) first << "; bound 2^" << (int)std::ceil(rs->pre[s]) << " before a shift of " << rs->shift[s] << ", exponent "
                   << rs->E[s];
     first << "\n    " << T;
@@ -1406,7 +1407,7 @@ bool emit_reg_step(std::vector<RegChunk> &out, const CompiledPlan &cp, const Reg
                 nx.push_back(mx[i]);
                 continue;
             }
-            const std::string t = "mx" + S + "_" + std::to_string(nm++);
+            const std::string t = "lmax" + S + "_" + std::to_string(nm++);
             o << "    const float " << t << " = ";
             if (i + 2 < mx.size())
                 o << "fmaxf(fmaxf(" << mx[i] << ", " << mx[i + 1] << "), " << mx[i + 2] << ");\n";
@@ -1520,13 +1521,14 @@ Recheck recheck_plan(const CompiledPlan &cp, const SpecCfg &cfg) {
     return r;
 }
 
-// recheck64: one row by one wave, the generic FP64 kernel's arithmetic.
+// recheck64: one row by one wave, the generic FP64 kernel's arithmetic; and
+// the flagged rows wave, wave + r.rows, .. of a tile.
 void emit_recheck_fn(std::ostringstream &o, const CompiledPlan &cp, const Recheck &r) {
     const int nb = std::max(1, cp.n_syn);
     const size_t const_n = cp.const_pool.size();
     o << "__device__ __attribute__((noinline)) void recheck64(const unsigned char *__restrict__ row, long long b,\n"
          "    const double *__restrict__ tab, double *__restrict__ mar, int *__restrict__ cls,\n"
-         "    unsigned char *__restrict__ ties, double tie_tol, double *work) {\n"
+         "    unsigned char *__restrict__ ties, double tie_tol, __attribute__((address_space(3))) double * work) {\n"
          "  using T = double;\n  constexpr int GLOG = 0, NOUT = "
       << (1 << cp.n_out) << ";\n  const int c0 = threadIdx.x & 63;\n";
     // the row's bits, uniform over the wave
@@ -1577,12 +1579,12 @@ void emit_recheck_fn(std::ostringstream &o, const CompiledPlan &cp, const Rechec
         o << "  { // step " << s << "\n";
         for (int side = 0; side < 2; ++side) {
             const OperandDesc &op = side ? st.b : st.a;
-            o << "    const T *p" << (side ? "b" : "a") << " = ";
+            o << "    const auto p" << (side ? "b" : "a") << " = ";
             if (op.kind == kInter) o << "work + " << (long long)op.off << ";\n";
             else if (r.tables) o << "work + " << r.at[s][side] << ";\n";
             else o << base(op) << ";\n";
         }
-        o << "    T *pc = work + " << (long long)st.c_off << ";\n";
+        o << "    const auto pc = work + " << (long long)st.c_off << ";\n";
         emit_outputs(o, st, 64, 4, true);
         o << "  }\n" << sync;
     }
@@ -1605,6 +1607,14 @@ void emit_recheck_fn(std::ostringstream &o, const CompiledPlan &cp, const Rechec
          "    const bool low = NOUT > 1 && second >= 0 && best - second <= tie_tol * best;\n"
          "    if (ties) ties[b] = low ? 1 : 0;\n"
          "  }\n" << sync << "}\n\n";
+    // LDS by its own address space (a generic pointer means flat loads and 182
+    // registers instead of 136 at d=7); the loop stays outside the call: inside, its address arithmetic takes
+    // registers (d=7: 248) that the call has to save
+    o << "__device__ __forceinline__ void recheck64(const unsigned char *syn, int nf, const int *flagged, int wave,\n"
+         "    const double *tab, double *mar, int *cls, unsigned char *ties, double tie_tol, __attribute__((address_space(3))) double * work) {\n"
+         "  for (int i = wave; i < nf; i += " << r.rows << ")\n"
+         "    recheck64(syn + (long long)flagged[i] * " << nb << ", (long long)flagged[i], tab, mar, cls, ties, tie_tol, work);\n"
+         "}\n\n";
 }
 
 std::string reg_source(const CompiledPlan &cp, const SpecCfg &cfg, std::string &err) {
@@ -1760,16 +1770,15 @@ std::string reg_source(const CompiledPlan &cp, const SpecCfg &cfg, std::string &
              "        }\n"
              "      }\n";
     o << "    }\n"
+         "    }\n"
          "   }\n"
          "   __syncthreads();\n";
     if (inl)
         // at most G flagged rows (one per valid row of the tile)
         o << "   const int nf = seg_n;\n"
              "   if (wave < "
-          << rck.rows << ")\n"
-             "     for (int i = wave; i < nf; i += "
-          << rck.rows << ")\n"
-             "       recheck64(syn + (long long)flagged[i] * NBITS, flagged[i], gtab64, mar, cls, ties, tie_tol, work64[wave]);\n"
+          << rck.rows << ") recheck64(syn, nf, flagged, wave, gtab64, mar, cls, ties, tie_tol,\n"
+             "      (__attribute__((address_space(3))) double *)work64[wave]);\n"
              "   if (threadIdx.x == 0 && rcount) rcount[t] = nf;\n"
              "   __syncthreads();\n";
     else
