@@ -478,13 +478,28 @@ SamplerArgs sampler_args(const tqec_sampler *s, uint64_t seed, int64_t first, in
     return a;
 }
 
-int launch_sample(const SamplerArgs &a, hipStream_t stream) {
-    const size_t lds = sample_lds(a.kind == 0 ? 2 : 1, a.nvar, a.nsyn, a.nlog);
-    if (lds <= kSampleLds)
-        hipLaunchKernelGGL(sample_kernel, dim3((unsigned)((a.n + 63) / 64)), dim3(256), lds, stream, a);
-    else
-        hipLaunchKernelGGL(sample_large_kernel, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, stream, a);
-    TQS_HIP(hipGetLastError());
+// Samples of one launch: a grid holds fewer than 2^32 work-items, and the
+// kernel below takes four per sample.
+constexpr int64_t kSampleLaunch = int64_t(1) << 29;
+
+int launch_sample(const SamplerArgs &all, hipStream_t stream) {
+    const int es = all.kind == 0 ? 2 : 1;
+    const size_t lds = sample_lds(es, all.nvar, all.nsyn, all.nlog);
+    for (int64_t off = 0; off < all.n; off += kSampleLaunch) {
+        SamplerArgs a = all;
+        a.first += off;
+        a.n = std::min(kSampleLaunch, all.n - off);
+        a.syn += off * a.nsyn;
+        if (a.cls) a.cls += off;
+        if (a.err) a.err += off * es * a.nvar;
+        if (a.synm) a.synm += off / 64 * a.nsyn;
+        if (a.errm) a.errm += off / 64 * es * a.nvar;
+        if (lds <= kSampleLds)
+            hipLaunchKernelGGL(sample_kernel, dim3((unsigned)((a.n + 63) / 64)), dim3(256), lds, stream, a);
+        else
+            hipLaunchKernelGGL(sample_large_kernel, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, stream, a);
+        TQS_HIP(hipGetLastError());
+    }
     return TQEC_OK;
 }
 
