@@ -88,8 +88,14 @@ struct SamplerArgs {
     unsigned long long *errm;   // [ceil(n / 64)][2 nvar] (2 j: x, 2 j + 1: z) or [..][nvar]
 };
 
-// Bit i of a mask, by its 32-bit half: kernels with 64-bit shifts by a
-// register have returned wrong bits now and then.
+// Bit i of a mask, by its 32-bit half.  Two builds of the max-product wave
+// kernel took such bits with a 64-bit shift by a vector register, and in some
+// runs a few rows came out with one wrong bit (always of the same label, the
+// log-probabilities right); the same source with 32-bit halves gave none in 60
+// configurations of 60 runs.  Reading the two builds showed no missing wait or
+// ordering between lanes, so the cause is not known, and no kernel of the
+// library shifts 64 bits by a vector register any more (shifts by a scalar
+// register, as of a uniform index, were never seen to fail).
 __device__ __forceinline__ uint32_t mask_bit(unsigned long long m, int i) {
     const uint32_t w = i < 32 ? (uint32_t)m : (uint32_t)(m >> 32);
     return (w >> (i & 31)) & 1u;

@@ -2353,8 +2353,8 @@ std::string spec_map_wave_source(const CompiledPlan &cp, int glog, int waves) {
         for (int j = 0; j < ms.nc; ++j)
             if (known[lab[j]]) o << "      c |= L" << lab[j] << " << " << j << ";\n";
         o << "      const unsigned at = ((c & " << lanes - 1 << "u) << GLOG) | (unsigned)g;\n";
-        // 32-bit halves: no variable 64-bit shifts (a kernel made of those gave
-        // wrong bits now and then)
+        // 32-bit halves: no 64-bit shifts by a vector register (see mask_bit in
+        // sampler_hip.hip)
         const bool low = (int64_t(1) << (st.rc + glog)) <= 32;
         for (int j = 0; j < nb; ++j)
             for (int x = 0; x < blocks; ++x) {

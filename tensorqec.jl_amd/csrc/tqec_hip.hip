@@ -112,6 +112,12 @@ __device__ __forceinline__ T contract_one(const StepDesc &st, uint32_t c, const 
     return acc;
 }
 
+// (int64_t)v << r for 0 <= r < 32, by 32-bit halves: no 64-bit shift by a
+// vector register (see mask_bit in sampler_hip.hip).
+__device__ __forceinline__ int64_t shl64(uint32_t v, int r) {
+    return (int64_t)(((uint64_t)((v >> 1) >> (31 - r)) << 32) | (uint64_t)(v << r));
+}
+
 // Base pointer of an operand for syndrome b of the plain executor.
 template <typename T>
 __device__ __forceinline__ const T *plain_base(const OperandDesc &op, int64_t b, const T *ws, int64_t ldw,
@@ -120,7 +126,7 @@ __device__ __forceinline__ const T *plain_base(const OperandDesc &op, int64_t b,
     if (op.kind == kConst) return pools.cpool + op.off;
     uint32_t v = 0;
     for (int j = 0; j < op.nev; ++j) v |= (uint32_t)synT[(int64_t)op.ev_bit[j] * ldw + b] << j;
-    return pools.spool + op.off + ((int64_t)v << op.rank);
+    return pools.spool + op.off + shl64(v, op.rank);
 }
 
 // Per-slot, per-syndrome scale of the wide FP32 executor: the largest
@@ -319,7 +325,7 @@ __device__ __forceinline__ const T *fused_base(const OperandDesc &op, int g, int
     if (op.kind == kConst) return cpool + op.off;
     uint32_t v = 0;
     for (int j = 0; j < op.nev; ++j) v |= (uint32_t)synl[(op.ev_bit[j] << glog) + g] << j;
-    return spool + op.off + ((int64_t)v << op.rank);
+    return spool + op.off + shl64(v, op.rank);
 }
 
 template <typename T, bool SCALE, bool AW, bool BW>
