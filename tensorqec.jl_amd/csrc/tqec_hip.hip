@@ -2006,6 +2006,17 @@ int grow_pinned(void **ptr, size_t *cap, size_t need) {
     return TQEC_OK;
 }
 
+// Waits for a host call's copies when it returns early: they may still be
+// reading the staging buffer, which the next call on the stream writes on the
+// CPU, or the caller's arrays.
+struct CopiesInFlight {
+    hipStream_t stream;
+    bool pending = false;
+    ~CopiesInFlight() {
+        if (pending) (void)hipStreamSynchronize(stream);
+    }
+};
+
 // Decode a host batch and, when asked, recover its error patterns.
 int decode_host(tqec_plan *p, const uint8_t *syn, int64_t n, int32_t mode, double *mar, int32_t *cls, uint8_t *tie,
                 const HostRecovery *rec, void *stream) {
@@ -2047,6 +2058,8 @@ int decode_host(tqec_plan *p, const uint8_t *syn, int64_t n, int32_t mode, doubl
         if ((rc = grow((char **)&w.d_syn, &w.d_syn_bytes, total))) return rc;
         d = (char *)w.d_syn;
     }
+    CopiesInFlight copies{st};
+    copies.pending = true;
     if (staged) {
         std::memcpy(h + o_syn, syn, syn_b);
         TQ_HIP(hipMemcpyAsync(d, h, o_syn + syn_b, hipMemcpyHostToDevice, st));
@@ -2072,6 +2085,7 @@ int decode_host(tqec_plan *p, const uint8_t *syn, int64_t n, int32_t mode, doubl
         for (const auto &o : outs)
             if (o.bytes) TQ_HIP(hipMemcpyAsync(o.to, d + o.off, o.bytes, hipMemcpyDeviceToHost, st));
     TQ_HIP(hipStreamSynchronize(st));
+    copies.pending = false;
     if (staged)
         for (const auto &o : outs)
             if (o.bytes) std::memcpy(o.to, h + o.off, o.bytes);

@@ -1,0 +1,48 @@
+// The HIP calls of the library's host paths on host memory, for CPU tests
+// (preloaded in front of the runtime): allocations are malloc's, copies are
+// memcpy's, kernels do nothing.  Every call that the tests look at is printed
+// on stderr; TQEC_STUB_FAIL names one that fails.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+
+static hipError_t g_last = hipSuccess;
+
+static hipError_t call(const char *name) {
+    const char *f = getenv("TQEC_STUB_FAIL");
+    const bool bad = f && !strcmp(f, name);
+    fprintf(stderr, "stub %s%s\n", name, bad ? " failed" : "");
+    return bad ? (g_last = hipErrorUnknown) : hipSuccess;
+}
+
+extern "C" {
+hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_t *p, int) {
+    memset(p, 0, sizeof *p);
+    p->sharedMemPerBlock = p->maxSharedMemoryPerMultiProcessor = 160 * 1024;
+    p->multiProcessorCount = 256;
+    return hipSuccess;
+}
+hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t hipMalloc(void **p, size_t n) { *p = malloc(n ? n : 1); return hipSuccess; }
+hipError_t hipFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { *p = malloc(n ? n : 1); return hipSuccess; }
+hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) {
+    const hipError_t e = call(k == hipMemcpyHostToDevice ? "copy_in" : "copy_out");
+    if (!e) memcpy(d, s, n);
+    return e;
+}
+hipError_t hipStreamSynchronize(hipStream_t) { return call("wait"); }
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return call("launch"); }
+hipError_t hipGetLastError() {
+    const hipError_t e = g_last;
+    g_last = hipSuccess;
+    return e;
+}
+}

@@ -1,0 +1,59 @@
+"""Host paths of the library over a stub of the HIP calls on host memory
+(hip_stub.cpp): what they enqueue and wait for, and what they choose, without
+a GPU."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+REPO = os.path.dirname(HERE)
+
+PLAN = """
+import sys
+sys.path[:0] = [%r, %r]
+import numpy as np
+from tensorqec import decoders as D, lib as L
+from tensorqec.codes import CSSTannerGraph, SurfaceCode
+from tensorqec.errors import iid_error
+t = CSSTannerGraph.from_code(SurfaceCode(3, 3))
+ct = D.compile(D.TNMMAP(), t, iid_error(0.02, 0.02, 0.02, t.nq))
+""" % (REPO, os.path.join(REPO, "tensorqec.jl_amd"))
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    hipcc = "/opt/rocm/bin/hipcc" if os.path.exists("/opt/rocm/bin/hipcc") else shutil.which("hipcc")
+    if not hipcc:
+        pytest.skip("hipcc not available")
+    out = tmp_path_factory.mktemp("stub") / "libhip_stub.so"
+    subprocess.run([hipcc, "-x", "hip", "--offload-arch=gfx950", "-O1", "-shared", "-fPIC", os.path.join(HERE, "hip_stub.cpp"), "-o", str(out)],
+                   check=True, capture_output=True, timeout=300)
+    return str(out)
+
+
+def run(stub, code, **env):
+    r = subprocess.run([sys.executable, "-c", PLAN + code], capture_output=True, text=True, timeout=300,
+                       env={**os.environ, "LD_PRELOAD": stub, **env})
+    assert r.returncode == 0, r.stderr[-2000:]
+    return r.stdout, [l[5:] for l in r.stderr.splitlines() if l.startswith("stub ")]
+
+
+@pytest.mark.parametrize("rows", [3, 200000])          # pinned staging, copies of the caller's arrays
+@pytest.mark.parametrize("fail", ["launch", "copy_out"])
+@pytest.mark.parametrize("patterns", [False, True])
+def test_failed_host_call_waits_for_its_copies(stub, rows, fail, patterns):
+    """The staging buffer is written again by the next call, the caller's
+    arrays may be gone: neither before the copies out of them have ended."""
+    out, calls = run(stub, """
+S = np.zeros((%d, ct.plan.n_syndrome_bits), np.uint8)
+try:
+    D.decode_batch(ct, S, error_patterns=%r)
+except L.TqecError:
+    print("failed")
+""" % (rows, patterns), TQEC_STUB_FAIL=fail)
+    assert out.strip() == "failed" and fail + " failed" in calls
+    assert "wait" in calls[max(i for i, c in enumerate(calls) if c.startswith("copy_in")):]
+    assert calls[-1] == "wait"
