@@ -314,8 +314,11 @@ int tqec_mixed_set_graph(tqec_mixed *m, int32_t enable);
 int tqec_mixed_set_order(tqec_mixed *m, int32_t order);
 /* Kernel of the executor: the generic interpreter of the step descriptors
  * (default), or one kernel generated from every plan's specialised code
- * (each plan's current SPEC_F32 tile, 256 threads, compiled with hiprtc
- * here; results bit-identical).  Waits for calls in flight. */
+ * (each plan's pinned or tuned SPEC_F32 tile, else a default that depends on
+ * the plan only; 256 threads, compiled with hiprtc here).  Results are
+ * bit-identical, except within the FP32 tolerance where a tile's GEMM-shaped
+ * steps run on FP32 MFMA: plans too wide for LDS, and tiles pinned or tuned
+ * so.  Waits for calls in flight. */
 #define TQEC_MIXED_KERNEL_GENERIC 0
 #define TQEC_MIXED_KERNEL_SPEC 1
 int tqec_mixed_set_kernel(tqec_mixed *m, int32_t kind);

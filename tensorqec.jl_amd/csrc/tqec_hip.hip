@@ -880,6 +880,7 @@ struct tqec_plan {
     int n_cu = 0;
     SpecCfg spec_cfg;
     bool spec_cfg_set = false;
+    bool spec_cfg_pinned = false;   // spec_cfg came from the caller or the autotuner, not from choose_spec
     std::map<std::tuple<int, int, int, int, int, int, int>, SpecKernel> spec;   // (device, glog, threads, tab_lds, waves, fp64, flags)
     bool map_spec = true;               // max-product plans: plan-specialised kernel (else the generic one)
     std::string map_spec_note;          // why the specialised max-product kernel was given up, if it was
@@ -1952,6 +1953,7 @@ int autotune_spec(tqec_plan *p, const uint8_t *d_syn, int64_t n, hipStream_t st,
     }
     tcfg = best;
     tset = true;
+    if (!bf16) p->spec_cfg_pinned = true;
     if (tile) *tile = 1 << best.glog;
     if (threads) *threads = best.threads;
     return TQEC_OK;
@@ -2224,9 +2226,9 @@ void mixed_drop_graphs(tqec_mixed *m) {
     }
 }
 
-// Per-plan tiles of the generated mixed kernel: each plan's current SPEC_F32
-// LDS-tile configuration (or the default: a register-resident configuration
-// does not apply here) with the kernel's thread count and no
+// Per-plan tiles of the generated mixed kernel: each plan's pinned or tuned
+// SPEC_F32 LDS-tile configuration (or a default: a register-resident
+// configuration does not apply here) with the kernel's thread count and no
 // tables in LDS, its tile shrunk until it fits half the LDS (else a slab),
 // and an FP64 tile of one syndrome for the re-checks.
 int mixed_spec_layout(const std::vector<tqec_plan *> &plans, int nt, size_t lds_limit, std::vector<MixedSpecPlan> &sp,
@@ -2241,7 +2243,9 @@ int mixed_spec_layout(const std::vector<tqec_plan *> &plans, int nt, size_t lds_
         if (p->cp.semiring != TQEC_SEMIRING_SUM)
             return set_error(TQEC_EINVAL, "plan " + std::to_string(i) + " is a max-product plan");
         SpecCfg c;
-        const bool tuned = p->spec_cfg_set && p->spec_cfg.glog >= 0 && !p->spec_cfg.reg;
+        // a default that some other call happened to choose before does not
+        // count: the kernel depends on the plans and their pinned tiles only
+        const bool tuned = p->spec_cfg_pinned && p->spec_cfg.glog >= 0 && !p->spec_cfg.reg;
         if (tuned) {
             c = p->spec_cfg;
         } else {
@@ -2854,7 +2858,7 @@ int tqec_plan_set_tile(tqec_plan *p, int32_t mode, int32_t tile, int32_t threads
         if (!spec_fits(p, c)) c.tab_lds = false;
         if (!spec_fits(p, c)) return set_error(TQEC_EUNSUPPORTED, "tile does not fit in LDS");
         p->spec_cfg = c;
-        p->spec_cfg_set = true;
+        p->spec_cfg_set = p->spec_cfg_pinned = true;
         return TQEC_OK;
     }
     const bool f32 = mode == TQEC_MODE_FUSED_F32;
@@ -3253,7 +3257,7 @@ int tqec_plan_set_spec(tqec_plan *p, int32_t tile, int32_t threads, int32_t flag
         p->specb_cfg_set = true;
     } else {
         p->spec_cfg = c;
-        p->spec_cfg_set = true;
+        p->spec_cfg_set = p->spec_cfg_pinned = true;
     }
     return TQEC_OK;
 }

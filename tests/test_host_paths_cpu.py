@@ -57,3 +57,19 @@ except L.TqecError:
     assert out.strip() == "failed" and fail + " failed" in calls
     assert "wait" in calls[max(i for i, c in enumerate(calls) if c.startswith("copy_in")):]
     assert calls[-1] == "wait"
+
+
+def test_mixed_kernel_does_not_depend_on_earlier_calls(stub):
+    """A plan whose default FP32 tile runs GEMM-shaped steps on MFMA: asking
+    for that default, or decoding with it, leaves the mixed-code kernel as it
+    was; a pinned tile changes it."""
+    out, _ = run(stub, """
+from tensorqec.circuits import detector_error_model_from_stim, rotated_memory_z
+hip = D.compile(D.TNMMAP(optimizer=D.Dissection(seeds=1)), detector_error_model_from_stim(rotated_memory_z(3, 3, 0.001))).hip
+first = L.mixed_spec_source([ct.hip, hip], 256)
+cfg = hip.spec_config()
+print(cfg["mfma32"], cfg["slab"], L.mixed_spec_source([ct.hip, hip], 256) == first)
+hip.set_spec(1, 256, False, mfma32=True)
+print("mfma" in first, "mfma" in L.mixed_spec_source([ct.hip, hip], 256))
+""")
+    assert out.split() == ["True", "False", "True", "False", "True"]
