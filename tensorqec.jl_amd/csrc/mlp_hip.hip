@@ -44,7 +44,7 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 __device__ __forceinline__ float bf2f(bf16 h) { return __uint_as_float(((uint32_t)h) << 16); }
 // Round to nearest even, one v_cvt_pk_bf16_f32 for two values (rounding in
 // integer arithmetic, five instructions a value, made the fused forward kernel
-// 83 us instead of 75 at 65,536 rows).
+// 73.6 us instead of 67.5 at 65,536 rows of 48 inputs).
 typedef __attribute__((__vector_size__(2 * sizeof(float)))) float f32x2;
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bfx2;
 __device__ __forceinline__ uint32_t f2bf2(float a, float b) {
@@ -126,17 +126,22 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g) {
 
 // Forward GEMM of a hidden layer: H[M][N] = relu(A[M][K] * W + bias) with
 // the weights given transposed, Wt[N][K], so both tiles are rows of 16-byte
-// k-chunks.  Block tile 128 x (64 * NW), K step KS (64, or 32 when K is not
-// a multiple of 64), 4 waves in a 2 x 2 grid each owning 64 x (32 * NW) =
-// 2 x NW MFMA tiles;
-// the next K step's tiles are loaded into registers while the current one
-// is multiplied out of LDS.  Same MFMA sequence (k ascending in steps of 16)
-// as gemm_bf16_kernel, so the results are identical.
-template <int KS, int NW>
+// k-chunks.  Block tile 128 x 128, K step KS (64, or 32 when K is not a
+// multiple of 64), 4 waves in a 2 x 2 grid each owning 64 x 64 = 2 x 2 MFMA
+// tiles (64 x 128 were slower: one wave per SIMD); the next K step's tiles are
+// loaded into registers while the current one is multiplied out of LDS.  Same
+// MFMA sequence (k ascending in steps of 16) as gemm_bf16_kernel, so the
+// results are identical.  The biases are loaded in front of the K loop and the
+// outputs rounded in front of the branches around their stores: a bias waited
+// for after a store is a wait for that store, too (loads and stores share a
+// counter).  Forward pass of 65,536 rows of 48 inputs, width 512: 189 us, 254
+// with each output biased, rounded and stored in a branch of its own (width
+// 1024: 691 and 823, width 256: 130 and 165).
+template <int KS>
 __global__ void __launch_bounds__(256) gemm_fwd_kernel(const bf16 *__restrict__ A, const bf16 *__restrict__ Wt,
                                                        int M, int N, int K, const float *__restrict__ bias,
                                                        bf16 *__restrict__ out) {
-    constexpr int TN = 64 * NW;                // block tile columns
+    constexpr int NW = 2, TN = 64 * NW;        // MFMA tiles per wave, block tile columns
     constexpr int LK = KS + 8;                 // padded LDS row (bf16)
     constexpr int PA = 128 * KS / 8 / 256;     // 16-byte chunks per thread: A tile
     constexpr int PB = TN * KS / 8 / 256;      //                             B tile
@@ -174,6 +179,8 @@ __global__ void __launch_bounds__(256) gemm_fwd_kernel(const bf16 *__restrict__ 
     for (int i = 0; i < 2; ++i)
         for (int j = 0; j < NW; ++j)
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+    float bc[NW];
+    for (int j = 0; j < NW; ++j) bc[j] = bias[min(n0 + wn + j * 32 + (lane & 31), N - 1)];
     fetch(0);
     stash();
     __syncthreads();
@@ -199,12 +206,16 @@ __global__ void __launch_bounds__(256) gemm_fwd_kernel(const bf16 *__restrict__ 
     for (int i = 0; i < 2; ++i)
         for (int j = 0; j < NW; ++j) {
             const int col = n0 + wn + j * 32 + (lane & 31);
+            // in pairs, and before the branches around the stores
+            uint32_t u[8];
+#pragma unroll
+            for (int v = 0; v < 8; ++v)
+                u[v] = f2bf2(fmaxf(acc[i][j][2 * v] + bc[j], 0.f), fmaxf(acc[i][j][2 * v + 1] + bc[j], 0.f));
             if (col >= N) continue;
-            const float bc = bias[col];
+#pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int row = m0 + wm + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                if (row >= M) continue;
-                out[(size_t)row * N + col] = f2bf(fmaxf(acc[i][j][v] + bc, 0.f));
+                if (row < M) out[(size_t)row * N + col] = (bf16)(u[v >> 1] >> (16 * (v & 1)));
             }
         }
 }
@@ -1233,25 +1244,14 @@ int forward(tqec_mlp *p, const uint8_t *d_syn, int64_t B, hipStream_t st, bool k
         p->wt_stale = false;
     }
     for (int l = 0; l < 3; ++l) {
-        // 64 x 128 wave tiles (NW = 4) measured slower at d=7 sizes: 252 VGPRs leave one wave per SIMD
-        const bool wide = false;
-        const dim3 grid((unsigned)(p->hid / (wide ? 256 : 128)), (unsigned)((B + 127) / 128));
+        const dim3 grid((unsigned)(p->hid / 128), (unsigned)((B + 127) / 128));
         const float *bias = p->w + p->off[2 * l + 1];
-        if (kdim[l] % 64 == 0) {
-            if (wide)
-                hipLaunchKernelGGL((gemm_fwd_kernel<64, 4>), grid, dim3(256), 0, st, in[l], p->wt[l], (int)B, p->hid,
-                                   kdim[l], bias, out[l]);
-            else
-                hipLaunchKernelGGL((gemm_fwd_kernel<64, 2>), grid, dim3(256), 0, st, in[l], p->wt[l], (int)B, p->hid,
-                                   kdim[l], bias, out[l]);
-        } else {
-            if (wide)
-                hipLaunchKernelGGL((gemm_fwd_kernel<32, 4>), grid, dim3(256), 0, st, in[l], p->wt[l], (int)B, p->hid,
-                                   kdim[l], bias, out[l]);
-            else
-                hipLaunchKernelGGL((gemm_fwd_kernel<32, 2>), grid, dim3(256), 0, st, in[l], p->wt[l], (int)B, p->hid,
-                                   kdim[l], bias, out[l]);
-        }
+        if (kdim[l] % 64 == 0)
+            hipLaunchKernelGGL(gemm_fwd_kernel<64>, grid, dim3(256), 0, st, in[l], p->wt[l], (int)B, p->hid, kdim[l],
+                               bias, out[l]);
+        else
+            hipLaunchKernelGGL(gemm_fwd_kernel<32>, grid, dim3(256), 0, st, in[l], p->wt[l], (int)B, p->hid, kdim[l],
+                               bias, out[l]);
     }
     const unsigned rows_per_block = 4;
     if (p->hid == 512 && p->nout <= 4) {

@@ -46,3 +46,15 @@ def test_generated_kernels_shift_64_bits_by_no_vector_register(kw, tmp_path):
     f = tmp_path / "spec.hip"
     f.write_text("#include <hip/hip_runtime.h>\n" + src)
     assert vector_shifts(assembly(f, tmp_path)) == []
+
+
+def test_layered_forward_waits_for_no_store_before_its_last(tmp_path):
+    """Loads and stores share a counter, so a load waited for behind a store is
+    a wait for the store: a hidden layer's epilogue loads nothing between the
+    first of its stores and the last."""
+    asm = assembly(os.path.join(CSRC, "mlp_hip.hip"), tmp_path)
+    bodies = re.findall(r"^(\S*gemm_fwd_kernel\S*):(.*?)^\.Lfunc_end", asm, re.M | re.S)
+    assert len(bodies) == 2                                # K steps of 64 and of 32
+    for _, body in bodies:
+        stores = body[body.index("global_store_short"):]
+        assert stores.count("global_store_short") == 64 and "vmcnt" not in stores
