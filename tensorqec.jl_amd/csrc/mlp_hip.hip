@@ -1099,7 +1099,7 @@ struct tqec_mlp {
     bf16 *wk[2] = {nullptr, nullptr};   // of the two inner hidden layers, for the backward pass
     bf16 *w4 = nullptr;                 // output layer's rows, padded
     bool wf_stale = true;
-    bool fused = true;             // forward / gate on the fused kernel where it applies
+    bool fused = true;             // forward, gate and training on the fused kernels where they apply
     int64_t zcap = 0;              // rows the logits buffer z holds
     bool fused_attr = false;
     int64_t step = 0;
@@ -1128,10 +1128,11 @@ int64_t param_count(int kin, int hid, int nout, int64_t off[8]) {
 }
 
 bool fused_ok(const tqec_mlp *p) { return p->hid == kFusedHid && p->nout <= 32 && p->kin <= kFusedHid; }
+bool use_fused(const tqec_mlp *p) { return p->fused && fused_ok(p); }
 
 // Partial sums of the loss that a training pass over B rows leaves.
 int64_t loss_blocks(const tqec_mlp *p, int64_t B) {
-    return fused_ok(p) ? B / kTrainRows : (B + 255) / 256;
+    return use_fused(p) ? B / kTrainRows : (B + 255) / 256;
 }
 
 int ensure_cap(tqec_mlp *p, int64_t B) {
@@ -1149,7 +1150,7 @@ int ensure_cap(tqec_mlp *p, int64_t B) {
     TQM_HIP(hipMalloc((void **)&p->z, (size_t)B * p->nout * sizeof(float)));
     p->zcap = B;
     TQM_HIP(hipMalloc((void **)&p->dz, (size_t)B * p->nout * sizeof(float)));
-    const int64_t nb = loss_blocks(p, B);
+    const int64_t nb = (B + kTrainRows - 1) / kTrainRows;   // enough for either kind of pass
     if (p->loss_cap < nb) {
         if (p->loss_parts) (void)hipFree(p->loss_parts);
         TQM_HIP(hipMalloc((void **)&p->loss_parts, (size_t)nb * sizeof(float)));
@@ -1227,7 +1228,7 @@ int forward_fused(tqec_mlp *p, const uint8_t *d_syn, int64_t B, hipStream_t st) 
 
 int forward(tqec_mlp *p, const uint8_t *d_syn, int64_t B, hipStream_t st, bool keep = true) {
     int rc;
-    if (!keep && p->fused && fused_ok(p)) return forward_fused(p, d_syn, B, st);
+    if (!keep && use_fused(p)) return forward_fused(p, d_syn, B, st);
     if ((rc = ensure_cap(p, B))) return rc;
     const int64_t nx = B * p->kin;
     hipLaunchKernelGGL(embed_kernel, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, st, d_syn, B, p->n_in, p->kin,
@@ -1427,8 +1428,8 @@ int backward(tqec_mlp *p, const float *d_q, int64_t B, float *grad, hipStream_t 
     return weight_gradients(p, dc, B, (int)tiles, grad, st);
 }
 
-// Training reduces over the batch inside the weight-gradient GEMM, whose K
-// loop needs a multiple of 32 rows; inference takes any batch size.
+// Training takes tiles of 32 rows (mlp_train_rows_kernel has no ragged one, and
+// the layer-by-layer pass keeps its rule); inference takes any batch size.
 int check_batch(tqec_mlp *p, int64_t B, bool training) {
     if (!p) return fail(TQEC_ENULL, "null network");
     if (B <= 0 || B > (int64_t(1) << 30)) return fail(TQEC_EINVAL, "batch size out of range");
@@ -1516,7 +1517,7 @@ int tqec_mlp_gradients(tqec_mlp *p, const uint8_t *d_syn, const float *d_targets
     if (!d_syn || !d_targets) return fail(TQEC_ENULL, "null device pointer");
     hipStream_t st = (hipStream_t)stream;
     float *grad = d_grad ? d_grad : p->g;
-    if (fused_ok(p)) {
+    if (use_fused(p)) {
         if ((rc = train_fused(p, d_syn, d_targets, B, grad, st))) return rc;
     } else {
         if ((rc = forward(p, d_syn, B, st))) return rc;
@@ -1587,7 +1588,7 @@ int tqec_mlp_set_inference(tqec_mlp *p, int32_t kernel) {
 
 int tqec_mlp_inference(const tqec_mlp *p, int32_t *kernel) {
     if (!p || !kernel) return fail(TQEC_ENULL, "null argument");
-    *kernel = (p->fused && fused_ok(p)) ? 1 : 0;
+    *kernel = use_fused(p) ? 1 : 0;
     return TQEC_OK;
 }
 

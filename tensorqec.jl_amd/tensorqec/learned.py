@@ -106,8 +106,8 @@ class HipMLP:
                                        _vp(d_reject), _vp(d_count), _vp(stream)))
 
     def set_inference(self, kernel: int) -> None:
-        """Kernel of forward / gate: 1 fused (default where it applies), 0 the
-        layer-by-layer training kernels."""
+        """Kernels of forward, gate and training: 1 fused (default where they
+        apply), 0 layer by layer."""
         L.check(L.load().tqec_mlp_set_inference(self._h, int(kernel)))
 
     def inference(self) -> int:

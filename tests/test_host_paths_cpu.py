@@ -15,6 +15,7 @@ PLAN = """
 import sys
 sys.path[:0] = [%r, %r]
 import numpy as np
+from tensorqec.learned import HipMLP
 from tensorqec import decoders as D, lib as L
 from tensorqec.codes import CSSTannerGraph, SurfaceCode
 from tensorqec.errors import iid_error
@@ -73,3 +74,21 @@ hip.set_spec(1, 256, False, mfma32=True)
 print("mfma" in first, "mfma" in L.mixed_spec_source([ct.hip, hip], 256))
 """)
     assert out.split() == ["True", "False", "True", "False", "True"]
+
+
+@pytest.mark.parametrize("inference", [0, 1])
+def test_training_runs_the_chosen_kernels(stub, inference):
+    """Gradients and training steps run layer by layer where inference does."""
+    _, calls = run(stub, """
+S, Q, g = np.zeros((64, 8), np.uint8), np.full((64, 4), 0.25, np.float32), np.zeros(600000, np.float32)
+m = HipMLP(8, 4, hidden=512, seed=1)
+for k in (1 - %d, %d):
+    m.set_inference(k)
+    print("stub now", k, file=sys.stderr, flush=True)
+    m.gradients(S.ctypes.data, Q.ctypes.data, 64, g.ctypes.data)
+    m.train_step(S.ctypes.data, Q.ctypes.data, 64, 1e-3)
+""" % (inference, inference))
+    kernels = " ".join(c for c in calls[calls.index("now %d" % inference):] if c.startswith("kernel "))
+    assert kernels.count("mlp_train_rows_kernel") == (2 if inference else 0)
+    assert kernels.count("gemm_fwd_kernel") == (0 if inference else 6)
+    assert kernels.count("mlp_dw_kernel") == 2
