@@ -1561,6 +1561,27 @@ SpecKernel *spec_find(tqec_plan *p, int dev, const SpecCfg &cfg) {
 // minutes; such plans stay on the generic executors).
 constexpr size_t kMaxSpecSource = size_t(2) << 20;
 
+// Compile and load the kernel of a configuration: its module, function and the
+// workgroups per CU that its registers and LDS allow (0: not known).
+int spec_load(tqec_plan *p, const SpecCfg &cfg, SpecKernel &k, int &per_cu) {
+    const std::string src = spec_source(p->cp, cfg);
+    if (src.empty()) return set_error(TQEC_EUNSUPPORTED, "plan does not suit this specialised kernel");
+    if (src.size() > kMaxSpecSource)
+        return set_error(TQEC_EUNSUPPORTED, "specialised kernel source of " + std::to_string(src.size() >> 10) +
+                                                " KB is beyond the compile budget; use the generic executors");
+    std::vector<char> code;
+    int rc;
+    if ((rc = spec_code(src, code))) return rc;
+    TQ_HIP(hipModuleLoadData(&k.mod, code.data()));
+    const hipError_t e = hipModuleGetFunction(&k.fn, k.mod, spec_kernel_name(cfg));
+    if (e != hipSuccess) {
+        (void)hipModuleUnload(k.mod);
+        return set_error(TQEC_EDEVICE, std::string("hipModuleGetFunction: ") + hipGetErrorString(e));
+    }
+    if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k.fn, cfg.threads, 0) != hipSuccess) per_cu = 0;
+    return TQEC_OK;
+}
+
 int spec_get(tqec_plan *p, int dev, const SpecCfg &cfg, SpecKernel **out) {
     const auto key = spec_key(dev, cfg);
     auto it = p->spec.find(key);
@@ -1569,32 +1590,31 @@ int spec_get(tqec_plan *p, int dev, const SpecCfg &cfg, SpecKernel **out) {
         return TQEC_OK;
     }
     if (cfg.glog < 0 || !spec_fits(p, cfg)) return set_error(TQEC_EUNSUPPORTED, "specialised tile does not fit in LDS");
-    std::vector<char> code;
     int rc;
-    const std::string src = spec_source(p->cp, cfg);
-    if (src.empty()) return set_error(TQEC_EUNSUPPORTED, "plan does not suit this specialised kernel");
-    if (src.size() > kMaxSpecSource)
-        return set_error(TQEC_EUNSUPPORTED, "specialised kernel source of " + std::to_string(src.size() >> 10) +
-                                                " KB is beyond the compile budget; use the generic executors");
-    if ((rc = spec_code(src, code))) return rc;
     SpecKernel k;
     k.cfg = cfg;
     k.lds = spec_lds_bytes(p->cp, cfg);
     k.inline_recheck = spec_reg_inline_recheck(p->cp, cfg);
-    TQ_HIP(hipModuleLoadData(&k.mod, code.data()));
-    const hipError_t e = hipModuleGetFunction(&k.fn, k.mod, spec_kernel_name(cfg));
-    if (e != hipSuccess) {
-        (void)hipModuleUnload(k.mod);
-        return set_error(TQEC_EDEVICE, std::string("hipModuleGetFunction: ") + hipGetErrorString(e));
+    int per_cu = 0;
+    if ((rc = spec_load(p, cfg, k, per_cu))) return rc;
+    if (cfg.reg && cfg.waves > 1 && per_cu > 0 && per_cu * cfg.threads < cfg.waves * 256) {
+        // Held to `waves` per SIMD the compiler still went past their share of
+        // the registers (values moved to AGPRs and to scratch come on top of
+        // an aligned VGPR count), and the cap only costs: take the kernel
+        // without it where as many workgroups run.  d=7 plans, 65,536 rows,
+        // with the cap -> without: 260 -> 231 registers and a second wave,
+        // 77.9 -> 53.4 us; 274 -> 278, no scratch, 77.2 -> 73.8 us.
+        SpecCfg open = cfg;
+        open.waves = 0;
+        SpecKernel o = k;
+        int opc = 0;
+        if (spec_load(p, open, o, opc) == TQEC_OK) {
+            if (opc >= per_cu) std::swap(k, o), std::swap(per_cu, opc);
+            (void)hipModuleUnload(o.mod);
+        }
     }
-    k.blocks = p->n_cu * resident_per_cu(k.lds, cfg.threads, p->lds_limit);
-    if (cfg.reg || cfg.slab) {
-        // register-bound: the runtime's occupancy of the compiled kernel
-        int per_cu = 0;
-        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k.fn, cfg.threads, 0) == hipSuccess &&
-            per_cu > 0)
-            k.blocks = p->n_cu * per_cu;
-    }
+    // register-bound kernels: the runtime's occupancy of the compiled code
+    k.blocks = p->n_cu * ((cfg.reg || cfg.slab) && per_cu > 0 ? per_cu : resident_per_cu(k.lds, cfg.threads, p->lds_limit));
     if (cfg.slab) {
         // the kernel loops over tiles in as many workgroups as run: fewer of
         // them when their slabs would not fit the budget (plans of width 2^23:

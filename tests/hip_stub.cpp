@@ -55,6 +55,28 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream
     fprintf(stderr, "stub kernel %s\n", kernels()[f].c_str());
     return call("launch");
 }
+// modules are numbered from 1; TQEC_STUB_OCC: the workgroups per CU of each, a digit apiece
+hipError_t hipModuleLoadData(hipModule_t *m, const void *) {
+    static size_t n = 0;
+    *m = (hipModule_t)++n;
+    return call("load");
+}
+hipError_t hipModuleUnload(hipModule_t) { return call("unload"); }
+hipError_t hipModuleGetFunction(hipFunction_t *f, hipModule_t m, const char *) {
+    *f = (hipFunction_t)m;
+    return hipSuccess;
+}
+hipError_t hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(int *n, hipFunction_t f, int, size_t) {
+    const char *occ = getenv("TQEC_STUB_OCC");
+    const size_t i = (size_t)f - 1;
+    *n = occ && i < strlen(occ) ? occ[i] - '0' : 2;
+    return hipSuccess;
+}
+hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned, unsigned, unsigned, unsigned, unsigned, unsigned, unsigned,
+                                 hipStream_t, void **, void **) {
+    fprintf(stderr, "stub module %zu\n", (size_t)f);
+    return call("launch");
+}
 hipError_t hipGetLastError() {
     const hipError_t e = g_last;
     g_last = hipSuccess;

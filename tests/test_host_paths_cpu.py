@@ -92,3 +92,17 @@ for k in (1 - %d, %d):
     assert kernels.count("mlp_train_rows_kernel") == (2 if inference else 0)
     assert kernels.count("gemm_fwd_kernel") == (0 if inference else 6)
     assert kernels.count("mlp_dw_kernel") == 2
+
+
+@pytest.mark.parametrize("occ,module,loads", [("2", 1, 1), ("12", 2, 2), ("11", 2, 2)])
+def test_register_kernel_without_a_cap_that_the_compiler_missed(stub, occ, module, loads):
+    """Held to two waves per SIMD (256 threads: two workgroups per CU): a build
+    that does not reach them gives way to one without the cap."""
+    _, calls = run(stub, """
+cfg = ct.hip.spec_config()
+assert cfg["reg"] and cfg["waves"] == 2 and cfg["threads"] == 256
+D.decode_batch(ct, np.zeros((3, 8), np.uint8), mode="spec_f32")
+assert ct.hip.spec_config() == cfg
+""", TQEC_STUB_OCC=occ)
+    assert calls.count("load") == loads and calls.count("unload") >= loads - 1
+    assert [c for c in calls if c.startswith("module ")] == ["module %d" % module]
