@@ -73,13 +73,17 @@ size_t split_k_entries(const CompiledPlan &cp, const SpecCfg &cfg) {
 // A slab plan's steps are bound by memory traffic, and the widest few tensors
 // make the slab necessary while most of the traffic is in smaller ones, so as
 // many intermediates as fit live in LDS instead, each from the step that makes
-// it to the step that reads it.  The LDS of a CU is divided among the eight
-// waves (two per SIMD) that a slab kernel's registers allow.  Measured with
-// 256 threads (76 KB): circuit-level d=5, 2 rounds 2.79 -> 2.22 ms per 4,096
-// (it ran at 4.7 TB/s of HBM traffic, 34% of it in tensors of at most 2^13
-// entries), toric L=3 772 -> 594 us per 8,192; toric L=5, whose traffic is in
-// its 2^21-entry tensors, is unchanged.  Fewer workgroups with smaller slabs
-// in all (171 MB, less than the memory-side cache) changed nothing.
+// it to the step that reads it.  The LDS of a CU is divided among as many waves
+// per SIMD as the configuration asks for, two at least (what a slab kernel's
+// registers allow when it is held to none).  Measured with 256 threads and two
+// (76 KB): circuit-level d=5, 2 rounds 2.79 -> 2.22 ms per 4,096 (it ran at 4.7
+// TB/s of HBM traffic, 34% of it in tensors of at most 2^13 entries), toric L=3
+// 772 -> 594 us per 8,192; toric L=5, whose traffic is in its 2^21-entry
+// tensors, is unchanged.  With BF16 steps the d=5 plan takes 26.3 ms per 16,384
+// instead of 33.5 at two waves; at four, with the LDS divided by two, its tuned
+// configuration took 37.3, divided by four 31.0, without placement 33.8.  Fewer
+// workgroups with smaller slabs in all (171 MB, less than the memory-side
+// cache) changed nothing.
 struct Places {
     std::vector<int64_t> lds;                // per step: output's LDS entry offset (per syndrome), -1 in the slab
     std::vector<std::array<int, 2>> prod;    // per step: steps that made its operands, -1 for tables
@@ -106,7 +110,8 @@ Places slab_places(const CompiledPlan &cp, const SpecCfg &cfg) {
                 }
         }
     if (!cfg.slab || cfg.fp64) return P;
-    const int64_t room = (int64_t)(kSlabLds * std::min(cfg.threads, 512) / 512 / 4) >> cfg.glog;
+    const int per_cu = 256 * std::max(2, cfg.waves);   // threads of a CU
+    const int64_t room = (int64_t)(kSlabLds * std::min(cfg.threads, per_cu) / per_cu / 4) >> cfg.glog;
     std::vector<int> order(ns);
     for (int s = 0; s < ns; ++s) order[s] = s;
     int64_t best = 0;

@@ -44,6 +44,15 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hip
 }
 hipError_t hipMemset(void *d, int v, size_t n) { memset(d, v, n); return hipSuccess; }
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t *e) { *e = nullptr; return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {   // everything later is slower
+    static float t = 0;
+    *ms = t += 1;
+    return hipSuccess;
+}
 hipError_t hipStreamSynchronize(hipStream_t) { return call("wait"); }
 hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
 hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
@@ -56,9 +65,16 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream
     return call("launch");
 }
 // modules are numbered from 1; TQEC_STUB_OCC: the workgroups per CU of each, a digit apiece
-hipError_t hipModuleLoadData(hipModule_t *m, const void *) {
+hipError_t hipModuleLoadData(hipModule_t *m, const void *image) {
     static size_t n = 0;
     *m = (hipModule_t)++n;
+    // the kernel's LDS, from its metadata (a big-endian 16- or 32-bit number follows the key)
+    const char key[] = ".group_segment_fixed_size";
+    const unsigned char *p = (const unsigned char *)image;
+    while (memcmp(p, key, sizeof key - 1)) ++p;
+    p += sizeof key - 1;
+    const unsigned lds = *p == 0xcd ? p[1] << 8 | p[2] : *p == 0xce ? p[1] << 24 | p[2] << 16 | p[3] << 8 | p[4] : *p;
+    fprintf(stderr, "stub lds %u\n", lds);
     return call("load");
 }
 hipError_t hipModuleUnload(hipModule_t) { return call("unload"); }

@@ -106,3 +106,19 @@ assert ct.hip.spec_config() == cfg
 """, TQEC_STUB_OCC=occ)
     assert calls.count("load") == loads and calls.count("unload") >= loads - 1
     assert [c for c in calls if c.startswith("module ")] == ["module %d" % module]
+
+
+def test_slab_intermediates_leave_lds_for_the_waves_asked_for(stub):
+    """The LDS of a CU divided by the workgroups that `waves` waves per SIMD
+    make, two at least."""
+    _, calls = run(stub, """
+from tensorqec.codes import ToricCode
+t = CSSTannerGraph.from_code(ToricCode(4, 4))
+hip = D.compile(D.TNMMAP(optimizer=D.TreeSA(ntrials=1, sweeps=50, restarts=1)), t, iid_error(0.02, 0.02, 0.02, t.nq)).hip
+for waves in (2, 3, 4):
+    hip.set_spec(1, 256, False, waves, slab=True, unroll=1)
+    hip.decode(np.zeros((1, t.ns), np.uint8), "spec_f32")
+""")
+    lds = [int(c.split()[1]) for c in calls if c.startswith("lds ")]
+    lds = [lds[0]] + lds[2:]                               # the second is the FP64 re-check's
+    assert 53 * 1024 < lds[0] <= 80 * 1024 and 16 * 1024 < lds[1] <= 53 * 1024 and 16 * 1024 < lds[2] <= 40 * 1024
