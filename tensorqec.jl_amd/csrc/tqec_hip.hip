@@ -1544,6 +1544,19 @@ SpecCfg choose_spec(const tqec_plan *p, bool fp64 = false) {
     return c;
 }
 
+// What SPEC_F32 and SPEC_BF16 run until a configuration is pinned or tuned.
+SpecCfg default_spec(const tqec_plan *p, bool bf16) {
+    SpecCfg cfg = choose_spec(p);
+    if (bf16 && cfg.glog >= 0) {
+        // MFMA steps need tiles of one syndrome; BF16 steps replace the FP32 ones
+        cfg.glog = 0;
+        cfg.threads = 256;
+        cfg.mfma = true;
+        cfg.mfma32 = false;
+    }
+    return cfg;
+}
+
 std::tuple<int, int, int, int, int, int, int> spec_key(int dev, const SpecCfg &cfg) {
     return std::make_tuple(dev, cfg.glog, cfg.threads, cfg.tab_lds ? 1 : 0, cfg.waves, cfg.fp64 ? 1 : 0,
                            (cfg.slab ? 1 : 0) | (cfg.mfma ? 2 : 0) | (cfg.reg ? 4 : 0) | (cfg.unroll << 3) |
@@ -1743,14 +1756,7 @@ int run_spec(tqec_plan *p, DeviceData *dd, Workspace &w, const uint8_t *d_syn, i
     SpecCfg &cfg = bf16 ? p->specb_cfg : p->spec_cfg;
     bool &cfg_set = bf16 ? p->specb_cfg_set : p->spec_cfg_set;
     if (!cfg_set) {
-        cfg = choose_spec(p);
-        if (bf16 && cfg.glog >= 0) {
-            // MFMA steps need tiles of one syndrome; BF16 steps replace the FP32 ones
-            cfg.glog = 0;
-            cfg.threads = 256;
-            cfg.mfma = true;
-            cfg.mfma32 = false;
-        }
+        cfg = default_spec(p, bf16);
         cfg_set = true;
     }
     if (cfg.glog < 0)
@@ -1829,9 +1835,9 @@ void spec_precompile(const tqec_plan *p, const std::vector<SpecCfg> &cands) {
     for (auto &j : jobs) j.get();
 }
 
-// Autotuner of the specialised kernel, in two stages: (tile 1..64, 64/128/256
-// threads) and the register-resident kernel at 64/128/256 threads, all with
-// tables in global memory; then, for an LDS tile, the best pair with tables
+// Autotuner of the specialised kernel, in two stages: the untuned default,
+// (tile 1..64, 64/128/256 threads) and the register-resident kernel at
+// 64/128/256 threads, all with tables in global memory; then, for an LDS tile, the best pair with tables
 // in LDS, a 4-waves-per-SIMD register cap and 1/2/4/8 outputs per lane block,
 // or, for the register-resident kernel, tables in LDS (when they fit) and a
 // 2-waves-per-SIMD register cap.  Each configuration is timed
@@ -1885,6 +1891,7 @@ int autotune_spec(tqec_plan *p, const uint8_t *d_syn, int64_t n, hipStream_t st,
         }
     };
     std::vector<SpecCfg> stage1;
+    const SpecCfg untuned = default_spec(p, bf16);
     for (int gl = 0; gl <= (bf16 ? 0 : 6); ++gl)
         for (int thr : {64, 128, 256}) {
             if (thr < (1 << gl)) continue;
@@ -1919,6 +1926,11 @@ int autotune_spec(tqec_plan *p, const uint8_t *d_syn, int64_t n, hipStream_t st,
             }
     }
     if (stage1.empty()) rc = set_error(TQEC_EUNSUPPORTED, "no specialised tile fits");
+    if (!rc && untuned.glog >= 0 && spec_fits(p, untuned)) {
+        // first, so that tuning never ends with a slower kernel than without
+        time_all({untuned});
+        rc = TQEC_OK;   // one that does not build is no candidate
+    }
     if (!rc) time_all(stage1);
     if (!rc && best.glog >= 0) {
         std::vector<SpecCfg> stage2;

@@ -108,6 +108,14 @@ assert ct.hip.spec_config() == cfg
     assert [c for c in calls if c.startswith("module ")] == ["module %d" % module]
 
 
+def test_tuning_keeps_a_default_that_nothing_beats(stub):
+    run(stub, """
+cfg, S = ct.hip.spec_config(), np.zeros((64, 8), np.uint8)
+ct.hip.autotune("spec_f32", S.ctypes.data, 64)
+assert ct.hip.spec_config() == cfg and cfg["reg"]
+""")
+
+
 def test_slab_intermediates_leave_lds_for_the_waves_asked_for(stub):
     """The LDS of a CU divided by the workgroups that `waves` waves per SIMD
     make, two at least."""
