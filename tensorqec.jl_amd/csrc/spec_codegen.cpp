@@ -1981,6 +1981,16 @@ bool spec_plan_uses_mfma32(const CompiledPlan &cp, const SpecCfg &cfg) {
     return false;
 }
 
+double spec_mfma32_share(const CompiledPlan &cp, const SpecCfg &cfg) {
+    double all = 0, gemm = 0;
+    for (const StepDesc &st : cp.steps) {
+        const double macs = std::ldexp(1.0, st.rc + st.nk);
+        all += macs;
+        if (spec_step_uses_mfma32(st, cfg)) gemm += macs;
+    }
+    return all > 0 ? gemm / all : 0;
+}
+
 bool spec_step_uses_mfma(const StepDesc &st, const SpecCfg &cfg) {
     if (!cfg.mfma || cfg.fp64 || cfg.glog != 0 || cfg.threads % 64 != 0) return false;
     if (st.nk < 4) return false;

@@ -75,6 +75,8 @@ bool spec_step_uses_mfma(const StepDesc &st, const SpecCfg &cfg);
 // their FP32 values; only the summation order differs from the scalar steps.
 bool spec_step_uses_mfma32(const StepDesc &st, const SpecCfg &cfg);
 bool spec_plan_uses_mfma32(const CompiledPlan &cp, const SpecCfg &cfg);
+// Their share of the plan's multiply-adds.
+double spec_mfma32_share(const CompiledPlan &cp, const SpecCfg &cfg);
 
 // Static LDS bytes of the specialised kernel for this configuration.
 size_t spec_lds_bytes(const CompiledPlan &cp, const SpecCfg &cfg);

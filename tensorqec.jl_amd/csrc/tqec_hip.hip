@@ -1460,22 +1460,26 @@ bool spec_fits(const tqec_plan *p, const SpecCfg &c) {
 
 // Default before tuning: the register-resident FP32 kernel when the plan's
 // live tensors fit a quad's registers (256 threads, tables in global memory,
-// two waves per SIMD when the live set leaves room); else, for FP32 plans with
-// GEMM-shaped steps, one syndrome per workgroup with those steps on FP32 MFMA,
-// in LDS or from a slab (choose_gemm); else the largest tile whose LDS
+// two waves per SIMD when the live set leaves room); else, for FP32 plans whose
+// GEMM-shaped steps weigh enough, one syndrome per workgroup with those steps
+// on FP32 MFMA, in LDS or from a slab (choose_gemm); else the largest tile whose LDS
 // image (tables included when they fit) lets three workgroups share a CU
 // (else two, else one), 16 threads per syndrome within [64, 128], blocks of
 // 4 outputs per lane; else per-workgroup slabs, 256 threads, blocks of 4.
 //
-// One syndrome per workgroup is what MFMA steps need, and it beats larger
-// tiles on every plan with such steps that was measured: circuit-level d=3
-// with 3 rounds (24 KB of LDS) 330 us per 16,384 syndromes instead of 834 in
-// tiles of 2, d=9 (37 KB) 1.18 instead of 1.33 ms, toric L=3 (slab) 594 us per
-// 8,192 instead of 2,080 in tiles of 16, circuit-level d=5 with 2 rounds
-// (slab) 2.2 ms per 4,096 instead of 11.1 in tiles of 4.  Two waves per SIMD
-// (at most 256 registers) let one wave's MFMAs cover the other's loads; an LDS
-// plan takes as many threads as bring its workgroups per CU to four or more
-// waves (64 threads were faster than 128 or 256 at four and six workgroups).
+// One syndrome per workgroup is what MFMA steps need.  It beats larger tiles
+// where those steps hold a good part of the multiply-adds: circuit-level d=3
+// with 3 rounds (24 KB of LDS, 87% of them) 330 us per 16,384 syndromes instead
+// of 834 in tiles of 2; three d=9 plans (37 to 43 KB; 43, 37 and 30%) 4.4, 5.2
+// and 4.2 ms per 65,536 instead of 5.1, 6.9 and 4.6; toric L=3 (slab) 594 us
+// per 8,192 instead of 2,080 in tiles of 16; circuit-level d=5 with 2 rounds
+// (slab) 2.2 ms per 4,096 instead of 11.1 in tiles of 4.  A d=8 plan with 16%
+// (13 KB) runs 65,536 in 2.07 ms in tiles of 4 and 2.20 so (4,096, which leave
+// tiles of 4 half of the chip, in 192 and 140 us); hence the line at a quarter,
+// for plans that fit LDS.  Two waves per SIMD (at most 256 registers) let one
+// wave's MFMAs cover the other's loads; an LDS plan takes as many threads as
+// bring its workgroups per CU to four or more waves (64 threads were faster
+// than 128 or 256 at four and six workgroups).
 bool choose_gemm(const tqec_plan *p, SpecCfg &out) {
     SpecCfg c;
     c.glog = 0;
@@ -1486,6 +1490,7 @@ bool choose_gemm(const tqec_plan *p, SpecCfg &out) {
     c.waves = 2;
     if (!spec_plan_uses_mfma32(p->cp, c)) return false;
     const size_t lds = spec_lds_bytes(p->cp, c);
+    if (lds <= p->lds_limit && spec_mfma32_share(p->cp, c) < 0.25) return false;
     if (lds <= p->lds_limit) {
         const size_t per_cu = p->lds_limit / std::max<size_t>(lds, 1);
         c.threads = per_cu >= 4 ? 64 : per_cu >= 2 ? 128 : 256;

@@ -130,3 +130,22 @@ for waves in (2, 3, 4):
     lds = [int(c.split()[1]) for c in calls if c.startswith("lds ")]
     lds = [lds[0]] + lds[2:]                               # the second is the FP64 re-check's
     assert 53 * 1024 < lds[0] <= 80 * 1024 and 16 * 1024 < lds[1] <= 53 * 1024 and 16 * 1024 < lds[2] <= 40 * 1024
+
+
+@pytest.mark.parametrize("k,mfma", [(1, False), (4, True)])
+def test_default_tile_by_the_share_of_gemm_steps(stub, k, mfma):
+    """A 32 x 32 product over k labels beside one of 2^13 entries without a
+    contraction, too wide for registers: one-syndrome MFMA tiles only where the
+    product is a quarter of the multiply-adds."""
+    out, _ = run(stub, """
+from tensorqec.planner import Plan
+rng = np.random.default_rng(1)
+a, b, k, x, o = range(10, 15), range(20, 25), range(30, 30 + %d), range(40, 53), [70]
+leaves = [[0, *a, *k], [1, *k, *b], [2, *x], [3, *x], [0, *a[:2], *b[:2], *o], [1, *x[:3], *o]]
+outs = [[*a, *b], [*x], [*o], [*o], [*o]]
+p = Plan(6, leaves, [rng.uniform(0.1, 1, 1 << len(l)) for l in leaves], [-1] * 6, [0, 2, 6, 7, 8], [1, 3, 4, 5, 9],
+         outs, [*o], 4, {i: i for i in range(4)})
+cfg = L.HipPlan(p, tabulate_bits=0).spec_config()
+print(cfg["reg"], cfg["mfma32"])
+""" % k)
+    assert out.split() == ["False", str(mfma)]
