@@ -1489,8 +1489,12 @@ bool choose_gemm(const tqec_plan *p, SpecCfg &out) {
     c.mfma32 = true;
     c.waves = 2;
     if (!spec_plan_uses_mfma32(p->cp, c)) return false;
+    SpecCfg plain = c;   // the same tile without the split contractions' partial sums
+    plain.mfma32 = false;
     const size_t lds = spec_lds_bytes(p->cp, c);
     if (lds <= p->lds_limit && spec_mfma32_share(p->cp, c) < 0.25) return false;
+    // a plan that fits LDS stays there: calls without allocation take no slab
+    if (lds > p->lds_limit && spec_lds_bytes(p->cp, plain) <= p->lds_limit) return false;
     if (lds <= p->lds_limit) {
         const size_t per_cu = p->lds_limit / std::max<size_t>(lds, 1);
         c.threads = per_cu >= 4 ? 64 : per_cu >= 2 ? 128 : 256;

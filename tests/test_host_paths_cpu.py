@@ -149,3 +149,42 @@ cfg = L.HipPlan(p, tabulate_bits=0).spec_config()
 print(cfg["reg"], cfg["mfma32"])
 """ % k)
     assert out.split() == ["False", str(mfma)]
+
+
+def test_partial_sums_push_no_plan_out_of_lds(stub):
+    """A plan whose one-syndrome tile fills the LDS to the last 64 bytes, so
+    that the partial sums of a split contraction have no room: it keeps an LDS
+    tile, which calls without allocation and captured ones can take."""
+    out, _ = run(stub, """
+from tensorqec.planner import Plan
+rng, lab, T = np.random.default_rng(1), 100, []
+# pairs of tensors with `sh` labels in common, all made before the first pair is joined
+for ra, rb, sh in ((15, 9, 9), (12, 11, 11), (10, 8, 8), (7, 4, 4)):
+    a = list(range(lab, lab + ra))
+    T += [a, a[:sh]]
+    lab += ra
+leaves, outs = [], [list(x) for x in T]
+for i, x in enumerate(T):
+    k, h = [lab, lab + 1], len(x) // 2
+    lab += 2
+    leaves += [[2 * i, *x[:h], *k], [2 * i + 1, *k, *x[h:]]]
+n = len(leaves)
+lhs, rhs = list(range(0, n, 2)), list(range(1, n, 2))
+cur = []
+for i in range(0, 8, 2):
+    lhs, rhs = lhs + [n + i], rhs + [n + i + 1]
+    outs.append([l for l in T[i] if l not in T[i + 1]])
+    cur.append((n + 8 + i // 2, outs[-1]))
+while len(cur) > 1:
+    (x, a), (y, b) = cur[:2]
+    lhs, rhs = lhs + [x], rhs + [y]
+    outs.append(a + b)
+    cur = [(n + len(outs) - 1, a + b)] + cur[2:]
+p = Plan(n, leaves, [rng.uniform(0.1, 1, 1 << len(l)) for l in leaves], [-1] * n, lhs, rhs, outs, outs[-1], 16,
+         {i: i for i in range(16)})
+hip = L.HipPlan(p, tabulate_bits=0)
+size = [hip.spec_source(1, 64, False, unroll=4, mfma32=m).split("smem[")[1].split("]")[0] for m in (False, True)]
+assert int(size[0]) <= 160 * 1024 < int(size[1]), size
+print(hip.spec_config()["slab"])
+""")
+    assert out.strip() == "False"
