@@ -2408,6 +2408,8 @@ std::string spec_map_wave_source(const CompiledPlan &cp, int glog, int waves) {
     return o.str();
 }
 
+constexpr size_t kCuLds = 160 * 1024;   // of a CU
+
 size_t spec_mixed_lds_bytes(const std::vector<MixedSpecPlan> &plans) {
     size_t m = 16;
     for (const MixedSpecPlan &q : plans) {
@@ -2434,12 +2436,20 @@ std::string spec_mixed_source(const std::vector<MixedSpecPlan> &plans, int threa
         emit_tile_fn(o, *plans[i].cp, plans[i].f32, "p" + std::to_string(i) + "_f32", true);
         emit_tile_fn(o, *plans[i].cp, plans[i].f64, "p" + std::to_string(i) + "_f64", true);
     }
-    // Three workgroups of 256 threads per CU: many tiles run 1.6 times as fast
-    // as with one, which is what the compiler's own choice of registers allows
-    // once it has moved every plan's address arithmetic out of the tile loop
-    // (the tile functions hide their thread id to keep it inside; else 300
-    // registers spill).
-    o << "extern \"C\" __global__ void __launch_bounds__(" << threads << ", " << (threads == 256 ? 3 : 1)
+    // As many workgroups of 256 threads per CU as their LDS allows, three at
+    // most.  Left to itself the compiler takes registers for one, once it has
+    // moved every plan's address arithmetic out of the tile loop (the tile
+    // functions hide their thread id to keep it inside).  Held to three it
+    // spills where a plan runs from a slab on MFMA (24 registers, 100 B per
+    // lane; none in mixes of LDS plans), which still pays: 48 batches, 22,185
+    // rows of five codes, a third of them toric L=3, 557 us; held to two 720,
+    // to one 916 (24 batches, 6,783 rows with 76 of toric L=3: 59, 62 and 58).
+    // A d=7 plan's tiles leave room for two (67 KB): 24 batches of 3,000 rows
+    // of six codes 1,158 us, and 1,863 held to three, which the compiler takes
+    // for no bound at all.
+    const size_t lds = spec_mixed_lds_bytes(plans) + kMixedStaticLds;
+    const size_t wgs = threads == 256 ? std::max<size_t>(1, std::min<size_t>(3, kCuLds / lds)) : 1;
+    o << "extern \"C\" __global__ void __launch_bounds__(" << threads << ", " << wgs
       << ") tqec_mixed_spec(\n"
          "    const MBatch *__restrict__ batches, const MHeader *__restrict__ hdr, MCounters *ctr,\n"
          "    unsigned long long *t_done, const float *const *tabs32, const double *const *tabs64, float *slab32,\n"

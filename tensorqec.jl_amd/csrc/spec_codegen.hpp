@@ -114,6 +114,7 @@ struct MixedSpecPlan {
 // slabs hold slab32_entries / slab64_entries per workgroup; `cus` workgroups
 // alone take up to twice as many tiles.
 size_t spec_mixed_lds_bytes(const std::vector<MixedSpecPlan> &plans);
+constexpr size_t kMixedStaticLds = 8 + 4 + 256;   // its other variables
 std::string spec_mixed_source(const std::vector<MixedSpecPlan> &plans, int threads, size_t slab32_entries,
                               size_t slab64_entries, int cus);
 // Max-product (TNMAP) plan: kernel `tqec_map_spec(const unsigned char *syn,

@@ -3372,7 +3372,7 @@ int tqec_mixed_set_kernel(tqec_mixed *m, int32_t kind) {
     std::vector<int> glog, slabf;
     size_t s32 = 0, s64 = 0;
     if ((rc = mixed_spec_layout(m->plans, nt, lds_limit, sp, glog, slabf, s32, s64))) return rc;
-    const size_t lds = spec_mixed_lds_bytes(sp) + 8 + 4 + 256;
+    const size_t lds = spec_mixed_lds_bytes(sp) + kMixedStaticLds;
     if (lds > lds_limit) return set_error(TQEC_EUNSUPPORTED, "the plans' tiles exceed the LDS");
     std::vector<char> code;
     if ((rc = spec_code(spec_mixed_source(sp, nt, std::max<size_t>(s32, 1), std::max<size_t>(s64, 1), n_cu), code))) return rc;

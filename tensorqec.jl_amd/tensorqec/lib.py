@@ -610,8 +610,9 @@ class HipMixed:
         return us[:self.n_last], rc.value
 
 
-def mixed_spec_source(plans, threads: int = 128) -> str:
-    """Source of the mixed-code kernel generated for these HipPlans."""
+def mixed_spec_source(plans, threads: int = 256) -> str:
+    """Source of the mixed-code kernel generated for these HipPlans (256
+    threads: the one that the executor runs)."""
     arr = (ctypes.c_void_p * len(plans))(*[p.handle.value for p in plans])
     n = ctypes.c_size_t()
     check(load().tqec_mixed_spec_source(arr, len(plans), int(threads), None, 0, ctypes.byref(n)))

@@ -7,7 +7,8 @@ import subprocess
 import pytest
 
 from tensorqec import decoders as D
-from tensorqec.codes import CSSTannerGraph, SurfaceCode
+from tensorqec import lib as L
+from tensorqec.codes import CSSTannerGraph, SteaneCode, SurfaceCode, ToricCode
 from tensorqec.errors import iid_error
 
 REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -58,3 +59,24 @@ def test_layered_forward_waits_for_no_store_before_its_last(tmp_path):
     for _, body in bodies:
         stores = body[body.index("global_store_short"):]
         assert stores.count("global_store_short") == 64 and "vmcnt" not in stores
+
+
+@pytest.mark.parametrize("codes,wgs,scratch", [
+    ((SteaneCode(), SurfaceCode(3, 3), SurfaceCode(5, 5)), 3, 0),
+    ((SteaneCode(), SurfaceCode(3, 3), ToricCode(3, 3)), 3, 128),      # slab plan on MFMA
+    ((SteaneCode(), SurfaceCode(3, 3), SurfaceCode(7, 7)), 2, 0),
+], ids=["lds", "slab", "d7"])
+def test_mixed_kernel_that_runs(codes, wgs, scratch, tmp_path):
+    """256 threads, held to the workgroups per CU that its LDS allows (three at
+    most), with no scratch but where three of a mix with a slab plan pay for it."""
+    plans = []
+    for c in codes:
+        t = CSSTannerGraph.from_code(c)
+        plans.append(D.compile(D.TNMMAP(), t, iid_error(0.02, 0.02, 0.02, t.nq)).hip)
+    src = L.mixed_spec_source(plans)
+    assert src == L.mixed_spec_source(plans, 256) and "__launch_bounds__(256, %d)" % wgs in src
+    f = tmp_path / "mixed.hip"
+    f.write_text("#include <hip/hip_runtime.h>\n" + src)
+    asm = assembly(f, tmp_path)
+    lds, used = (int(re.search(r"\.%s_segment_fixed_size: +(\d+)" % k, asm)[1]) for k in ("group", "private"))
+    assert wgs * lds <= 160 * 1024 and (wgs == 3 or (wgs + 1) * lds > 160 * 1024) and used <= scratch
