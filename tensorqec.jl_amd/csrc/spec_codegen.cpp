@@ -1447,8 +1447,9 @@ bool emit_reg_step(std::vector<RegChunk> &out, const CompiledPlan &cp, const Reg
 // the loads where they are put.  Measured with emit_reg_syndrome on the d=7
 // plan: FP32 64.2 -> 55.0 us per 65,536 rows and 20.9 -> 15.0 us for one tile
 // (budgets of 8 to 24 agree within 2%, 32 and more spill: 70 us), FP64 117 ->
-// 99 us.  Two waves per SIMD (223 registers) then wait 21% of their time and
-// issue a multiply-add every 3.9 cycles; the SIMD's own limit is 2.25.
+// 99 us.  Two waves per SIMD (224 registers) then wait 22% of their time and
+// issue a VALU instruction every 4.7 cycles, 86% of them multiply-adds; chains
+// of those alone issue one every 2.7 cycles with two waves.
 void emit_reg_chunks(std::ostringstream &o, const std::vector<RegChunk> &chunks, int budget) {
     size_t next = 0;
     int flight = 0;
