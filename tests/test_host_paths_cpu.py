@@ -37,7 +37,8 @@ def stub(tmp_path_factory):
 
 def run(stub, code, **env):
     r = subprocess.run([sys.executable, "-c", PLAN + code], capture_output=True, text=True, timeout=300,
-                       env={**os.environ, "LD_PRELOAD": stub, **env})
+                       env={**os.environ, "LD_PRELOAD": " ".join([stub, os.environ.get("LD_PRELOAD", "")]).strip(),
+                            **env})
     assert r.returncode == 0, r.stderr[-2000:]
     return r.stdout, [l[5:] for l in r.stderr.splitlines() if l.startswith("stub ")]
 
