@@ -20,6 +20,8 @@ namespace {
 
 size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
+constexpr size_t kCuLds = 160 * 1024;   // of a CU
+
 struct Layout {
     size_t work = 0, tab = 0, mx = 0, ex = 0, syn = 0, low = 0, red = 0, total = 0;
     size_t tab_entries = 0;
@@ -1505,8 +1507,17 @@ void emit_reg_syndrome(std::ostringstream &o, const CompiledPlan &cp, const std:
 // 7.3 and under 1 us, and several rows of a tile run side by side (65,536 rows
 // of d=3 with 1,002 of them re-checked: 13.6 -> 9.9 us).
 
-// LDS a workgroup may spend on it (beyond it, the separate kernel runs instead).
+// LDS a workgroup may spend on it (beyond it, the separate kernel runs instead);
+// with the FP32 tables in LDS no more than they leave: the 130 KB of a d=7 plan
+// and the 33 KB of its four rows do not fit a CU together.
 constexpr size_t kInlineRecheckLds = 48 * 1024;
+
+size_t reg_tab_bytes(const CompiledPlan &cp, const SpecCfg &cfg) {
+    return cfg.tab_lds ? std::max<size_t>(1, cp.const_pool.size() + cp.sliced_pool.size()) * (cfg.fp64 ? 8 : 4) : 0;
+}
+
+// its count and list of flagged rows, each aligned to 16 bytes at most
+size_t reg_list_bytes(const SpecCfg &cfg) { return 16 + round_up((size_t)cfg.threads / 4 * 4, 16); }
 
 struct Recheck {
     bool tables = false;                  // table slices staged in LDS
@@ -1529,11 +1540,16 @@ Recheck recheck_plan(const CompiledPlan &cp, const SpecCfg &cfg) {
         }
         r.at.push_back(at);
     }
-    r.tables = (size_t)top * 8 <= kInlineRecheckLds;
+    size_t room = kInlineRecheckLds;
+    if (cfg.tab_lds) {
+        const size_t held = round_up(reg_tab_bytes(cp, cfg), 16) + reg_list_bytes(cfg);
+        room = std::min(room, (kCuLds - std::min(kCuLds, held)) / 16 * 16);
+    }
+    r.tables = (size_t)top * 8 <= room;
     const int64_t e = r.tables ? top : cp.ws_entries;
-    if ((size_t)e * 8 > kInlineRecheckLds) return r;
+    if ((size_t)e * 8 > room) return r;
     r.entries = (int)e;
-    r.rows = (int)std::min<size_t>((size_t)cfg.threads / 64, kInlineRecheckLds / ((size_t)e * 8));
+    r.rows = (int)std::min<size_t>((size_t)cfg.threads / 64, room / ((size_t)e * 8));
     return r;
 }
 
@@ -1811,7 +1827,12 @@ bool spec_reg_inline_recheck(const CompiledPlan &cp, const SpecCfg &cfg) {
 }
 
 size_t spec_lds_bytes(const CompiledPlan &cp, const SpecCfg &cfg) {
-    if (cfg.reg) return cfg.tab_lds ? round_up(std::max<size_t>(1, cp.const_pool.size() + cp.sliced_pool.size()) * 4, 16) : 0;
+    if (cfg.reg) {
+        const Recheck r = recheck_plan(cp, cfg);
+        const size_t tab = reg_tab_bytes(cp, cfg);
+        if (r.rows == 0) return tab + 4;   // and the tile's count of flagged rows
+        return round_up(tab, 16) + reg_list_bytes(cfg) + round_up((size_t)r.rows * r.entries * 8, 16);
+    }
     return layout(cp, cfg).total;
 }
 
@@ -2408,8 +2429,6 @@ std::string spec_map_wave_source(const CompiledPlan &cp, int glog, int waves) {
       << fence << "  }\n}\n";
     return o.str();
 }
-
-constexpr size_t kCuLds = 160 * 1024;   // of a CU
 
 size_t spec_mixed_lds_bytes(const std::vector<MixedSpecPlan> &plans) {
     size_t m = 16;
